@@ -5,348 +5,495 @@
 // PLEGMA_baryons_deltas.cu:61-110 (Delta iso-3/2, Cg_k x g4 (Cg_k)^dag g4)
 // with factorised forms.  For a diquark matrix A (Abar = g4 A^dag g4) and
 // propagators P (quarks outside the diquark's partner) and Qm:
-//   St^{bb'}_{nu nu'} = A_{nu lam} Qm^{bb'}_{lam lam'} Abar_{lam' nu'}
-//   Q^{cc'}  = eps_abc eps_a'b'c' sum_{nu nu'} P^{aa'}_{nu nu'} St^{bb'}_{nu nu'}
-//   D_{mu mu'} = sum_{cc'} Q^{cc'} P^{cc'}_{mu mu'}
-//   X_{mu mu'} = eps eps' sum_{nu nu'} P^{ca'}_{mu nu'} St^{bb'}_{nu nu'} P^{ac'}_{nu mu'}
+//   St^{bb'}_{nu nu'}  = A_{nu lam} Qm^{bb'}_{lam lam'} Abar_{lam' nu'}
+//   W^{ck}_{nu' mu'}   = eps_abc eps_kb'c' sum_nu St^{bb'}_{nu nu'} P^{ac'}_{nu mu'}
+//   X_{mu mu'}         = sum_{nu' c k} P^{ck}_{mu nu'} W^{ck}_{nu' mu'}
+//   D_{mu mu'}         = -sum_{ck} tr(W^{ck}) P^{ck}_{mu mu'}
 //   proton  (Qm = other flavour)      = D - X
 //   Delta_k (uuu, Cg_k symmetric)     = 2 D - 4 X
-// The reference bodies cost 27648 complex MACs per proton dataset and about
-// 99000 per Delta component; this form costs 2304 per block (all four blocks
-// of one dataset: 9216), with 16 lanes of a wave per lattice site:
+// (the direct term's colour sum eps eps' P St over nu = mu is minus the trace
+// of W, by renaming the eps' indices).  Both results are one product of P
+// with W whose diagonal takes up the trace:
+//   D - X     =    - sum P^{ck}_{mu nu'} (W^{ck}_{nu' mu'} + delta_{nu' mu'}     tr W^{ck})
+//   2 D - 4 X = -4 * sum P^{ck}_{mu nu'} (W^{ck}_{nu' mu'} + delta_{nu' mu'} 1/2 tr W^{ck})
 //
-//   step 1, lane (nu, nu'):  Q partials, DPP row sum over the 16 lanes, D
-//   step 2, lane (nu', mu'): W^{c a'}_{nu' mu'} = sum_nu eps eps' St P   -> LDS
-//   step 3, lane (mu, mu'):  X = sum_{nu' c a'} P^{c a'}_{mu nu'} W_{nu' mu'}
+// The four diquarks Cg5, Cg3 and Cg1, Cg2 are signed permutations of two xor
+// classes c; the two of a class differ by phases, so their W come from the
+// same colour products M(Qm_{nu^c nu'^c}, P_{nu mu'}) (sum x +- y over the two
+// kinds of rows nu).  M is symmetric in its arguments: with Qm = P, rows nu
+// and nu^c exchange (nu', mu') with (mu'^c, nu'^c), so half of the products
+// (one row of each pair for c = 1, one order of (a, b) for c = 0) give W by a
+// transposition.
 //
-// The four diquarks Cg5, Cg1, Cg2, Cg3 are signed permutations of two xor
-// classes; blocks of one class that share Qm (proton and Delta_3, Delta_1 and
-// Delta_2 on one propagator) differ only by phases, so their step-2 colour
-// contraction T(nu) is computed once and accumulated with both blocks' row
-// phases (compile-time); lane phases are applied once per block.
+// Work split: four lanes per site, 16 sites per wave, lane j = mu'; the other
+// spin index runs relative to it, nu' = j ^ s, s = 0..3, so the transposition
+// is the exchange of lanes j and j ^ s (or j ^ s ^ 1), a DPP operand of the
+// adds, the diagonal is s = 0, and W stays in registers.  The Abar phase of
+// nu' is a sign character of the spin index: sigma(j ^ s) = sigma(j) sigma(s),
+// a lane sign of the result and compile-time signs of the products.  The
+// operands come from the staged tile in LDS, 8 FMAs per 8-byte read.  One wave
+// contracts {Cg5, Cg3}, another {Cg1, Cg2} and each half of the mesons of
+// the same staged 16 sites.
+//
+// What bounds it: vector instructions (per site and propagator 278 of the 372
+// wave instructions are the products' FMAs, 9 300 flop per lane-site), and in
+// FP32 the power they take: two waves issue FMAs together (2.9 cycles per
+// instruction measured here, 2.45 in a loop of FMAs alone), and the clock
+// falls to 1.7 GHz.  Four waves per SIMD (18 KB of LDS per 2-wave workgroup,
+// 128 registers) measured best; two or three waves, operands read two or
+// three steps ahead, the next tile prefetched into registers, and 4 x 4 spin
+// products on v_mfma_f32_4x4x1 (12.8 cycles each, not beside the vector
+// unit's work) were within 5 % or slower.  Sixteen lanes per site with W
+// exchanged through LDS and the trace formed apart (the earlier form) took
+// 16.3 ms on 10.98 M sites x 80 channels in FP32, this one 7.1 ms (1 550 M
+// sites/s; the HBM floor of its 20 GB is 4.2 ms); FP64, two flavours, 276 k
+// sites x 128 channels: 2.36 -> 0.95 ms.
 #include "plg_tile.h"
 
 namespace plg {
 
-// LDS of one workgroup.  w holds the exchange intermediates of a block pair,
-// the meson Gram rows before the blocks and the output stage after them.
-// s2 is last so the one-propagator variant is allocated without it.
-template <typename T> struct BaryonShared {
-  cx<T> s1[144][BT_SP];
-  cx<T> w[BT_SITES][BT_WS];
-  cx<T> s2[144][BT_SP];
+// entry (mu, nu, colour pair cc) of site x at cc 256 + mu 64 + nu 16 + (x ^ SW nu):
+// the 16 lanes of an LDS pass, which hold the four nu of four sites (consecutive
+// ones for 8-byte reads, sites 0, 3, 5, 6 mod 8 for 16-byte reads), read distinct
+// banks; the spin mu and colour offsets are immediates
+constexpr int BQ_TILE = 144 * 16;
+constexpr int BQ_SW = 4;
+template <typename T> struct BqT {
+  static constexpr int EPU = sizeof(T) == 4 ? 2 : 1;  // sites of a 16-byte unit
+  static constexpr int WPE = sizeof(T) == 4 ? 4 : 2;  // waves per SIMD (LDS and registers)
+};
+template <typename T, int N> struct BqVec;
+template <> struct BqVec<float, 2> {  // two sites; site pairs are 8-byte aligned
+  typedef float v __attribute__((ext_vector_type(4), aligned(8)));
+};
+template <> struct BqVec<double, 1> {
+  typedef double v __attribute__((ext_vector_type(2)));
 };
 
-__constant__ MesonX c_mesonx = make_mesonx();
+// value of lane ^ S within the four lanes of a site
+template <int S> __device__ __forceinline__ float quad_xor(float v) {
+  if constexpr (S == 0) return v;
+  else return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), S == 1 ? 0xB1 : S == 2 ? 0x4E : 0x1B, 0xF, 0xF, true));
+}
+template <int S> __device__ __forceinline__ double quad_xor(double v) {
+  if constexpr (S == 0) return v;
+  else {
+    constexpr int ctrl = S == 1 ? 0xB1 : S == 2 ? 0x4E : 0x1B;
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_mov_dpp((int)b, ctrl, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), ctrl, 0xF, 0xF, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+  }
+}
+template <typename T> __device__ __forceinline__ T quad_sum(T v) {
+  v += quad_xor<1>(v);
+  v += quad_xor<2>(v);
+  return v;
+}
 
-// eps eps' contraction of two colour blocks x[a][a'] y[b][b'] into out[c][c'] (+=),
-// every term one complex FMA
-template <typename T> __device__ __forceinline__ void eps2(const cx<T> *x, const cx<T> *y, cx<T> *out) {
-  static_for<0, 6>([&](auto e1) {
-    static_for<0, 6>([&](auto e2) {
-      constexpr int a = EPS[e1.value][0], b = EPS[e1.value][1], c = EPS[e1.value][2];
-      constexpr int ap = EPS[e2.value][0], bp = EPS[e2.value][1], cp = EPS[e2.value][2];
-      constexpr int ph = SGN_EPS[e1.value] * SGN_EPS[e2.value] > 0 ? 0 : 2;
-      cfma_iph<ph>(out[c * 3 + cp], x[a * 3 + ap], y[b * 3 + bp]);
+// sign of a phase table relative to its entry 0, as a character of the index
+constexpr bool bq_char_ok(const int (&ph)[4]) {
+  for (int n = 0; n < 4; n++)
+    if (((ph[n] - ph[0]) & 1) != 0) return false;
+  return ((ph[1] - ph[0] + ph[2] - ph[0]) & 3) == ((ph[3] - ph[0]) & 3);
+}
+// lane j's sign of a character
+template <typename T> __device__ __forceinline__ T bq_sign(const int (&ph)[4], int j) {
+  T s = 1;
+#pragma unroll
+  for (int n = 1; n < 4; n++) s = (j == n && ((ph[n] - ph[0]) & 3) == 2) ? (T)-1 : s;
+  return s;
+}
+
+// R[b][mu] (column mu' = j) of diquark W0 and, if W1 >= 0, of W1 of its class:
+// sum over nu', c, k of P (W + kappa delta tr W), up to the scale and lane
+// sign of bq_scale.  P, Q: the tiles at (lane, s = 0 column); SAME: Q = P
+template <int W0, int W1> struct BqClass {
+  static constexpr SPerm A0 = diquark(W0), A1 = diquark(W1 >= 0 ? W1 : W0);
+  static constexpr SPerm Ab0 = diquark_bar(W0), Ab1 = diquark_bar(W1 >= 0 ? W1 : W0);
+  static constexpr int cls = sp_class(A0);
+  static constexpr int RA = (A1.ph[0] - A0.ph[0]) & 3;
+  // the second diquark's row phases are A1.ph = A0.ph + RA + kind
+  static constexpr int kind(int nu) { return (A1.ph[nu] - A0.ph[nu] - RA) & 3; }
+  // the n-th row of the halved sum (c = 1): one of each pair, of kind 0
+  static constexpr int row(int n) {
+    for (int nu = 0; nu < 4; nu++)
+      if ((W1 >= 0 ? kind(nu) == 0 : nu < (nu ^ cls)) && n-- == 0) return nu;
+    return -1;
+  }
+  // phase of row nu ^ c relative to row nu: 0 symmetric, 2 antisymmetric
+  static constexpr int partner = cls ? (A0.ph[row(0) ^ cls] - A0.ph[row(0)]) & 3 : 0;
+  static constexpr bool ok() {
+    if (sp_class(A1) != cls || sp_class(Ab0) != cls || sp_class(Ab1) != cls || cls > 1) return false;
+    for (int nu = 0; nu < 4; nu++)
+      if (kind(nu) & 1) return false;
+    if (cls && (((A0.ph[row(1) ^ cls] - A0.ph[row(1)]) & 3) != partner || (partner & 1))) return false;
+    return bq_char_ok(Ab0.ph) && bq_char_ok(Ab1.ph);
+  }
+  // phase of Abar row nu' (character of nu', with the class shift as an offset)
+  static constexpr int ab(int b, int n) { return b == 0 ? Ab0.ph[n ^ cls] : Ab1.ph[n ^ cls]; }
+  static constexpr int sig(int b, int s) { return (ab(b, s) - ab(b, 0)) & 3; }  // 0 or 2
+  // phase of a whole result
+  static constexpr int phase(int b) { return (ab(b, 0) + (b == 1 ? RA : 0)) & 3; }
+};
+
+template <typename T, int W0, int W1, bool SAME>
+__device__ __forceinline__ void bq_class(const cx<T> *P, const cx<T> *Q, int site, int j, cx<T> (&R)[2][4]) {
+  using B = BqClass<W0, W1>;
+  static_assert(B::ok(), "row phases, symmetry and sign characters of the class");
+  constexpr int NB = W1 >= 0 ? 2 : 1, cls = B::cls;
+  constexpr bool HALF_NU = SAME && cls == 1, HALF_AB = SAME && cls == 0;
+  constexpr int NN = HALF_NU ? 2 : 4;                       // rows nu summed
+  constexpr bool TWO_ACC = NB == 2 && !HALF_NU;             // kinds summed apart
+  // columns nu' = j ^ s of the tiles
+  const cx<T> *pc[4], *qc[4];
+#pragma unroll
+  for (int s = 0; s < 4; s++) {
+    const int n = j ^ s;
+    pc[s] = P + n * 16 + (site ^ (BQ_SW * n));
+    qc[s] = SAME ? pc[s] : Q + n * 16 + (site ^ (BQ_SW * n));
+  }
+#pragma unroll
+  for (int b = 0; b < 2; b++)
+#pragma unroll
+    for (int m = 0; m < 4; m++) R[b][m] = cmake<T>(0, 0);
+  // The operands of a step are read from LDS while the previous step's
+  // products run (two buffers): a step is a row nu and an s in the sums of W,
+  // an s and a row mu in the products with P.  The scheduler, left alone,
+  // places the reads next to their use.
+  cx<T> p[2][2][3], q[2][2][3];
+  auto load_p = [&](auto r_, int o0, int o1) {
+    constexpr int r = r_.value, nu = HALF_NU ? B::row(r) : r;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      p[r & 1][0][k] = pc[0][nu * 64 + o0 + k * 256];
+      if constexpr (!HALF_AB) p[r & 1][1][k] = pc[0][nu * 64 + o1 + k * 256];
+    }
+  };
+  auto load_q = [&](auto i_, int o0, int o1) {
+    constexpr int i = i_.value, r = i / 4, s = i % 4, nu = HALF_NU ? B::row(r) : r;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+      if constexpr (!HALF_AB) q[i & 1][0][k] = qc[s ^ cls][(nu ^ cls) * 64 + o0 + k * 256];
+      q[i & 1][1][k] = qc[s ^ cls][(nu ^ cls) * 64 + o1 + k * 256];
+    }
+  };
+  auto load_x = [&](auto i_, int oc) {
+    constexpr int i = i_.value, s = i / 4, m = i % 4;
+#pragma unroll
+    for (int k = 0; k < 3; k++) q[i & 1][0][k] = pc[s][m * 64 + oc + k * 256];
+  };
+  load_p(ic<0>{}, 768, 1536);
+  load_q(ic<0>{}, 768, 1536);
+#pragma unroll 1
+  for (int c = 0; c < 3; c++) {
+    const int o0 = (c < 2 ? c + 1 : 0) * 768, o1 = (c > 0 ? c - 1 : 2) * 768;
+    cx<T> x[4][3], y[4][3];
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+#pragma unroll
+      for (int k = 0; k < 3; k++) x[s][k] = y[s][k] = cmake<T>(0, 0);
+    static_for<0, 4 * NN>([&](auto i_) {
+      constexpr int i = i_.value, r = i / 4, s = i % 4, nu = HALF_NU ? B::row(r) : r;
+      if constexpr (s == 2 && r + 1 < NN) load_p(ic<r + 1>{}, o0, o1);
+      if constexpr (i + 1 < 4 * NN) load_q(ic<i + 1>{}, o0, o1);
+      else load_x(ic<0>{}, c * 768);
+      __builtin_amdgcn_sched_barrier(0);
+      // the eps_abc orders (a, b) = (r0, r1), (r1, r0), the eps_kb'c' orders of every k
+      static_for<0, (HALF_AB ? 1 : 2)>([&](auto e1) {
+        static_for<0, 2>([&](auto e2) {
+          static_for<0, 3>([&](auto k_) {
+            constexpr int k = k_.value, bp = (k + 1 + e2.value) % 3, cp = (k + 2 - e2.value) % 3;
+            constexpr int ph = B::A0.ph[nu] + (e1.value == e2.value ? 0 : 2);
+            if constexpr (TWO_ACC && B::kind(nu) == 2)
+              cfma_iph<ph>(y[s][k], q[i & 1][1 - e1.value][bp], p[r & 1][e1.value][cp]);
+            else
+              cfma_iph<ph>(x[s][k], q[i & 1][1 - e1.value][bp], p[r & 1][e1.value][cp]);
+          });
+        });
+      });
+      __builtin_amdgcn_sched_barrier(0);
     });
+    // V[0] = x + y, V[1] = x - y (times i^RA, in the result's phase)
+    cx<T> V[2][4][3];
+    static_for<0, 4>([&](auto s_) {
+      constexpr int s = s_.value;
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        cx<T> a = x[s][k], d = y[s][k];
+        if constexpr (HALF_AB) {
+          a = cmake<T>(a.re + quad_xor<s>(a.re), a.im + quad_xor<s>(a.im));
+          if constexpr (TWO_ACC) d = cmake<T>(d.re + quad_xor<s>(d.re), d.im + quad_xor<s>(d.im));
+        }
+        if constexpr (HALF_NU) {
+          d = cmake<T>(quad_xor<s ^ 1>(a.re), quad_xor<s ^ 1>(a.im));
+          V[0][s][k] = B::partner == 0 ? a + d : a - d;
+          V[1][s][k] = B::partner == 0 ? a - d : a + d;
+        } else if constexpr (TWO_ACC) {
+          V[0][s][k] = a + d;
+          V[1][s][k] = a - d;
+        } else {
+          V[0][s][k] = a;
+        }
+      }
+    });
+    // the trace over nu' = mu' joins the diagonal s = 0 with weight kappa; up
+    // to the lane sign sigma(j), sum_j' sigma(j') v(j') = sum_s sigma(s) v(j ^ s)
+    static_for<0, NB>([&](auto b_) {
+      constexpr int b = b_.value;
+      constexpr T kap = (b == 0 ? W0 : W1) == 0 ? (T)1 : (T)0.5;
+      auto trace = [&](T t) {
+        t = B::sig(b, 1) == 0 ? t + quad_xor<1>(t) : t - quad_xor<1>(t);
+        return B::sig(b, 2) == 0 ? t + quad_xor<2>(t) : t - quad_xor<2>(t);
+      };
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        cx<T> &v = V[b][0][k];
+        v = cmake<T>(fma(kap, trace(v.re), v.re), fma(kap, trace(v.im), v.im));
+      }
+    });
+    // R[b][mu] += P[mu][nu'] . V[b][nu'], the sign of s included
+    static_for<0, 16>([&](auto i_) {
+      constexpr int i = i_.value, s = i / 4, m = i % 4;
+      if constexpr (i < 15) {
+        load_x(ic<i + 1>{}, c * 768);
+      } else {  // the next colour row's first operands
+        load_p(ic<0>{}, (c < 1 ? c + 2 : c - 1) * 768, c * 768);
+        load_q(ic<0>{}, (c < 1 ? c + 2 : c - 1) * 768, c * 768);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < 3; k++) {
+        const cx<T> pv = q[i & 1][0][k];
+        // (an antisymmetric diquark has no s = 1 part)
+        if constexpr (!(HALF_NU && s == 1 && B::partner == 2)) cfma_iph<B::sig(0, s)>(R[0][m], pv, V[0][s][k]);
+        if constexpr (NB == 2 && !(HALF_NU && s == 1 && B::partner == 0)) cfma_iph<B::sig(1, s)>(R[1][m], pv, V[1][s][k]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  }
+  // lane sign and phase of the results
+  static_for<0, NB>([&](auto b_) {
+    constexpr int b = b_.value;
+    const T sg = bq_sign<T>(b == 0 ? B::Ab0.ph : B::Ab1.ph, j);
+#pragma unroll
+    for (int m = 0; m < 4; m++) R[b][m] = sg * cmul_iph(R[b][m], B::phase(b));
   });
 }
-// exchange form: out[c][a'] += i^PH eps eps' st[b][b'] p[a][c']
-template <int PH, typename T>
-__device__ __forceinline__ void eps2x(const cx<T> *st, const cx<T> *p, cx<T> *out) {
-  static_for<0, 6>([&](auto e1) {
-    static_for<0, 6>([&](auto e2) {
-      constexpr int a = EPS[e1.value][0], b = EPS[e1.value][1], c = EPS[e1.value][2];
-      constexpr int ap = EPS[e2.value][0], bp = EPS[e2.value][1], cp = EPS[e2.value][2];
-      constexpr int ph = PH + (SGN_EPS[e1.value] * SGN_EPS[e2.value] > 0 ? 0 : 2);
-      cfma_iph<ph>(out[c * 3 + ap], st[b * 3 + bp], p[a * 3 + cp]);
+
+// phases of the meson channels: op, class and i^ph of X = g5 G per row
+constexpr MesonX BQ_X = make_mesonx();
+// the n-th op of xor class d
+constexpr int bq_op(int d, int n) {
+  for (int op = 0; op < 16; op++)
+    if (BQ_X.cls[op] == d && n-- == 0) return op;
+  return -1;
+}
+
+// mesons of the xor classes [D0, D1): G_d[al][be] = sum_cc S[al][be] conj(S[al^d][be^d]),
+// channel op of class d: sum_{al be} i^(ph[al^d] + ph[be]) G_d[al][be].
+// Lane j holds column be = j.  Of the pair (al, j), (al^d, j^d), whose entries
+// are conjugate, each lane sums its own column at the al without d's top bit;
+// the other half comes from the partner lane.  Of the four channels of a
+// class, lane n of the site receives the n-th (store(op, value)).
+template <int D0, int D1, typename T, typename F>
+__device__ __forceinline__ void bq_mesons(const cx<T> *S, int site, int j, F &&store) {
+  const cx<T> *col = S + j * 16 + (site ^ (BQ_SW * j));
+  T n0[4] = {0, 0, 0, 0};
+  cx<T> g[3][2];
+#pragma unroll
+  for (int d = 0; d < 3; d++) g[d][0] = g[d][1] = cmake<T>(0, 0);
+#pragma unroll 3
+  for (int cc = 0; cc < 9; cc++) {
+    cx<T> s[4];
+#pragma unroll
+    for (int al = 0; al < 4; al++) s[al] = col[al * 64 + cc * 256];
+    static_for<D0, D1>([&](auto d_) {
+      constexpr int d = d_.value;
+      if constexpr (d == 0) {
+#pragma unroll
+        for (int al = 0; al < 4; al++) n0[al] = fma(s[al].re, s[al].re, fma(s[al].im, s[al].im, n0[al]));
+      } else {
+        static_for<0, 2>([&](auto h) {
+          constexpr int al = d >= 2 ? h.value : 2 * h.value;
+          const cx<T> o = cmake<T>(quad_xor<d>(s[al ^ d].re), quad_xor<d>(s[al ^ d].im));
+          cfma_conj(g[d - 1][h.value], s[al], o);
+        });
+      }
     });
+  }
+  static_for<D0, D1>([&](auto d_) {
+    constexpr int d = d_.value;
+    cx<T> G[4];
+    if constexpr (d == 0) {
+#pragma unroll
+      for (int al = 0; al < 4; al++) G[al] = cmake<T>(n0[al], 0);
+    } else {
+      static_for<0, 2>([&](auto h) {
+        constexpr int al = d >= 2 ? h.value : 2 * h.value;
+        G[al] = g[d - 1][h.value];
+        G[al ^ d] = cmake<T>(quad_xor<d>(G[al].re), -quad_xor<d>(G[al].im));
+      });
+    }
+    cx<T> v[4];
+    static_for<0, 4>([&](auto n) {
+      constexpr int op = bq_op(d, n.value);
+      static_assert(op >= 0 && bq_char_ok(BQ_X.ph[op < 0 ? 0 : op]), "four channels per class, sign characters");
+      cx<T> w = cmake<T>(0, 0);
+      static_for<0, 4>([&](auto al) { w = w + cmul_iph(G[al.value], BQ_X.ph[op][al.value ^ d] + BQ_X.ph[op][0]); });
+      v[n.value] = bq_sign<T>(BQ_X.ph[op], j) * w;
+    });
+    // sums over the four lanes, lane n keeping channel n
+    const bool odd = j & 1, hi = j & 2;
+    auto pick = [&](T a, T b, T c, T e) {
+      const T a1 = odd ? b : a, b1 = odd ? a : b, c1 = odd ? e : c, e1 = odd ? c : e;
+      const T lo2 = a1 + quad_xor<1>(b1), hi2 = c1 + quad_xor<1>(e1);
+      const T keep = hi ? hi2 : lo2, send = hi ? lo2 : hi2;
+      return keep + quad_xor<2>(send);
+    };
+    const int op = j == 0 ? bq_op(d, 0) : j == 1 ? bq_op(d, 1) : j == 2 ? bq_op(d, 2) : bq_op(d, 3);
+    store(op, cmake<T>(pick(v[0].re, v[1].re, v[2].re, v[3].re), pick(v[0].im, v[1].im, v[2].im, v[3].im)));
   });
 }
 
-// D and X of diquark W0 and, if W1 >= 0, of W1 (same spin class, same Qm).
-// pa: this lane's P[hi][lo] colour block (lane = (nu, nu') = (mu, mu')).
-template <typename T, int W0, int W1>
-__device__ __forceinline__ void baryon_group(const cx<T> (*P)[BT_SP], const cx<T> (*Qm)[BT_SP],
-                                             cx<T> (*Wsh)[16][9], int s, int lane, const cx<T> *pa,
-                                             cx<T> *D, cx<T> *X) {
-  constexpr int NB = W1 >= 0 ? 2 : 1;
-  constexpr SPerm A0 = diquark(W0), Ab0 = diquark_bar(W0);
-  constexpr SPerm A1 = diquark(W1 >= 0 ? W1 : W0), Ab1 = diquark_bar(W1 >= 0 ? W1 : W0);
-  constexpr int c = sp_class(A0);
-  static_assert(sp_class(A1) == c && sp_class(Ab0) == c && sp_class(Ab1) == c, "one spin class per group");
-  const int hi = lane >> 2, lo = lane & 3;
-
-  // ---- step 1: lane (nu, nu') -> Q partial, row sum, D on lane (mu, mu')
-  {
-    cx<T> q[9], Qr[9];
-#pragma unroll
-    for (int i = 0; i < 9; i++) {
-      q[i] = Qm[pidx(hi ^ c, lo ^ c, 0, 0) + i][s];
-      Qr[i] = cmake<T>(0, 0);
-    }
-    eps2(pa, q, Qr);
-    static_for<0, NB>([&](auto k) {
-      constexpr SPerm A = k.value == 0 ? A0 : A1;
-      constexpr SPerm Ab = k.value == 0 ? Ab0 : Ab1;
-      int ph = 0;
-      // lane phase A[nu][nu^c] * Abar[nu'^c][nu']
-#pragma unroll
-      for (int i = 0; i < 4; i++) ph += (hi == i ? A.ph[i] : 0) + (lo == i ? Ab.ph[i ^ c] : 0);
-      cx<T> d = cmake<T>(0, 0);
-#pragma unroll
-      for (int i = 0; i < 9; i++) {
-        cx<T> v = cmul_iph_rt(Qr[i], ph);
-        v.re = rowsum16(v.re);
-        v.im = rowsum16(v.im);
-        cfma(d, v, pa[i]);
-      }
-      D[k.value] = d;
-    });
+// rotation of a staged tile to the physical basis in place (nthr threads)
+template <typename T> __device__ __forceinline__ void bq_rotate(cx<T> *S, int sign, int thr, int nthr) {
+  for (int it = thr; it < 16 * 36; it += nthr) {
+    const int s = it & 15, cq = it >> 4, cp = cq % 9, q = cq / 9, m = q >> 1, n = q & 1;
+    auto at = [&](int mu, int nu) -> cx<T> & { return S[cp * 256 + mu * 64 + nu * 16 + (s ^ (BQ_SW * nu))]; };
+    cx<T> a = at(m, n), b = at(m, n + 2), c = at(m + 2, n), d = at(m + 2, n + 2);
+    rot_physical(a, b, c, d, sign);
+    at(m, n) = a;
+    at(m, n + 2) = b;
+    at(m + 2, n) = c;
+    at(m + 2, n + 2) = d;
   }
-  // ---- step 2: lane (nu', mu') -> W = sum_nu A-phase(nu) T(nu); the
-  // Abar-phase of row nu' is applied by the readers in step 3
-  // The second block's row phases are A1.ph = A0.ph + RA or + RA + 2 (mod 4),
-  // so U_0 and U_1 (the A0-phased T(nu) of the two kinds of rows) are
-  // accumulated by FMA and W_0 = U_0 + U_1, W_1 = i^RA (U_0 - U_1).
-  {
-    constexpr int RA = (A1.ph[0] - A0.ph[0]) & 3;
-    cx<T> W[NB][9];
-#pragma unroll
-    for (int b = 0; b < NB; b++)
-#pragma unroll
-      for (int i = 0; i < 9; i++) W[b][i] = cmake<T>(0, 0);
-    static_for<0, 4>([&](auto nu) {
-      constexpr int r = (A1.ph[nu.value] - A0.ph[nu.value] - RA) & 3;
-      static_assert(r == 0 || r == 2, "row phases of a class pair differ by +-i^RA");
-      constexpr int acc = (NB == 2 && r == 2) ? 1 : 0;
-      cx<T> sq[9], pp[9];
-#pragma unroll
-      for (int i = 0; i < 9; i++) {
-        sq[i] = Qm[pidx(nu.value ^ c, hi ^ c, 0, 0) + i][s];
-        pp[i] = P[pidx(nu.value, lo, 0, 0) + i][s];
-      }
-      eps2x<A0.ph[nu.value]>(sq, pp, W[acc]);
-    });
-    if constexpr (NB == 2) {
-#pragma unroll
-      for (int i = 0; i < 9; i++) {
-        const cx<T> u0 = W[0][i], u1 = W[1][i];
-        W[0][i] = u0 + u1;
-        W[1][i] = cmul_iph(u0 - u1, RA);
-      }
-    }
-    // shared without this lane's Abar phase: the reader knows the row
-    // (nu' = its loop index) and folds the phase into its FMAs
-#pragma unroll
-    for (int b = 0; b < NB; b++)
-#pragma unroll
-      for (int i = 0; i < 9; i++) Wsh[b][lane][i] = W[b][i];
-  }
-  wave_lds_sync();
-  // ---- step 3: lane (mu, mu') -> X = sum_{nu'} P[mu][nu'] . W[nu'][mu']
-  {
-    cx<T> x[NB];
-#pragma unroll
-    for (int b = 0; b < NB; b++) x[b] = cmake<T>(0, 0);
-    static_for<0, 4>([&](auto nu) {
-      constexpr int nup = nu.value;
-      // the Abar phase of the writing lane (row nu')
-      constexpr int ph0 = Ab0.ph[nup ^ c], ph1 = Ab1.ph[nup ^ c];
-#pragma unroll
-      for (int i = 0; i < 9; i++) {
-        const cx<T> p = P[pidx(hi, nup, 0, 0) + i][s];
-        cfma_iph<ph0>(x[0], p, Wsh[0][nup * 4 + lo][i]);
-        if constexpr (NB == 2) cfma_iph<ph1>(x[1], p, Wsh[1][nup * 4 + lo][i]);
-      }
-    });
-#pragma unroll
-    for (int b = 0; b < NB; b++) X[b] = x[b];
-  }
-  wave_lds_sync();  // W is overwritten by the next group of this wavefront
 }
+
+// waves of a workgroup and the work of each: the datasets times the halves
+// (diquark classes {Cg5, Cg3} and {Cg1, Cg2}, or baryons and mesons)
+template <bool TWO, bool MES, int GMASK> struct BqSplit {
+  static constexpr bool H0 = GMASK & 1, H1 = GMASK & (1 << 7), H2 = GMASK & (1 << 8), H3 = GMASK & (1 << 9);
+  static_assert(H1 == H2 && H2 == H3, "the Delta groups are computed together");
+  static constexpr int halves = (H1 || MES) ? 2 : 1;
+  static constexpr int ND = TWO ? 2 : 1;
+  static constexpr int threads = 64 * halves * ND;
+};
 
 // Output channels per row (from ch0): [16 mesons of S1 if MES], then for each
 // dataset d (2 if TWO) and each selected group g in the reference order
 // (nucl_nucl, deltapp_deltamm_11, _22, _33): 16 components mu*4 + mu'.
-// FP32 tiles fit two workgroups per CU in LDS, so their register budget is
-// capped at two waves per SIMD.
 template <typename T, bool TWO, bool MES, int GMASK>
-__global__ __launch_bounds__(BT_THREADS) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 2 : 1)))
-void k_baryon(const PropDev<T> *__restrict__ props,
-                                                       const RowDev *__restrict__ rows,
-                                                       cx<T> *__restrict__ out, int64_t V3, int T_lat,
-                                                       int nch_total, int ch0, int ntiles) {
-  constexpr bool H0 = GMASK & 1, H1 = GMASK & (1 << 7), H2 = GMASK & (1 << 8), H3 = GMASK & (1 << 9);
-  constexpr int NG = (int)H0 + (int)H1 + (int)H2 + (int)H3;
-  constexpr int R0 = 0, R1 = (int)H0, R2 = (int)H0 + (int)H1, R3 = (int)H0 + (int)H1 + (int)H2;
-  constexpr int ND = TWO ? 2 : 1;
+__global__ __launch_bounds__((BqSplit<TWO, MES, GMASK>::threads)) __attribute__((amdgpu_waves_per_eu(BqT<T>::WPE)))
+void k_baryon(const PropDev<T> *__restrict__ props, const RowDev *__restrict__ rows, cx<T> *__restrict__ out,
+              int64_t V3, int T_lat, int nch_total, int ch0, int ntiles) {
+  using B = BqSplit<TWO, MES, GMASK>;
+  constexpr bool H0 = B::H0, HD = B::H1;
+  constexpr int NG = (int)H0 + 3 * (int)HD;
+  constexpr int R0 = 0, R1 = (int)H0, R2 = R1 + 1, R3 = R1 + 2;
   constexpr int MOFF = MES ? 1 : 0;
-  constexpr int NOUT = MOFF + ND * NG;
-  static_assert(NOUT <= 9, "output stage holds 9 values per lane");
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  BaryonShared<T> &sh = *reinterpret_cast<BaryonShared<T> *>(smem_raw);
-
+  constexpr int NT = 64 * B::halves;  // threads that stage a propagator
+  // staging: UPC threads of a spin pair load the 16 sites of a component in
+  // 16-byte units; thread group g takes the spin pairs g + PG h, the nine
+  // colour pairs of each (nu = g % 4: one LDS offset per thread)
+  constexpr int EPU = BqT<T>::EPU, UPC = 16 / EPU, PG = NT / UPC, NH = 16 / PG, NU = 9 * NH;
+  static_assert(PG % 4 == 0 && NH * PG == 16, "whole passes over the spin pairs");
+  typedef typename BqVec<T, EPU>::v vec;
+  __shared__ __align__(16) cx<T> tile[B::ND][BQ_TILE];
   const RowDev row = rows[blockIdx.y];
-  const PropDev<T> P1 = props[row.pa];
-  const PropDev<T> P2 = props[TWO ? row.pb : row.pa];
-  const int tid = threadIdx.x;
-  const int s = tid >> 4, lane = tid & 15;
-  const int hi = lane >> 2, lo = lane & 3;
-  const int64_t plane1 = (int64_t)((row.t - P1.t_first + T_lat) % T_lat) * V3;
-  const int64_t plane2 = (int64_t)((row.t - P2.t_first + T_lat) % T_lat) * V3;
-  // preparation of the loaded entries (boundary sign, rotation)
-  const T sg1 = prop_sign(P1, row.t), sg2 = prop_sign(P2, row.t);
-  const bool prep_rot = P1.rot != 0 || (TWO && P2.rot != 0);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int half = wave % B::halves, ds = wave / B::halves;
+  const PropDev<T> P1 = props[row.pa], P2 = props[TWO ? row.pb : row.pa];
+  // the propagator this wave stages: its dataset's
+  const PropDev<T> PD = ds == 0 ? P1 : P2;
+  const int thr = threadIdx.x - ds * NT, g0 = thr / UPC, e0 = (thr % UPC) * EPU;
+  const cx<T> *src = PD.data + (int64_t)((row.t - PD.t_first + T_lat) % T_lat) * V3 + (int64_t)(g0 * 9) * PD.cs + e0;
+  // the boundary signs multiply the results: a baryon of dataset d holds its
+  // propagator squared times the diquark's other one (proton) or cubed
+  const T sgp = prop_sign(PD, row.t), sgo = TWO ? prop_sign(ds == 0 ? P2 : P1, row.t) : sgp;
+  const int64_t ncols = (int64_t)gridDim.y * nch_total, col0 = (int64_t)blockIdx.y * nch_total + ch0;
 
-  // tile staging: thread -> site tid%16, components tid/16 + 16 j (j < 9).
-  // The components of tile t+1 are fetched into registers while tile t is
-  // contracted (coalesced: 16 consecutive sites per component).
-  constexpr int NF = 144 / (BT_THREADS / BT_SITES);
-  cx<T> pf1[NF], pf2[TWO ? NF : 1];
-  // one pointer per propagator, advanced by 16 components per load
-  const cx<T> *f1 = P1.data + plane1 + (int64_t)(tid >> 4) * P1.cs + (tid & 15);
-  const cx<T> *f2 = P2.data + plane2 + (int64_t)(tid >> 4) * P2.cs + (tid & 15);
-  const int64_t st1 = 16 * P1.cs, st2 = 16 * P2.cs;
-  auto fetch = [&](int tl) {
-    const int64_t x0 = (int64_t)tl * BT_SITES;
-    const cx<T> *b1 = f1 + x0, *b2 = f2 + x0;
-    if (x0 + BT_SITES <= V3) {
+  for (int tl = blockIdx.x; tl < ntiles; tl += gridDim.x) {
+    const int64_t x0 = (int64_t)tl * 16;
+    // opaque: addresses and masks derived from it are formed per tile instead
+    // of being kept in registers across the loop
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int j = tid & 3, site = (tid & 63) >> 2;
+    cx<T> *dst = tile[ds] + g0 * 16 + (e0 ^ (BQ_SW * (g0 & 3)));
+    __syncthreads();  // the previous tile's reads are done
+    if (x0 + 16 <= V3) {
+      vec v[NU];
 #pragma unroll
-      for (int j = 0; j < NF; j++) {
-        pf1[j] = gload(b1);
-        if constexpr (TWO) pf2[j] = gload(b2);
-        b1 += st1;
-        b2 += st2;
+      for (int k = 0; k < NU; k++)
+        v[k] = *(const __attribute__((address_space(1))) vec *)(src + x0 + ((k / 9) * (9 * PG) + k % 9) * PD.cs);
+#pragma unroll
+      for (int k = 0; k < NU; k++) {
+        typedef T av __attribute__((ext_vector_type(2 * EPU)));
+        *(av *)&dst[(k / 9) * (16 * PG) + (k % 9) * 256] = v[k];
       }
     } else {
-      const bool ok = x0 + (tid & 15) < V3;
+#pragma unroll 1
+      for (int k = 0; k < NU; k++)
 #pragma unroll
-      for (int j = 0; j < NF; j++) {
-        pf1[j] = ok ? gload(b1 + j * st1) : cmake<T>(0, 0);
-        if constexpr (TWO) pf2[j] = ok ? gload(b2 + j * st2) : cmake<T>(0, 0);
-      }
-    }
-  };
-  if (blockIdx.x < ntiles) fetch(blockIdx.x);
-  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int64_t x0 = (int64_t)tile * BT_SITES;
-#pragma unroll
-    for (int j = 0; j < NF; j++) {
-      sh.s1[(tid >> 4) + 16 * j][tid & 15] = cmake<T>(sg1 * pf1[j].re, sg1 * pf1[j].im);
-      if constexpr (TWO) sh.s2[(tid >> 4) + 16 * j][tid & 15] = cmake<T>(sg2 * pf2[j].re, sg2 * pf2[j].im);
+        for (int e = 0; e < EPU; e++)
+          dst[(k / 9) * (16 * PG) + (k % 9) * 256 + e] =
+              x0 + e0 + e < V3 ? gload(src + x0 + ((k / 9) * (9 * PG) + k % 9) * PD.cs + e) : cmake<T>(0, 0);
     }
     __syncthreads();
-    if (prep_rot) {  // rotation to the physical basis on the staged tiles
-      if (P1.rot) rot_tile(sh.s1, P1.rot);
-      if (TWO && P2.rot) rot_tile(sh.s2, P2.rot);
+    if (P1.rot != 0 || (TWO && P2.rot != 0)) {
+      if (PD.rot) bq_rotate(tile[ds], PD.rot, thr, NT);
       __syncthreads();
     }
-    if (tile + (int)gridDim.x < ntiles) fetch(tile + gridDim.x);
-    const cx<T>(*S1)[BT_SP] = sh.s1;
-    const cx<T>(*S2)[BT_SP] = TWO ? sh.s2 : sh.s1;
-
-    cx<T> res[NOUT];
-    cx<T> pa1[9];
+    const bool in = x0 + site < V3;
+    cx<T> *o = out + ((x0 >> 4) * ncols + col0) * 16 + site;
+    // the 4 rows mu of column mu' = j: a wave's stores of a row cover 4 columns of 16 sites
+    auto put = [&](int g, T scale, const cx<T> (&r)[4]) {
+      if (in)
 #pragma unroll
-    for (int i = 0; i < 9; i++) pa1[i] = S1[pidx(hi, lo, 0, 0) + i][s];
-    // ---- mesons: lane p = (alpha, beta) forms G[p][p ^ (d,d)], lane op sums
-    if constexpr (MES) {
-      cx<T>(*g)[16] = reinterpret_cast<cx<T>(*)[16]>(&sh.w[s][0]);
-      static_for<0, 4>([&](auto d) {
-        const int q = lane ^ ((d.value << 2) | d.value);
-        cx<T> gv = cmake<T>(0, 0);
-#pragma unroll
-        for (int cc = 0; cc < 9; cc++) cfma_conj(gv, pa1[cc], d.value == 0 ? pa1[cc] : S1[q * 9 + cc][s]);
-        g[d.value][lane] = gv;
-      });
-      wave_lds_sync();
-      const int cX = c_mesonx.cls[lane];
-      cx<T> acc = cmake<T>(0, 0);
-#pragma unroll
-      for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int b = 0; b < 4; b++)
-          acc = acc + cmul_iph_rt(g[cX][a * 4 + b], c_mesonx.ph[lane][a ^ cX] + c_mesonx.ph[lane][b]);
-      res[0] = acc;
-      wave_lds_sync();
-    }
-    // ---- baryon blocks per dataset
-    static_for<0, ND>([&](auto dd) {
-      constexpr int d = dd.value;
-      const cx<T>(*P)[BT_SP] = d == 0 ? S1 : S2;
-      const cx<T>(*Qo)[BT_SP] = d == 0 ? S2 : S1;  // the proton's other flavour
-      cx<T> pa[9];
-#pragma unroll
-      for (int i = 0; i < 9; i++) pa[i] = d == 0 ? pa1[i] : P[pidx(hi, lo, 0, 0) + i][s];
-      constexpr int base = MOFF + d * NG;
-      cx<T> D[2], X[2];
-      // class of Cg5 and Cg3: proton with Delta_3 when both use this propagator
-      if constexpr (H0 && H3 && !TWO) {
-        baryon_group<T, 0, 3>(P, P, reinterpret_cast<cx<T>(*)[16][9]>(&sh.w[s][0]), s, lane, pa, D, X);
-        res[base + R0] = D[0] - X[0];
-        res[base + R3] = cmake<T>(2, 0) * D[1] - cmake<T>(4, 0) * X[1];
+        for (int m = 0; m < 4; m++) gstore(o + (int64_t)((MOFF + g) * 16 + 4 * m + j) * 16, scale * r[m]);
+    };
+    auto put_meson = [&](int op, cx<T> v) {
+      if (in) gstore(o + (int64_t)op * 16, v);
+    };
+    const cx<T> *P = tile[TWO ? ds : 0], *Qo = tile[TWO ? 1 - ds : 0];
+    const int base = ds * NG;
+    cx<T> R[2][4];
+    if (half == 0) {
+      if constexpr (H0 && HD && !TWO) {
+        bq_class<T, 0, 3, true>(P, P, site, j, R);
+        put(base + R0, -sgo, R[0]);
+        put(base + R3, -4 * sgp, R[1]);
       } else {
         if constexpr (H0) {
-          baryon_group<T, 0, -1>(P, Qo, reinterpret_cast<cx<T>(*)[16][9]>(&sh.w[s][0]), s, lane, pa, D, X);
-          res[base + R0] = D[0] - X[0];
+          bq_class<T, 0, -1, !TWO>(P, Qo, site, j, R);
+          put(base + R0, -sgo, R[0]);
         }
-        if constexpr (H3) {
-          baryon_group<T, 3, -1>(P, P, reinterpret_cast<cx<T>(*)[16][9]>(&sh.w[s][0]), s, lane, pa, D, X);
-          res[base + R3] = cmake<T>(2, 0) * D[0] - cmake<T>(4, 0) * X[0];
-        }
-      }
-      // class of Cg1 and Cg2
-      if constexpr (H1 && H2) {
-        baryon_group<T, 1, 2>(P, P, reinterpret_cast<cx<T>(*)[16][9]>(&sh.w[s][0]), s, lane, pa, D, X);
-        res[base + R1] = cmake<T>(2, 0) * D[0] - cmake<T>(4, 0) * X[0];
-        res[base + R2] = cmake<T>(2, 0) * D[1] - cmake<T>(4, 0) * X[1];
-      } else {
-        if constexpr (H1) {
-          baryon_group<T, 1, -1>(P, P, reinterpret_cast<cx<T>(*)[16][9]>(&sh.w[s][0]), s, lane, pa, D, X);
-          res[base + R1] = cmake<T>(2, 0) * D[0] - cmake<T>(4, 0) * X[0];
-        }
-        if constexpr (H2) {
-          baryon_group<T, 2, -1>(P, P, reinterpret_cast<cx<T>(*)[16][9]>(&sh.w[s][0]), s, lane, pa, D, X);
-          res[base + R2] = cmake<T>(2, 0) * D[0] - cmake<T>(4, 0) * X[0];
+        if constexpr (HD) {
+          bq_class<T, 3, -1, true>(P, P, site, j, R);
+          put(base + R3, -4 * sgp, R[0]);
         }
       }
-    });
-    // ---- stage [k][lane] per site in w, then coalesced stores along x
-    cx<T> *stage = &sh.w[0][0];
-    constexpr int SST = BT_WS;  // complex per site in w
-#pragma unroll
-    for (int k = 0; k < NOUT; k++) stage[s * SST + lane * 9 + k] = res[k];
-    __syncthreads();
-    {
-      const int ls = tid & 15;
-      const int64_t x = x0 + ls;
-      if (x < V3) {
-        const int64_t ncols = (int64_t)gridDim.y * nch_total, col0 = (int64_t)blockIdx.y * nch_total + ch0;
-        for (int ch = tid >> 4; ch < NOUT * 16; ch += BT_THREADS / BT_SITES)
-          gstore(out + ctile_idx(col0 + ch, x, ncols), stage[ls * SST + (ch & 15) * 9 + (ch >> 4)]);
+      if constexpr (MES && (HD || !H0)) bq_mesons<0, 2>(P, site, j, put_meson);
+    } else {
+      if constexpr (HD) {
+        bq_class<T, 1, 2, true>(P, P, site, j, R);
+        put(base + R1, -4 * sgp, R[0]);
+        put(base + R2, -4 * sgp, R[1]);
       }
+      if constexpr (MES && (HD || !H0)) bq_mesons<2, 4>(P, site, j, put_meson);
+      if constexpr (MES && H0 && !HD) bq_mesons<0, 4>(P, site, j, put_meson);
     }
-    __syncthreads();
   }
 }
 
 template <typename T, bool TWO, bool MES, int GM>
 static int launch_baryon_t(const PropDev<T> *props, const RowDev *rows, int nrows, cx<T> *out, int64_t V3,
                            int T_lat, int nch_total, int ch0, int tiles_per_block, hipStream_t st) {
-  const int ntiles = (int)((V3 + BT_SITES - 1) / BT_SITES);
+  const int ntiles = (int)((V3 + 15) / 16);
   const int gx = (ntiles + tiles_per_block - 1) / tiles_per_block;
-  dim3 grid((unsigned)gx, (unsigned)nrows), block(BT_THREADS);
-  size_t shm = sizeof(BaryonShared<T>);
-  if (!TWO) shm -= sizeof(cx<T>) * 144 * BT_SP;  // s2 is the last member
-  static bool attr_set = false;
-  if (!attr_set) {
-    if (hipFuncSetAttribute((const void *)k_baryon<T, TWO, MES, GM>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            (int)shm) != hipSuccess)
-      return PLG_ERR_HIP;
-    attr_set = true;
-  }
-  k_baryon<T, TWO, MES, GM><<<grid, block, shm, st>>>(props, rows, out, V3, T_lat, nch_total, ch0, ntiles);
+  dim3 grid((unsigned)gx, (unsigned)nrows), block(BqSplit<TWO, MES, GM>::threads);
+  k_baryon<T, TWO, MES, GM><<<grid, block, 0, st>>>(props, rows, out, V3, T_lat, nch_total, ch0, ntiles);
   return hipGetLastError() == hipSuccess ? PLG_OK : PLG_ERR_HIP;
 }
 
