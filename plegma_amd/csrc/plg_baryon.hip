@@ -62,49 +62,6 @@ template <typename T> struct BqT {
   static constexpr int EPU = sizeof(T) == 4 ? 2 : 1;  // sites of a 16-byte unit
   static constexpr int WPE = sizeof(T) == 4 ? 4 : 2;  // waves per SIMD (LDS and registers)
 };
-template <typename T, int N> struct BqVec;
-template <> struct BqVec<float, 2> {  // two sites; site pairs are 8-byte aligned
-  typedef float v __attribute__((ext_vector_type(4), aligned(8)));
-};
-template <> struct BqVec<double, 1> {
-  typedef double v __attribute__((ext_vector_type(2)));
-};
-
-// value of lane ^ S within the four lanes of a site
-template <int S> __device__ __forceinline__ float quad_xor(float v) {
-  if constexpr (S == 0) return v;
-  else return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), S == 1 ? 0xB1 : S == 2 ? 0x4E : 0x1B, 0xF, 0xF, true));
-}
-template <int S> __device__ __forceinline__ double quad_xor(double v) {
-  if constexpr (S == 0) return v;
-  else {
-    constexpr int ctrl = S == 1 ? 0xB1 : S == 2 ? 0x4E : 0x1B;
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_mov_dpp((int)b, ctrl, 0xF, 0xF, true);
-    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), ctrl, 0xF, 0xF, true);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-  }
-}
-template <typename T> __device__ __forceinline__ T quad_sum(T v) {
-  v += quad_xor<1>(v);
-  v += quad_xor<2>(v);
-  return v;
-}
-
-// sign of a phase table relative to its entry 0, as a character of the index
-constexpr bool bq_char_ok(const int (&ph)[4]) {
-  for (int n = 0; n < 4; n++)
-    if (((ph[n] - ph[0]) & 1) != 0) return false;
-  return ((ph[1] - ph[0] + ph[2] - ph[0]) & 3) == ((ph[3] - ph[0]) & 3);
-}
-// lane j's sign of a character
-template <typename T> __device__ __forceinline__ T bq_sign(const int (&ph)[4], int j) {
-  T s = 1;
-#pragma unroll
-  for (int n = 1; n < 4; n++) s = (j == n && ((ph[n] - ph[0]) & 3) == 2) ? (T)-1 : s;
-  return s;
-}
-
 // R[b][mu] (column mu' = j) of diquark W0 and, if W1 >= 0, of W1 of its class:
 // sum over nu', c, k of P (W + kappa delta tr W), up to the scale and lane
 // sign of bq_scale.  P, Q: the tiles at (lane, s = 0 column); SAME: Q = P
@@ -128,7 +85,7 @@ template <int W0, int W1> struct BqClass {
     for (int nu = 0; nu < 4; nu++)
       if (kind(nu) & 1) return false;
     if (cls && (((A0.ph[row(1) ^ cls] - A0.ph[row(1)]) & 3) != partner || (partner & 1))) return false;
-    return bq_char_ok(Ab0.ph) && bq_char_ok(Ab1.ph);
+    return char_ok(Ab0.ph) && char_ok(Ab1.ph);
   }
   // phase of Abar row nu' (character of nu', with the class shift as an offset)
   static constexpr int ab(int b, int n) { return b == 0 ? Ab0.ph[n ^ cls] : Ab1.ph[n ^ cls]; }
@@ -275,19 +232,10 @@ __device__ __forceinline__ void bq_class(const cx<T> *P, const cx<T> *Q, int sit
   // lane sign and phase of the results
   static_for<0, NB>([&](auto b_) {
     constexpr int b = b_.value;
-    const T sg = bq_sign<T>(b == 0 ? B::Ab0.ph : B::Ab1.ph, j);
+    const T sg = char_sign<T>(b == 0 ? B::Ab0.ph : B::Ab1.ph, j);
 #pragma unroll
     for (int m = 0; m < 4; m++) R[b][m] = sg * cmul_iph(R[b][m], B::phase(b));
   });
-}
-
-// phases of the meson channels: op, class and i^ph of X = g5 G per row
-constexpr MesonX BQ_X = make_mesonx();
-// the n-th op of xor class d
-constexpr int bq_op(int d, int n) {
-  for (int op = 0; op < 16; op++)
-    if (BQ_X.cls[op] == d && n-- == 0) return op;
-  return -1;
 }
 
 // mesons of the xor classes [D0, D1): G_d[al][be] = sum_cc S[al][be] conj(S[al^d][be^d]),
@@ -337,22 +285,14 @@ __device__ __forceinline__ void bq_mesons(const cx<T> *S, int site, int j, F &&s
     }
     cx<T> v[4];
     static_for<0, 4>([&](auto n) {
-      constexpr int op = bq_op(d, n.value);
-      static_assert(op >= 0 && bq_char_ok(BQ_X.ph[op < 0 ? 0 : op]), "four channels per class, sign characters");
+      constexpr int op = meson_op(d, n.value);
+      static_assert(op >= 0 && char_ok(MESON_X.ph[op < 0 ? 0 : op]), "four channels per class, sign characters");
       cx<T> w = cmake<T>(0, 0);
-      static_for<0, 4>([&](auto al) { w = w + cmul_iph(G[al.value], BQ_X.ph[op][al.value ^ d] + BQ_X.ph[op][0]); });
-      v[n.value] = bq_sign<T>(BQ_X.ph[op], j) * w;
+      static_for<0, 4>([&](auto al) { w = w + cmul_iph(G[al.value], MESON_X.ph[op][al.value ^ d] + MESON_X.ph[op][0]); });
+      v[n.value] = char_sign<T>(MESON_X.ph[op], j) * w;
     });
-    // sums over the four lanes, lane n keeping channel n
-    const bool odd = j & 1, hi = j & 2;
-    auto pick = [&](T a, T b, T c, T e) {
-      const T a1 = odd ? b : a, b1 = odd ? a : b, c1 = odd ? e : c, e1 = odd ? c : e;
-      const T lo2 = a1 + quad_xor<1>(b1), hi2 = c1 + quad_xor<1>(e1);
-      const T keep = hi ? hi2 : lo2, send = hi ? lo2 : hi2;
-      return keep + quad_xor<2>(send);
-    };
-    const int op = j == 0 ? bq_op(d, 0) : j == 1 ? bq_op(d, 1) : j == 2 ? bq_op(d, 2) : bq_op(d, 3);
-    store(op, cmake<T>(pick(v[0].re, v[1].re, v[2].re, v[3].re), pick(v[0].im, v[1].im, v[2].im, v[3].im)));
+    const int op = j == 0 ? meson_op(d, 0) : j == 1 ? meson_op(d, 1) : j == 2 ? meson_op(d, 2) : meson_op(d, 3);
+    store(op, quad_scatter_sum(v, j));
   });
 }
 
@@ -398,7 +338,7 @@ void k_baryon(const PropDev<T> *__restrict__ props, const RowDev *__restrict__ r
   // colour pairs of each (nu = g % 4: one LDS offset per thread)
   constexpr int EPU = BqT<T>::EPU, UPC = 16 / EPU, PG = NT / UPC, NH = 16 / PG, NU = 9 * NH;
   static_assert(PG % 4 == 0 && NH * PG == 16, "whole passes over the spin pairs");
-  typedef typename BqVec<T, EPU>::v vec;
+  typedef typename SiteVec<T, EPU>::v vec;
   __shared__ __align__(16) cx<T> tile[B::ND][BQ_TILE];
   const RowDev row = rows[blockIdx.y];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

@@ -1,21 +1,11 @@
 // plg_tile.h -- the site tile shared by the per-site contraction kernels
-// (baryons, fused two-point, meson-meson): 16 lattice sites per 256-thread
-// workgroup, 16 lanes (one DPP row of a wavefront) per site, propagator
-// components staged in LDS as [component][site].
+// (baryons, fused two-point, meson-meson): 16 lattice sites staged in LDS,
+// four lanes of a wavefront per site (a DPP quad), and the spin algebra those
+// lanes share.
 #pragma once
 #include "plg_internal.h"
 
 namespace plg {
-
-constexpr int BT_SITES = 16;  // sites per workgroup tile
-constexpr int BT_THREADS = 256;
-// LDS strides chosen for the access patterns of a wavefront (4 sites x 16
-// lanes, 8-byte complex = 2 banks): a component row of 17 sites makes the 16
-// lanes of a site that read components 9 l + i fall on 16 distinct bank
-// pairs; a per-site exchange stride of 292 (= 8 banks mod 32) keeps the 4
-// sites x 4 columns of transposed reads on distinct banks.
-constexpr int BT_SP = BT_SITES + 1;
-constexpr int BT_WS = 2 * 16 * 9 + 4;
 
 // per meson channel op (GAMMAS order): xor class and phases of X = g5 G
 struct MesonX {
@@ -31,63 +21,76 @@ constexpr MesonX make_mesonx() {
   }
   return m;
 }
-
-// ---- DPP row reductions (16-lane rows = the lanes of one site)
-template <int CTRL> __device__ __forceinline__ float dpp(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
+constexpr MesonX MESON_X = make_mesonx();
+// the n-th channel of xor class d (four each)
+constexpr int meson_op(int d, int n) {
+  for (int op = 0; op < 16; op++)
+    if (MESON_X.cls[op] == d && n-- == 0) return op;
+  return -1;
 }
+
+// ---- DPP row exchanges
 template <int CTRL> __device__ __forceinline__ double dpp(double v) {
   const long long b = __double_as_longlong(v);
   const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xF, 0xF, false);
   const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, false);
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
-template <typename T> __device__ __forceinline__ T rowsum16(T v) {
-  v += dpp<0xB1>(v);   // quad_perm [1,0,3,2]
-  v += dpp<0x4E>(v);   // quad_perm [2,3,0,1]
-  v += dpp<0x141>(v);  // row_half_mirror: the other quad of the half row
-  v += dpp<0x140>(v);  // row_mirror: the other half row
+
+// ---- staging of a tile: 16-byte units of EPU sites
+template <typename T, int N> struct SiteVec;
+template <> struct SiteVec<float, 2> {  // two sites; site pairs are 8-byte aligned
+  typedef float v __attribute__((ext_vector_type(4), aligned(8)));
+};
+template <> struct SiteVec<double, 1> {
+  typedef double v __attribute__((ext_vector_type(2)));
+};
+
+// value of lane ^ S within the four lanes of a site
+template <int S> __device__ __forceinline__ float quad_xor(float v) {
+  if constexpr (S == 0) return v;
+  else return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), S == 1 ? 0xB1 : S == 2 ? 0x4E : 0x1B, 0xF, 0xF, true));
+}
+template <int S> __device__ __forceinline__ double quad_xor(double v) {
+  if constexpr (S == 0) return v;
+  else {
+    constexpr int ctrl = S == 1 ? 0xB1 : S == 2 ? 0x4E : 0x1B;
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_mov_dpp((int)b, ctrl, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), ctrl, 0xF, 0xF, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+  }
+}
+template <typename T> __device__ __forceinline__ T quad_sum(T v) {
+  v += quad_xor<1>(v);
+  v += quad_xor<2>(v);
   return v;
 }
 
-// The 16 lanes of a site are one DPP row of one wavefront, so data a site's
-// lanes exchange through LDS needs ordering at wavefront scope only (LDS
-// operations of a wavefront complete in issue order).
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+// sign of a phase table relative to its entry 0, as a character of the index
+constexpr bool char_ok(const int (&ph)[4]) {
+  for (int n = 0; n < 4; n++)
+    if (((ph[n] - ph[0]) & 1) != 0) return false;
+  return ((ph[1] - ph[0] + ph[2] - ph[0]) & 3) == ((ph[3] - ph[0]) & 3);
 }
-
-// runtime phase i^ph (lane-dependent)
-template <typename T> __device__ __forceinline__ cx<T> cmul_iph_rt(cx<T> a, int ph) {
-  ph &= 3;
-  const T re = (ph & 1) ? -a.im : a.re;
-  const T im = (ph & 1) ? a.re : a.im;
-  return (ph & 2) ? cmake<T>(-re, -im) : cmake<T>(re, im);
-}
-
-// rotation to the physical basis of a staged tile S[component][site] in
-// place (all threads of the workgroup; the caller synchronises after it)
-template <typename T> __device__ __forceinline__ void rot_tile(cx<T> (*S)[BT_SP], int sign) {
-  for (int it = threadIdx.x; it < BT_SITES * 36; it += BT_THREADS) {
-    const int s = it % BT_SITES, cq = it / BT_SITES, cp = cq % 9, q = cq / 9, m = q >> 1, n = q & 1;
-    cx<T> a = S[(m * 4 + n) * 9 + cp][s], b = S[(m * 4 + n + 2) * 9 + cp][s];
-    cx<T> c = S[((m + 2) * 4 + n) * 9 + cp][s], d = S[((m + 2) * 4 + n + 2) * 9 + cp][s];
-    rot_physical(a, b, c, d, sign);
-    S[(m * 4 + n) * 9 + cp][s] = a;
-    S[(m * 4 + n + 2) * 9 + cp][s] = b;
-    S[((m + 2) * 4 + n) * 9 + cp][s] = c;
-    S[((m + 2) * 4 + n + 2) * 9 + cp][s] = d;
-  }
-}
-
-// entry i of a compile-time 4-vector at a runtime index (selects, no scratch)
-__device__ __forceinline__ int pick4(const int (&v)[4], int i) {
-  int r = 0;
+// lane j's sign of a character
+template <typename T> __device__ __forceinline__ T char_sign(const int (&ph)[4], int j) {
+  T s = 1;
 #pragma unroll
-  for (int k = 0; k < 4; k++) r += i == k ? v[k] : 0;
-  return r;
+  for (int n = 1; n < 4; n++) s = (j == n && ((ph[n] - ph[0]) & 3) == 2) ? (T)-1 : s;
+  return s;
+}
+// of four values per lane, the sums over the four lanes: lane n keeps value n
+template <typename T> __device__ __forceinline__ T quad_scatter_sum(T a, T b, T c, T d, int j) {
+  const bool odd = j & 1, hi = j & 2;
+  const T a1 = odd ? b : a, b1 = odd ? a : b, c1 = odd ? d : c, d1 = odd ? c : d;
+  const T lo2 = a1 + quad_xor<1>(b1), hi2 = c1 + quad_xor<1>(d1);
+  const T keep = hi ? hi2 : lo2, send = hi ? lo2 : hi2;
+  return keep + quad_xor<2>(send);
+}
+template <typename T> __device__ __forceinline__ cx<T> quad_scatter_sum(const cx<T> (&v)[4], int j) {
+  return cmake<T>(quad_scatter_sum(v[0].re, v[1].re, v[2].re, v[3].re, j),
+                  quad_scatter_sum(v[0].im, v[1].im, v[2].im, v[3].im, j));
 }
 
 }  // namespace plg
