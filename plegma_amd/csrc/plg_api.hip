@@ -47,8 +47,9 @@ struct Context {
   int M = 1;                     // lcm(Lx,Ly,Lz)
   double *d_cos = nullptr, *d_sin = nullptr;
   uint32_t *d_wtab = nullptr;    // [M][6] packed bf16 operand pairs (see plg_init)
-  // udsc baryon schedules on the device, built on first use per product
-  std::map<int, UdscSched> udsc;
+  // udsc baryon schedules on the device, built on first use per set of
+  // products, propagator order and precision
+  std::map<std::vector<int>, UdscAll> udsc;
   std::vector<void *> udsc_mem;
   // grow-only workspace
   void *ws_c = nullptr;
@@ -181,7 +182,7 @@ static int kind_shape(int kind, int mask, int &ng, int &nd, int &nch) {
 
 // ------------------------------------------------------------------ plans
 struct Launch {
-  enum { MESON, BARYON, MESMES, UDSC, TETRA } what;
+  enum { MESON, BARYON, MESMES, UDSC, TETRA, UDSC_ALL } what;
   int set;          // meson set
   bool two, mes;    // baryon
   int gmask;
@@ -228,8 +229,10 @@ struct Plan {
   // separable projection (both precisions): host tables and their device copy
   SepHost sep;
   void *d_sep = nullptr;
-  // udsc baryons: the flavour product's schedule (device arrays owned by the context)
+  // a caller's baryon table (device arrays owned by the caller of the plan)
   UdscSched udsc{};
+  // udsc baryons: the products' schedule (device arrays owned by the context)
+  UdscAll udsc_all{};
   // four-propagator tables: terms (owned by the caller of the plan) and rows
   TetraSched tetra{}, tetra2{};  // the table's two term sets (tetra2: views P1, P2, P4, P3)
   std::vector<RowDev4> rows4;
@@ -670,7 +673,7 @@ static std::string launch_name(const Plan &P, const Launch &l) {
   std::string t = P.T == PLG_F64 ? "f64" : "f32";
   if (l.what == Launch::MESON) return "contract_mesons_" + t;
   if (l.what == Launch::MESMES) return "contract_mesmes_" + t;
-  if (l.what == Launch::UDSC) return "contract_udsc_" + t;
+  if (l.what == Launch::UDSC || l.what == Launch::UDSC_ALL) return "contract_udsc_" + t;
   if (l.what == Launch::TETRA) return "contract_tetra_" + t;
   return std::string(l.mes ? "contract_twopt_" : "contract_baryons_") + t;
 }
@@ -685,6 +688,8 @@ template <typename T> static int launch_contract_t(const Plan &P, const Launch &
     return launch_mesmes<T>(pd, P.d_rows, nrows, (cx<T> *)c, g_ctx.V3, g_ctx.L[3], P.nch_c, l.ch0, P.tpb, st);
   case Launch::UDSC:
     return launch_udsc<T>(P.udsc, pd, P.d_rows, nrows, (cx<T> *)c, g_ctx.V3, g_ctx.L[3], P.nch_c, l.ch0, P.tpb, st);
+  case Launch::UDSC_ALL:
+    return launch_udsc_all<T>(P.udsc_all, pd, P.d_rows, nrows, (cx<T> *)c, g_ctx.V3, g_ctx.L[3], P.nch_c, st);
   case Launch::TETRA:  // set 1 runs on the second half of the rows (views P1, P2, P4, P3)
     return launch_tetra<T>(l.set ? P.tetra2 : P.tetra, pd, P.d_rows4 + (l.set ? nrows : 0), nrows, (cx<T> *)c,
                            g_ctx.V3, g_ctx.L[3], P.nch_c, P.tpb, st);
@@ -1381,38 +1386,45 @@ int plg_baryons_udsc_size(const plg_prop *up, const plg_prop *dn, const plg_prop
 }
 
 // the device schedule of a flavour product, uploaded once per context
-static int udsc_device_schedule(int prod, UdscSched &out) {
+static int udsc_device_schedule(const std::vector<int> &prods, const int fidx[4], int nprops, int T, UdscAll &out) {
   std::lock_guard<std::mutex> lk(g_mu);
-  auto it = g_ctx.udsc.find(prod);
+  std::vector<int> key = prods;
+  key.insert(key.end(), fidx, fidx + 4);
+  key.push_back(T);
+  auto it = g_ctx.udsc.find(key);
   if (it != g_ctx.udsc.end()) {
     out = it->second;
     return PLG_OK;
   }
-  UdscSchedHost h;
-  int rc = udsc_schedule(prod, h);
+  UdscAllHost h;
+  int rc = udsc_groups(prods, fidx, h);
   if (rc) return fail(rc, "udsc schedule");
-  short *q = nullptr;
-  signed char *t = nullptr;
-  uint16_t *e = nullptr;
-  float *c = nullptr;
-  if ((rc = upload(&q, h.quads, nullptr))) return rc;
-  g_ctx.udsc_mem.push_back(q);
-  if ((rc = upload(&t, h.tp, nullptr))) return rc;
-  g_ctx.udsc_mem.push_back(t);
-  if ((rc = upload(&e, h.ents, nullptr))) return rc;
-  g_ctx.udsc_mem.push_back(e);
-  if ((rc = upload(&c, h.coef, nullptr))) return rc;
-  g_ctx.udsc_mem.push_back(c);
-  h.s.quads = q;
-  h.s.tp = t;
-  h.s.ents = e;
-  h.s.coef = c;
-  g_ctx.udsc[prod] = h.s;
+  auto put = [&](auto &v, auto **d) {
+    const int r = upload(d, v, nullptr);
+    if (!r) g_ctx.udsc_mem.push_back(*d);
+    return r;
+  };
+  uint32_t *st = nullptr, *un = nullptr;
+  if ((rc = put(h.steps, &st))) return rc;
+  if ((rc = put(h.units, &un))) return rc;
+  if (T == PLG_F64) {
+    double *c = nullptr;
+    if ((rc = put(h.coef, &c))) return rc;
+    h.s.coef = c;
+  } else {
+    std::vector<float> cf(h.coef.begin(), h.coef.end());
+    float *c = nullptr;
+    if ((rc = put(cf, &c))) return rc;
+    h.s.coef = c;
+  }
+  h.s.nprops = nprops;
+  h.s.steps = st;
+  h.s.units = un;
+  g_ctx.udsc[key] = h.s;
   out = h.s;
   return PLG_OK;
 }
 
-// stage_ms (optional): summed per-stage milliseconds over the products
 static int udsc_check_args(const void *out, const int *source, int out_precision, int mode, int space,
                            const int *moms, int nmom) {
   if (!g_ctx.init) return fail(PLG_ERR_NOT_INIT, "plg_init not called");
@@ -1424,11 +1436,35 @@ static int udsc_check_args(const void *out, const int *source, int out_precision
   return PLG_OK;
 }
 
+// tables, workspace and launches of a plan of a single call, waited for
+static int plan_run(Plan &P, void *out, int out_precision, hipStream_t hs, std::map<std::string, double> *stage_ms) {
+  int rc;
+  if ((rc = upload_plan(P, hs))) return rc;
+  std::lock_guard<std::mutex> wl(g_ws_mu);  // until the stream is synchronised below
+  {
+    std::lock_guard<std::mutex> lk(g_mu);
+    if ((rc = ensure(&g_ctx.ws_c, &g_ctx.ws_c_bytes, c_bytes(P)))) return rc;
+    if ((rc = ensure(&g_ctx.ws_part, &g_ctx.ws_part_bytes, part_bytes(P)))) return rc;
+  }
+  StageLog log;
+  rc = enqueue(P, g_ctx.ws_c, g_ctx.ws_part, out, out_precision, hs, stage_ms ? &log : nullptr);
+  // the plan's tables are freed on return: wait for every launch, also after an error
+  const hipError_t se = hipStreamSynchronize(hs);
+  if (!rc && se != hipSuccess) rc = fail(PLG_ERR_HIP, "udsc sync failed");
+  for (size_t i = 0; i + 1 < log.ev.size(); i++) {
+    float t = 0;
+    if (!rc) hipEventElapsedTime(&t, log.ev[i], log.ev[i + 1]);
+    (*stage_ms)[log.name[i + 1]] += t;
+  }
+  for (hipEvent_t e : log.ev) hipEventDestroy(e);
+  return rc;
+}
+
 // one three-propagator table contraction (views S1, S2, S3 of the table),
 // its operators written as datasets d0 .. d0 + nops - 1 of the output
 static int udsc_one(const plg_prop *const views[3], const UdscSched &S, int nops, int d0, int nd_total,
                     const int source[4], int totalT, const int *moms, int nmom, int mode, int space, int out_precision,
-                    void *out, hipStream_t hs, std::map<std::string, double> *stage_ms) {
+                    void *out, hipStream_t hs) {
   int lt, rc;
   if ((rc = plg_window(source, totalT, nullptr, nullptr, &lt))) return rc;
   const Window w = window_of(g_ctx.L, source, totalT);
@@ -1480,25 +1516,7 @@ static int udsc_one(const plg_prop *const views[3], const UdscSched &S, int nops
   P.udsc = S;
   choose_tiles(P);
   P.tpb = 64;  // sites per workgroup of the udsc kernel
-  if ((rc = upload_plan(P, hs))) return rc;
-  std::lock_guard<std::mutex> wl(g_ws_mu);  // until the stream is synchronised below
-  {
-    std::lock_guard<std::mutex> lk(g_mu);
-    if ((rc = ensure(&g_ctx.ws_c, &g_ctx.ws_c_bytes, c_bytes(P)))) return rc;
-    if ((rc = ensure(&g_ctx.ws_part, &g_ctx.ws_part_bytes, part_bytes(P)))) return rc;
-  }
-  StageLog log;
-  rc = enqueue(P, g_ctx.ws_c, g_ctx.ws_part, out, out_precision, hs, stage_ms ? &log : nullptr);
-  // the plan's tables are freed on return: wait for every launch, also after an error
-  const hipError_t se = hipStreamSynchronize(hs);
-  if (!rc && se != hipSuccess) rc = fail(PLG_ERR_HIP, "udsc sync failed");
-  for (size_t i = 0; i + 1 < log.ev.size(); i++) {
-    float t = 0;
-    if (!rc) hipEventElapsedTime(&t, log.ev[i], log.ev[i + 1]);
-    (*stage_ms)[log.name[i + 1]] += t;
-  }
-  for (hipEvent_t e : log.ev) hipEventDestroy(e);
-  return rc;
+  return plan_run(P, out, out_precision, hs, nullptr);
 }
 
 static int udsc_run(const plg_prop *up, const plg_prop *dn, const plg_prop *st, const plg_prop *ch, int only_st,
@@ -1510,19 +1528,82 @@ static int udsc_run(const plg_prop *up, const plg_prop *dn, const plg_prop *st, 
   std::vector<int> prods;
   int nd_total;
   udsc_select(fl, only_st, only_ch, prods, nd_total);
-  int d0 = 0;
-  for (int prod : prods) {
-    const char *f = udsc_flavours(prod);
-    const plg_prop *views[3];
-    for (int i = 0; i < 3; i++)
-      views[i] = fl[std::find(UDSC_LETTERS, UDSC_LETTERS + 4, f[i]) - UDSC_LETTERS];
-    UdscSched S;
-    if ((rc = udsc_device_schedule(prod, S))) return rc;
-    const int nops = udsc_nops(prod);
-    if ((rc = udsc_one(views, S, nops, d0, nd_total, source, totalT, moms, nmom, mode, space, out_precision, out,
-                       (hipStream_t)stream, stage_ms)))
-      return rc;
-    d0 += nops;
+  if (prods.empty()) return PLG_OK;
+  int lt;
+  if ((rc = plg_window(source, totalT, nullptr, nullptr, &lt))) return rc;
+  const Window w = window_of(g_ctx.L, source, totalT);
+  const int T = g_ctx.L[3];
+  const int64_t V3 = g_ctx.V3;
+  const int64_t inner = space == PLG_MOMENTUM_SPACE ? (int64_t)nmom : V3;
+  // the propagators the products read, in the order u, d, s, c
+  int fidx[4] = {-1, -1, -1, -1};
+  std::vector<plg_prop> props;
+  for (int i = 0; i < 4; i++)
+    for (int prod : prods)
+      if (fidx[i] < 0 && std::strchr(udsc_flavours(prod), UDSC_LETTERS[i])) {
+        fidx[i] = (int)props.size();
+        props.push_back(*fl[i]);
+      }
+  UdscAll S;
+  const int prec = mode == PLG_MODE_F64 ? PLG_F64 : PLG_F32;
+  if ((rc = udsc_device_schedule(prods, fidx, (int)props.size(), prec, S))) return rc;
+  // The products of a call share one launch; the site correlator holds all
+  // their operators, so the time slices are taken in pieces that keep it
+  // within 1 GiB, or within what 16 operators over all slices take.
+  const int64_t row_bytes = (int64_t)nd_total * ctile_sites(V3) * (prec == PLG_F64 ? 16 : 8);
+  int64_t per = std::max<int64_t>((int64_t)1 << 30, row_bytes / nd_total * 16 * lt) / row_bytes;
+  per = std::max<int64_t>(1, std::min<int64_t>({per, lt, 32768 / nd_total}));
+  const int npiece = (int)((lt + per - 1) / per);
+  for (int ip = 0; ip < npiece; ip++) {
+    const int j0 = lt * ip / npiece, j1 = lt * (ip + 1) / npiece;
+    Plan P;
+    P.kind = -1;
+    P.mode = mode;
+    P.terms = PLG_SPLIT_BF16X6;
+    P.space = space;
+    P.T = prec;
+    P.props = props;
+    P.nmom = space == PLG_MOMENTUM_SPACE ? nmom : 0;
+    if (P.nmom) P.moms.assign(moms, moms + 3 * P.nmom);
+    P.ms = scaled_moms(P.moms.data(), P.nmom, 1);
+    if (P.nmom > 0) P.npairs = make_pairs(P.ms, g_ctx.M, P.pair_ms, P.mom_pair, &P.zero_pair);
+    P.nch_c = nd_total;
+    for (int j = j0; j < j1; j++) {
+      const int t = row_time(g_ctx.L, source, w, j);
+      for (const plg_prop &v : P.props)
+        if ((rc = check_prop(v, P.T, t))) return rc;
+      P.rows.push_back({t, 0, 0, 0, 0});
+    }
+    int d0 = 0;
+    for (int prod : prods) {
+      const char *f = udsc_flavours(prod);
+      const plg_prop *v[3];  // trilinear in the three views: one plane exponent of each
+      for (int i = 0; i < 3; i++) v[i] = &props[fidx[std::find(UDSC_LETTERS, UDSC_LETTERS + 4, f[i]) - UDSC_LETTERS]];
+      for (int k = 0; k < udsc_nops(prod); k++, d0++)
+        for (int j = j0; j < j1; j++) {
+          const int t = P.rows[j - j0].t;
+          OutRowDev o{};
+          o.crow = j - j0;
+          o.ch_base = d0;
+          o.nch_row = 1;
+          o.sx = source[0]; o.sy = source[1]; o.sz = source[2];
+          o.base = ((int64_t)d0 * lt + j) * inner;
+          auto plane = [&](const plg_prop &p) { return ((t - p.t_first) % T + T) % T; };
+          o.ea = v[0]->plane_exp; o.pla = plane(*v[0]); o.ka = 1;
+          o.eb = v[1]->plane_exp; o.plb = plane(*v[1]); o.kb = 1;
+          o.ec = v[2]->plane_exp; o.plc = plane(*v[2]); o.kc = 1;
+          P.orows.push_back(o);
+        }
+    }
+    P.csel = {0};
+    P.ch_off = {0};
+    P.m_stride = 1;
+    P.out_elems = (int64_t)nd_total * lt * inner;
+    P.nsites = (int64_t)(j1 - j0) * V3;
+    P.launches.push_back({Launch::UDSC_ALL, 0, false, false, 0, 0});
+    P.udsc_all = S;
+    choose_tiles(P);
+    if ((rc = plan_run(P, out, out_precision, (hipStream_t)stream, stage_ms))) return rc;
   }
   return PLG_OK;
 }
@@ -1902,8 +1983,7 @@ int plg_baryons_table(const plg_prop *p1, const plg_prop *p2, const plg_prop *p3
     h.s.ents = e;
     h.s.coef = c;
     const plg_prop *views[3] = {p1, p2, p3};
-    rc = udsc_one(views, h.s, nops, 0, nops, source, totalT, moms, nmom, mode, space, out_precision, out, hs,
-                  nullptr);
+    rc = udsc_one(views, h.s, nops, 0, nops, source, totalT, moms, nmom, mode, space, out_precision, out, hs);
   }
   hipStreamSynchronize(hs);  // no launch may still read the schedule
   for (void *p : mem) hipFree(p);

@@ -97,13 +97,44 @@ struct UdscSchedHost {
   std::vector<uint16_t> ents;
   std::vector<float> coef;
 };
-int udsc_schedule(int prod, UdscSchedHost &h);
 // one term of a table: six spin indices and a coefficient (the layout of the
 // generated tables, plg_udsc_tables.h)
 struct UdscTerm {
   signed char m[6];
   float re, im;
 };
+
+// The flavour products of one call in groups that share a pair of
+// propagators (pa, pb) and so the colour diquarks D of their spin pairs.
+// Product j of a group traces D with propagator third[j] into its nops[j]
+// operators, channels ch0[j]...  A wave's share of a group is nsteps steps
+// from step0.  Step, two words: the spin pairs of its four quads (m01 | m23
+// << 4, a byte each) and the term counts of the products (a byte each, the
+// largest of the four quads).  Per product the step's terms come in units of
+// four, numbered on from unit0: two words with the spin pair of the third
+// propagator (4 bits) of term e of quad i at bit 16 i + 4 e, and the
+// coefficients [quad i][operator k][term e] (0: no such term).
+constexpr int UD_WAVES = 8;       // waves of a workgroup
+constexpr int UD_NJ = 4;          // products of a group
+constexpr int UD_MAXGROUPS = 6;   // uu, dd, ss, cc, ud, sc
+struct UdscGroup {
+  int pa, pb, nprod;
+  int third[UD_NJ], nops[UD_NJ], ch0[UD_NJ];
+  int step0[UD_WAVES], nsteps[UD_WAVES], unit0[UD_WAVES];
+};
+struct UdscAll {
+  int ngroups, nprops;
+  UdscGroup g[UD_MAXGROUPS];
+  const uint32_t *steps, *units;
+  const void *coef;               // in the precision of the contraction
+};
+struct UdscAllHost {
+  UdscAll s{};
+  std::vector<uint32_t> steps, units;
+  std::vector<double> coef;
+};
+// fidx: the propagator of each flavour letter u, d, s, c
+int udsc_groups(const std::vector<int> &prods, const int fidx[4], UdscAllHost &h);
 int udsc_schedule_terms(const UdscTerm *terms, const int *first, const int *count, int nops, UdscSchedHost &h);
 
 // four-propagator table contractions (tetraquark table format)
@@ -149,6 +180,9 @@ const char *udsc_op_name(int prod, int k);
 template <typename T>
 int launch_udsc(const UdscSched &S, const PropDev<T> *props, const RowDev *rows, int nrows, cx<T> *out, int64_t V3,
                 int T_lat, int nch_total, int ch0, int spw, hipStream_t st);
+template <typename T>
+int launch_udsc_all(const UdscAll &S, const PropDev<T> *props, const RowDev *rows, int nrows, cx<T> *out, int64_t V3,
+                    int T_lat, int nch_total, hipStream_t st);
 
 template <typename T>
 int launch_meson(int set, const PropDev<T> *props, const RowDev *rows, int nrows, cx<T> *out,

@@ -5,24 +5,27 @@
 // fields by plegma_amd/gen_udsc.py).
 //
 // The reference gives every site one thread that walks all terms with its
-// three propagators in registers (PLEGMA_baryons_udsc.cu:86-121).  Here one
-// wave works on one site at a time with the site's 432 propagator entries in
-// LDS, and the terms are factorised through the colour "diquark" of the
-// first two propagators:
+// three propagators in registers (PLEGMA_baryons_udsc.cu:86-121).  Here the
+// terms are factorised through the colour "diquark" of two of the propagators:
 //   D_q[c][c'] = sum eps_abc eps_a'b'c' S1[m0m1][a][a'] S2[m2m3][b][b']   (q = m0m1, m2m3)
 //   T_m        = sum_cc' D_q[c][c'] S3[m4m5][c][c']                     (distinct terms m)
 //   O_k        = sum_m v_km T_m
-// Quads are processed in chunks of 64, one per lane: the lane forms D_q in
-// registers and the (at most four) distinct terms of its quad, which go to
-// LDS slots; then each operator sums its entries over those slots (4 lanes per
-// operator).  D costs 36 complex products per quad, a term 9, an entry 1.
+// The built-in products of a call share one launch (k_udsc_all, below).  A
+// caller's table (k_udsc): one wave works on one site at a time with the
+// site's 432 propagator entries in LDS; quads are processed in chunks of 64,
+// one per lane: the lane forms D_q in registers and the (at most four)
+// distinct terms of its quad, which go to LDS slots; then each operator sums
+// its entries over those slots (4 lanes per operator).  D costs 36 complex products per quad, a term 9, an entry 1.
 // A workgroup stages whole 128-byte lines of the propagators (16 FP32 or 8
 // FP64 consecutive sites), so every line is read from HBM once.
 #include "plg_internal.h"
 #include "plg_udsc_tables.h"
 
 #include <algorithm>
+#include <array>
+#include <cstring>
 #include <map>
+#include <string>
 #include <vector>
 
 namespace plg {
@@ -174,16 +177,162 @@ int udsc_schedule_terms(const UdscTerm *terms, const int *first, const int *coun
   return PLG_OK;
 }
 
-// the schedule of a flavour product of the built-in tables
-int udsc_schedule(int prod, UdscSchedHost &h) {
-  if (prod < 0 || prod >= UDSC_NPROD) return PLG_ERR_INVALID;
-  const UdscProd &P = UDSC_PRODS[prod];
-  std::vector<int> first(P.nops), count(P.nops);
-  for (int k = 0; k < P.nops; k++) {
-    first[k] = UDSC_OPS[P.first_op + k].first;
-    count[k] = UDSC_OPS[P.first_op + k].count;
+// ------------------------------------------------------------------ built-in products
+// The flavour products of one call, grouped by the pair of propagators whose
+// colour diquarks they share.  The colour structure is symmetric under an
+// exchange of the three propagators with their spin pairs, so a product may
+// take any two of its flavours as the pair:
+//  - two equal flavours are the pair (uuc, uud, uus and uuu share the diquarks
+//    of uu), and D of the spin pairs (a, b) equals D of (b, a): 136 quads
+//    instead of 256, and terms that differ by the exchange are one term (uuu:
+//    by all exchanges of the three);
+//  - of three different flavours u, d if both are there, else s, c (udc and
+//    uds share ud; usc and dsc share sc).
+// All 20 products: 1056 quads and 8.7 k terms instead of 4928 and 12.1 k.
+int udsc_groups(const std::vector<int> &prods, const int fidx[4], UdscAllHost &h) {
+  static const char letters[5] = "udsc";
+  struct Key {
+    int a, b;
+    bool operator<(const Key &o) const { return a != o.a ? a < o.a : b < o.b; }
+  };
+  struct Item {
+    int prod, third, perm[3], ch0;
+  };
+  std::map<Key, std::vector<Item>> by_pair;
+  int ch = 0;
+  for (int prod : prods) {
+    const char *f = UDSC_PRODS[prod].flavours;
+    Item it;
+    it.prod = prod;
+    it.ch0 = ch;
+    ch += UDSC_PRODS[prod].nops;
+    int x = 0, y = 1;  // the positions of the pair
+    if (f[0] == f[1]) x = 0, y = 1;
+    else if (f[1] == f[2]) x = 1, y = 2;
+    else if (f[0] == f[2]) x = 0, y = 2;
+    else {
+      const std::string fs(f, 3);
+      const bool ud = fs.find('u') != std::string::npos && fs.find('d') != std::string::npos;
+      x = (int)fs.find(ud ? 'u' : 's');
+      y = (int)fs.find(ud ? 'd' : 'c');
+    }
+    const int z = 3 - x - y;
+    it.perm[0] = x;
+    it.perm[1] = y;
+    it.perm[2] = z;
+    auto fl = [&](int i) { return fidx[std::strchr(letters, f[i]) - letters]; };
+    it.third = fl(z);
+    by_pair[Key{fl(x), fl(y)}].push_back(it);
   }
-  return udsc_schedule_terms(UDSC_TERMS, first.data(), count.data(), P.nops, h);
+  h = UdscAllHost{};
+  for (auto &kv : by_pair) {
+    if ((int)kv.second.size() > UD_NJ || h.s.ngroups >= UD_MAXGROUPS) return PLG_ERR_UNSUPPORTED;
+    UdscGroup &G = h.s.g[h.s.ngroups++];
+    G.pa = kv.first.a;
+    G.pb = kv.first.b;
+    G.nprod = (int)kv.second.size();
+    // quad -> per product: spin pair of the third propagator -> coefficient of every operator
+    typedef std::map<int, std::array<double, UD_MAXOPS>> Terms;
+    std::map<int, std::array<Terms, UD_NJ>> quads;
+    for (int j = 0; j < G.nprod; j++) {
+      const Item &it = kv.second[j];
+      const UdscProd &P = UDSC_PRODS[it.prod];
+      if (P.nops > UD_MAXOPS) return PLG_ERR_UNSUPPORTED;
+      G.third[j] = it.third;
+      G.nops[j] = P.nops;
+      G.ch0[j] = it.ch0;
+      for (int k = 0; k < P.nops; k++) {
+        const UdscOp &op = UDSC_OPS[P.first_op + k];
+        for (int i = 0; i < op.count; i++) {
+          const UdscTerm &t = UDSC_TERMS[op.first + i];
+          if (t.im != 0.f) return PLG_ERR_UNSUPPORTED;
+          int sp[3];
+          for (int v = 0; v < 3; v++) sp[v] = t.m[2 * it.perm[v]] * 4 + t.m[2 * it.perm[v] + 1];
+          if (G.pa == G.pb) {
+            if (it.third == G.pa) std::sort(sp, sp + 3);
+            else if (sp[0] > sp[1]) std::swap(sp[0], sp[1]);
+          }
+          auto &T = quads[sp[0] | sp[1] << 4][j];
+          auto e = T.emplace(sp[2], std::array<double, UD_MAXOPS>{}).first;
+          e->second[k] += (double)t.re;
+        }
+      }
+    }
+    for (auto &q : quads)  // terms whose coefficients cancelled
+      for (auto &T : q.second)
+        for (auto e = T.begin(); e != T.end();)
+          e = std::all_of(e->second.begin(), e->second.end(), [](double v) { return v == 0; }) ? T.erase(e)
+                                                                                              : std::next(e);
+    // steps of four quads with like term counts, most terms first
+    typedef std::pair<const int, std::array<Terms, UD_NJ>> Quad;
+    std::vector<const Quad *> order;
+    for (const Quad &q : quads) order.push_back(&q);
+    auto nterms = [](const Quad *q) {
+      size_t n = 0;
+      for (auto &T : q->second) n += T.size();
+      return n;
+    };
+    std::stable_sort(order.begin(), order.end(), [&](const Quad *a, const Quad *b) {
+      const size_t na = nterms(a), nb = nterms(b);
+      if (na != nb) return na > nb;
+      for (int j = 0; j < UD_NJ; j++)
+        if (a->second[j].size() != b->second[j].size()) return a->second[j].size() > b->second[j].size();
+      return false;
+    });
+    const int nsteps = ((int)order.size() + 3) / 4;
+    auto step_count = [&](int st, int j) {
+      size_t n = 0;
+      for (int i = 4 * st; i < std::min(4 * st + 4, (int)order.size()); i++) n = std::max(n, order[i]->second[j].size());
+      return (int)n;
+    };
+    // the steps go to the wave with the least work so far
+    std::vector<std::vector<int>> mine(UD_WAVES);
+    int load[UD_WAVES] = {0};
+    for (int st = 0; st < nsteps; st++) {
+      int cost = 5;  // a diquark costs four terms, and its loads
+      for (int j = 0; j < UD_NJ; j++) cost += step_count(st, j);
+      const int w = (int)(std::min_element(load, load + UD_WAVES) - load);
+      load[w] += cost;
+      mine[w].push_back(st);
+    }
+    for (int w = 0; w < UD_WAVES; w++) {
+      G.step0[w] = (int)h.steps.size() / 2;
+      G.nsteps[w] = (int)mine[w].size();
+      G.unit0[w] = (int)h.units.size() / 2;
+      for (int st : mine[w]) {
+        uint32_t qw = 0, cw = 0;
+        for (int i = 0; i < 4; i++)
+          if (4 * st + i < (int)order.size()) qw |= (uint32_t)order[4 * st + i]->first << (8 * i);
+        for (int j = 0; j < UD_NJ; j++) cw |= (uint32_t)step_count(st, j) << (8 * j);
+        h.steps.push_back(qw);
+        h.steps.push_back(cw);
+        for (int j = 0; j < UD_NJ; j++) {
+          const int n = step_count(st, j);
+          for (int e0 = 0; e0 < n; e0 += 4) {  // a unit: four terms of each of the step's quads
+            uint64_t pw = 0;
+            const size_t c0 = h.coef.size();
+            h.coef.resize(c0 + 256, 0.0);
+            for (int i = 0; i < 4; i++) {
+              if (4 * st + i >= (int)order.size()) continue;
+              const Terms &T = order[4 * st + i]->second[j];
+              auto e = T.begin();
+              for (int u = 0; u < e0 && e != T.end(); u++) ++e;
+              for (int u = 0; u < 4 && e != T.end(); u++, ++e) {
+                pw |= (uint64_t)e->first << (16 * i + 4 * u);
+                for (int k = 0; k < UD_MAXOPS; k++) h.coef[c0 + (i * 16 + k) * 4 + u] = e->second[k];
+              }
+            }
+            h.units.push_back((uint32_t)pw);
+            h.units.push_back((uint32_t)(pw >> 32));
+          }
+        }
+      }
+    }
+  }
+  // the kernel loads a wave's next unit ahead of its use
+  h.units.resize(h.units.size() + 2, 0u);
+  h.coef.resize(h.coef.size() + 256, 0.0);
+  return PLG_OK;
 }
 
 int udsc_products() { return UDSC_NPROD; }
@@ -206,6 +355,39 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// D[c][c'] = sum eps_abc eps_a'b'c' a[a][a'] b[b][b']
+template <typename T>
+__device__ __forceinline__ void udsc_diquark(const cx<T> (&a)[9], const cx<T> (&b)[9], cx<T> (&d)[9]) {
+#pragma unroll
+  for (int cc = 0; cc < 3; cc++) {
+    const int a1 = (cc + 1) % 3, a2 = (cc + 2) % 3;
+#pragma unroll
+    for (int dd = 0; dd < 3; dd++) {
+      const int e1 = (dd + 1) % 3, e2 = (dd + 2) % 3;
+      // + a[a1][e1] b[a2][e2] - a[a1][e2] b[a2][e1] - a[a2][e1] b[a1][e2] + a[a2][e2] b[a1][e1]
+      const cx<T> p0 = a[a1 * 3 + e1], q0 = b[a2 * 3 + e2], p1 = a[a1 * 3 + e2], q1 = b[a2 * 3 + e1];
+      const cx<T> p2 = a[a2 * 3 + e1], q2 = b[a1 * 3 + e2], p3 = a[a2 * 3 + e2], q3 = b[a1 * 3 + e1];
+      T re = p0.re * q0.re;
+      re = fma(-p0.im, q0.im, re);
+      re = fma(-p1.re, q1.re, re);
+      re = fma(p1.im, q1.im, re);
+      re = fma(-p2.re, q2.re, re);
+      re = fma(p2.im, q2.im, re);
+      re = fma(p3.re, q3.re, re);
+      re = fma(-p3.im, q3.im, re);
+      T im = p0.re * q0.im;
+      im = fma(p0.im, q0.re, im);
+      im = fma(-p1.re, q1.im, im);
+      im = fma(-p1.im, q1.re, im);
+      im = fma(-p2.re, q2.im, im);
+      im = fma(-p2.im, q2.re, im);
+      im = fma(p3.re, q3.im, im);
+      im = fma(p3.im, q3.re, im);
+      d[cc * 3 + dd] = cmake<T>(re, im);
+    }
+  }
+}
+
 template <typename T> struct UdscGeom {
   static constexpr int G = 128 / (int)sizeof(cx<T>);  // sites per line
   static constexpr int SPAD = 433;                    // LDS stride of a site (432 + 1)
@@ -213,7 +395,7 @@ template <typename T> struct UdscGeom {
   static constexpr int NT = 64 * W;
 };
 
-// RC: every coefficient is real (the built-in tables), an entry costs two
+// RC: every coefficient is real (as in the built-in tables), an entry costs two
 // FMAs instead of a complex product
 template <typename T, bool RC>
 __global__ __launch_bounds__(64 * UdscGeom<T>::W) void k_udsc(UdscSched S, const PropDev<T> *__restrict__ props,
@@ -315,34 +497,7 @@ __global__ __launch_bounds__(64 * UdscGeom<T>::W) void k_udsc(UdscSched S, const
             a[j] = A[j];
             b[j] = B[j];
           }
-#pragma unroll
-          for (int cc = 0; cc < 3; cc++) {
-            const int a1 = (cc + 1) % 3, a2 = (cc + 2) % 3;
-#pragma unroll
-            for (int dd = 0; dd < 3; dd++) {
-              const int e1 = (dd + 1) % 3, e2 = (dd + 2) % 3;
-              // + a[a1][e1] b[a2][e2] - a[a1][e2] b[a2][e1] - a[a2][e1] b[a1][e2] + a[a2][e2] b[a1][e1]
-              const cx<T> p0 = a[a1 * 3 + e1], q0 = b[a2 * 3 + e2], p1 = a[a1 * 3 + e2], q1 = b[a2 * 3 + e1];
-              const cx<T> p2 = a[a2 * 3 + e1], q2 = b[a1 * 3 + e2], p3 = a[a2 * 3 + e2], q3 = b[a1 * 3 + e1];
-              T re = p0.re * q0.re;
-              re = fma(-p0.im, q0.im, re);
-              re = fma(-p1.re, q1.re, re);
-              re = fma(p1.im, q1.im, re);
-              re = fma(-p2.re, q2.re, re);
-              re = fma(p2.im, q2.im, re);
-              re = fma(p3.re, q3.re, re);
-              re = fma(-p3.im, q3.im, re);
-              T im = p0.re * q0.im;
-              im = fma(p0.im, q0.re, im);
-              im = fma(-p1.re, q1.im, im);
-              im = fma(-p1.im, q1.re, im);
-              im = fma(-p2.re, q2.im, im);
-              im = fma(-p2.im, q2.re, im);
-              im = fma(p3.re, q3.im, im);
-              im = fma(p3.im, q3.re, im);
-              d[cc * 3 + dd] = cmake<T>(re, im);
-            }
-          }
+          udsc_diquark(a, b, d);
           // its distinct terms T = sum_cc' D[c][c'] S3[m4m5][c][c']
 #pragma unroll
           for (int e = 0; e < UD_TPQ; e++) {
@@ -412,5 +567,178 @@ template int launch_udsc<double>(const UdscSched &, const PropDev<double> *, con
                                  int64_t, int, int, int, int, hipStream_t);
 template int launch_udsc<float>(const UdscSched &, const PropDev<float> *, const RowDev *, int, cx<float> *,
                                 int64_t, int, int, int, int, hipStream_t);
+
+// ------------------------------------------------------------------ all products of a call
+// The contraction of a call's flavour products in one launch.  A workgroup of
+// 8 waves stages the four flavours of 16 consecutive sites in LDS, entries
+// outermost (a row of 16 sites is 128 or 256 bytes), and the lane of site s
+// and quarter q = lane / 16 forms the diquark of its quarter's quad of the
+// step, then its terms, so that the schedule is uniform over the wave and a
+// term's 64 values (16 sites, 4 quads) are, as they lie in the registers, the
+// B operand of a 16x16x4 matrix product with the coefficients of the 16
+// operators: O[k][site] += sum_q V[k][term of quad q] T[q][site], for the
+// real and the imaginary part.  The waves share a group's steps and their
+// sums meet in LDS at the group's end.
+// Bound by the vector unit and LDS (a term is 36 FMAs, two matrix instructions
+// and 9 reads; of 9.2 M cycles the FMAs take 4.5 M, the matrix instructions
+// 1.9 M, LDS is busy 5.5 M).  20 products on 24^3 x 16 sites, FP32: 20 launches
+// of k_udsc, 0.5 ms each -> 4.2 ms, the call 14.5 -> 4.4 ms.  k_udsc reads the
+// terms, coefficients and entry indexes of its operator sums and every
+// diquark's blocks from LDS 20 times per site, and is bound there.
+template <typename T> struct UdAcc;
+template <> struct UdAcc<float> {
+  typedef float v4 __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ v4 mma(float a, float b, v4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane >> 4) + r; }
+};
+template <> struct UdAcc<double> {
+  typedef double v4 __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ v4 mma(double a, double b, v4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int lane, int r) { return 4 * r + (lane >> 4); }
+};
+
+template <typename T>
+__global__ __launch_bounds__(64 * UD_WAVES, sizeof(T) == 4 ? 4 : 2) void k_udsc_all(
+    UdscAll S, const PropDev<T> *__restrict__ props, const RowDev *__restrict__ rows, cx<T> *__restrict__ out,
+    int64_t V3, int T_lat, int nch_total, int groups_per_block) {
+  typedef typename UdAcc<T>::v4 v4;
+  constexpr int NT = 64 * UD_WAVES;
+  __shared__ cx<T> sp[4 * 144 * 16];        // [flavour][m01][c c'][site]
+  __shared__ T red[UD_WAVES][256];          // the waves' sums of one product, real or imaginary
+  const int tid = threadIdx.x, lane = tid & 63, s = tid & 15, kq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const RowDev row = rows[blockIdx.y];
+  const int64_t x0 = (int64_t)blockIdx.x * 16;
+  {
+    const bool xin = x0 + s < V3;
+#pragma unroll
+    for (int f = 0; f < 4; f++) {
+      if (f >= S.nprops) break;
+      const PropDev<T> Q = props[f];
+      int plane = row.t - Q.t_first;
+      plane += plane < 0 ? T_lat : 0;
+      const cx<T> *b = Q.data + (int64_t)plane * V3 + x0 + s;
+#pragma unroll
+      for (int i = 0; i < (144 * 16 + NT - 1) / NT; i++) {
+        const int c = i * (NT / 16) + (tid >> 4);
+        if (c < 144) sp[(f * 144 + c) * 16 + s] = xin ? gload(b + (int64_t)c * Q.cs) : cmake<T>(0, 0);
+      }
+    }
+  }
+  __syncthreads();
+  int rot_any = 0;
+  for (int f = 0; f < S.nprops; f++) rot_any |= props[f].rot;
+  if (rot_any) {  // rotation to the physical basis, per (site, propagator, colour pair)
+    for (int k = tid; k < S.nprops * 9 * 16; k += NT) {
+      const int f = k / 144, cc = (k >> 4) % 9, rot = props[f].rot;
+      if (rot) {
+        cx<T> *b = sp + (f * 144 + cc) * 16 + (k & 15);
+        cx<T> w[16];
+#pragma unroll
+        for (int m = 0; m < 16; m++) w[m] = b[m * 9 * 16];
+        rot_spins(w, rot);
+#pragma unroll
+        for (int m = 0; m < 16; m++) b[m * 9 * 16] = w[m];
+      }
+    }
+    __syncthreads();
+  }
+  const int64_t ncols = (int64_t)gridDim.y * nch_total, col0 = (int64_t)blockIdx.y * nch_total;
+  const v4 *coef = (const v4 *)S.coef + lane;
+  const int g1 = min((int)(blockIdx.z + 1) * groups_per_block, S.ngroups);
+  for (int gi = blockIdx.z * groups_per_block; gi < g1; gi++) {
+    const UdscGroup &G = S.g[gi];
+    v4 ar[UD_NJ], ai[UD_NJ];
+#pragma unroll
+    for (int j = 0; j < UD_NJ; j++) ar[j] = ai[j] = (v4)(T)0;
+    const cx<T> *A = sp + G.pa * 2304 + s, *B = sp + G.pb * 2304 + s;
+    const int st0 = G.step0[wave], nst = G.nsteps[wave];
+    int un = G.unit0[wave];
+    v4 cf = coef[un * 64];
+    for (int st = st0; st < st0 + nst; st++) {
+      const uint32_t qw = S.steps[2 * st], cw = S.steps[2 * st + 1];
+      const int q = (qw >> (8 * kq)) & 255;
+      cx<T> d[9];
+      {
+        const cx<T> *Aq = A + (q & 15) * 144, *Bq = B + (q >> 4) * 144;
+        cx<T> a[9], b[9];
+#pragma unroll
+        for (int j = 0; j < 9; j++) {
+          a[j] = Aq[j * 16];
+          b[j] = Bq[j * 16];
+        }
+        udsc_diquark(a, b, d);
+      }
+#pragma unroll
+      for (int j = 0; j < UD_NJ; j++) {
+        const int nt = (cw >> (8 * j)) & 255;
+        if (nt == 0) continue;
+        const cx<T> *C = sp + G.third[j] * 2304 + s;
+        for (int e0 = 0; e0 < nt; e0 += 4, un++) {
+          const uint64_t pw = (uint64_t)S.units[2 * un] | (uint64_t)S.units[2 * un + 1] << 32;
+          const int pl = (int)(pw >> (16 * kq)) & 0xffff;
+          const v4 cn = coef[(un + 1) * 64];  // the next unit's
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            if (e0 + e >= nt) break;
+            const cx<T> *Cp = C + ((pl >> (4 * e)) & 15) * 144;
+            cx<T> t = cmake<T>(0, 0);
+#pragma unroll
+            for (int c = 0; c < 9; c++) cfma(t, d[c], Cp[c * 16]);
+            ar[j] = UdAcc<T>::mma(cf[e], t.re, ar[j]);
+            ai[j] = UdAcc<T>::mma(cf[e], t.im, ai[j]);
+          }
+          cf = cn;
+        }
+      }
+    }
+    // the waves' sums
+    const T sgp = prop_sign(props[G.pa], row.t) * prop_sign(props[G.pb], row.t);
+#pragma unroll
+    for (int j = 0; j < UD_NJ; j++) {
+      if (j >= G.nprod) break;
+      T o[2];
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) red[wave][r * 64 + lane] = h ? ai[j][r] : ar[j][r];
+        __syncthreads();
+        if (tid < 256) {
+          T v = red[0][tid];
+#pragma unroll
+          for (int w = 1; w < UD_WAVES; w++) v += red[w][tid];
+          o[h] = v;
+        }
+        __syncthreads();
+      }
+      const int k = UdAcc<T>::row(lane, wave);
+      if (tid < 256 && k < G.nops[j] && x0 + s < V3) {
+        const T sg = sgp * prop_sign(props[G.third[j]], row.t);
+        gstore(out + ctile_idx(col0 + G.ch0[j] + k, x0 + s, ncols), cmake<T>(sg * o[0], sg * o[1]));
+      }
+    }
+  }
+}
+
+template <typename T>
+int launch_udsc_all(const UdscAll &S, const PropDev<T> *props, const RowDev *rows, int nrows, cx<T> *out, int64_t V3,
+                    int T_lat, int nch_total, hipStream_t st) {
+  const int64_t tiles = (V3 + 15) / 16;
+  // few tiles: the groups go to workgroups of their own until the chip is full
+  const int split = (int)std::max<int64_t>(1, std::min<int64_t>(S.ngroups, 512 / std::max<int64_t>(1, tiles * nrows)));
+  const int gpb = (S.ngroups + split - 1) / split;
+  dim3 grid((unsigned)tiles, (unsigned)nrows, (unsigned)((S.ngroups + gpb - 1) / gpb));
+  k_udsc_all<T><<<grid, 64 * UD_WAVES, 0, st>>>(S, props, rows, out, V3, T_lat, nch_total, gpb);
+  return hipGetLastError() == hipSuccess ? PLG_OK : PLG_ERR_HIP;
+}
+
+template int launch_udsc_all<double>(const UdscAll &, const PropDev<double> *, const RowDev *, int, cx<double> *,
+                                     int64_t, int, int, hipStream_t);
+template int launch_udsc_all<float>(const UdscAll &, const PropDev<float> *, const RowDev *, int, cx<float> *,
+                                    int64_t, int, int, hipStream_t);
 
 }  // namespace plg
