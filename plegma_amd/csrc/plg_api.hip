@@ -233,10 +233,8 @@ struct Plan {
   UdscSched udsc{};
   // udsc baryons: the products' schedule (device arrays owned by the context)
   UdscAll udsc_all{};
-  // four-propagator tables: terms (owned by the caller of the plan) and rows
-  TetraSched tetra{}, tetra2{};  // the table's two term sets (tetra2: views P1, P2, P4, P3)
-  std::vector<RowDev4> rows4;
-  RowDev4 *d_rows4 = nullptr;
+  // four-propagator tables (device arrays kept by the caller of the plan)
+  std::vector<TetraSched> tetra;
   // batch-owned workspace (single calls use the context workspace)
   void *c = nullptr, *part = nullptr;
   size_t c_bytes = 0, part_bytes = 0;
@@ -252,7 +250,7 @@ struct Plan {
     if (graph) hipGraphDestroy(graph);
     if (cap_stream) hipStreamDestroy(cap_stream);
     for (void *p : {(void *)d_props, (void *)d_rows, (void *)d_orows, (void *)d_csel, (void *)d_choff, (void *)d_ms,
-                    (void *)d_pair_ms, (void *)d_mom_pair, (void *)d_pidx, (void *)d_rows4, d_sep})
+                    (void *)d_pair_ms, (void *)d_mom_pair, (void *)d_pidx, d_sep})
       if (p) hipFree(p);
     if (own_ws) {
       if (c) hipFree(c);
@@ -690,9 +688,8 @@ template <typename T> static int launch_contract_t(const Plan &P, const Launch &
     return launch_udsc<T>(P.udsc, pd, P.d_rows, nrows, (cx<T> *)c, g_ctx.V3, g_ctx.L[3], P.nch_c, l.ch0, P.tpb, st);
   case Launch::UDSC_ALL:
     return launch_udsc_all<T>(P.udsc_all, pd, P.d_rows, nrows, (cx<T> *)c, g_ctx.V3, g_ctx.L[3], P.nch_c, st);
-  case Launch::TETRA:  // set 1 runs on the second half of the rows (views P1, P2, P4, P3)
-    return launch_tetra<T>(l.set ? P.tetra2 : P.tetra, pd, P.d_rows4 + (l.set ? nrows : 0), nrows, (cx<T> *)c,
-                           g_ctx.V3, g_ctx.L[3], P.nch_c, P.tpb, st);
+  case Launch::TETRA:
+    return launch_tetra<T>(P.tetra[l.set], pd, P.d_rows, nrows, (cx<T> *)c, g_ctx.V3, g_ctx.L[3], P.nch_c, l.ch0, st);
   default:
     return launch_baryon<T>(l.two, l.mes, l.gmask, pd, P.d_rows, nrows, (cx<T> *)c, g_ctx.V3, g_ctx.L[3],
                             P.nch_c, l.ch0, P.tpb, st);
@@ -1100,6 +1097,7 @@ int plg_version(void) { return 100; }
 const char *plg_last_error(void) { return g_err.c_str(); }
 
 static void finalize_locked();
+static void tetra_tables_clear();
 
 int plg_init(const int L[4], int device) {
   std::lock_guard<std::mutex> sl(g_static_mu);
@@ -1172,6 +1170,7 @@ static void finalize_locked() {
   hipDeviceSynchronize();
   g_single.clear();
   g_ft.release();
+  tetra_tables_clear();
   for (void *p : {(void *)g_ctx.d_cos, (void *)g_ctx.d_sin, (void *)g_ctx.d_wtab, g_ctx.ws_c, g_ctx.ws_part})
     if (p) hipFree(p);
   for (void *p : g_ctx.udsc_mem) hipFree(p);
@@ -1450,7 +1449,7 @@ static int plan_run(Plan &P, void *out, int out_precision, hipStream_t hs, std::
   rc = enqueue(P, g_ctx.ws_c, g_ctx.ws_part, out, out_precision, hs, stage_ms ? &log : nullptr);
   // the plan's tables are freed on return: wait for every launch, also after an error
   const hipError_t se = hipStreamSynchronize(hs);
-  if (!rc && se != hipSuccess) rc = fail(PLG_ERR_HIP, "udsc sync failed");
+  if (!rc && se != hipSuccess) rc = fail(PLG_ERR_HIP, "synchronisation failed");
   for (size_t i = 0; i + 1 < log.ev.size(); i++) {
     float t = 0;
     if (!rc) hipEventElapsedTime(&t, log.ev[i], log.ev[i + 1]);
@@ -1608,12 +1607,25 @@ static int udsc_run(const plg_prop *up, const plg_prop *dn, const plg_prop *st, 
   return PLG_OK;
 }
 
-// Packed tables by content (the term order is a search over the table, a few
-// milliseconds per thousand terms): the last few tables packed, keyed by a
-// 64-bit hash of the counts, spins, colour slots and coefficients.
+// Packed tables by content (laying out a table takes milliseconds per ten
+// thousand terms): the last few tables, with their device arrays, keyed by a
+// 64-bit hash of the counts, spins, colour slots and coefficients and by the
+// precision.  A table whose device arrays are large is not kept.
+struct TetraTable {
+  std::vector<TetraSched> s;  // one per launch
+  std::vector<void *> mem;
+  ~TetraTable() {
+    for (void *p : mem) hipFree(p);
+  }
+};
 static std::mutex g_pack_mu;
-static std::vector<std::pair<uint64_t, std::shared_ptr<const TetraPacked>>> g_pack_cache;
-constexpr size_t PACK_CACHE = 8;
+static std::vector<std::pair<uint64_t, std::shared_ptr<const TetraTable>>> g_pack_cache;
+constexpr size_t PACK_CACHE = 8, PACK_BYTES = (size_t)32 << 20;
+
+static void tetra_tables_clear() {
+  std::lock_guard<std::mutex> lk(g_pack_mu);
+  g_pack_cache.clear();
+}
 
 static uint64_t hash_bytes(const void *data, size_t n, uint64_t h) {
   const unsigned char *b = (const unsigned char *)data;
@@ -1629,14 +1641,14 @@ static uint64_t hash_bytes(const void *data, size_t n, uint64_t h) {
 }
 
 static int tetra_pack_cached(const int16_t *idxs, const int16_t *cols, const float *vals, const int16_t *counts,
-                             int nops, TetraPacked &out) {
+                             int nops, int T, std::shared_ptr<const TetraTable> &out) {
   if (nops <= 0 || nops > TETRA_MAXOPS) return PLG_ERR_UNSUPPORTED;
   size_t nt = 0;
   for (int k = 0; k < nops; k++) {
     if (counts[k] < 0) return PLG_ERR_INVALID;
     nt += (size_t)counts[k];
   }
-  uint64_t h = 0xcbf29ce484222325ull ^ (uint64_t)nops;
+  uint64_t h = 0xcbf29ce484222325ull ^ (uint64_t)nops ^ (uint64_t)T << 32;
   h = hash_bytes(counts, nops * sizeof(int16_t), h);
   h = hash_bytes(idxs, nt * 8 * sizeof(int16_t), h);
   h = hash_bytes(cols, nt * 8 * sizeof(int16_t), h);
@@ -1645,17 +1657,36 @@ static int tetra_pack_cached(const int16_t *idxs, const int16_t *cols, const flo
     std::lock_guard<std::mutex> lk(g_pack_mu);
     for (auto &e : g_pack_cache)
       if (e.first == h) {
-        out = *e.second;
+        out = e.second;
         return PLG_OK;
       }
   }
-  auto pk = std::make_shared<TetraPacked>();
-  const int rc = tetra_pack(idxs, cols, vals, counts, nops, *pk);
+  std::vector<TetraPacked> pk;
+  const int per = T == PLG_F64 ? TT_OPS<double> : TT_OPS<float>;
+  int rc = tetra_pack(idxs, cols, vals, counts, nops, per, pk);
   if (rc) return rc;
-  out = *pk;
+  auto tab = std::make_shared<TetraTable>();
+  size_t bytes = 0;
+  auto put = [&](const auto &v, const void **d) {
+    typename std::decay_t<decltype(v)>::value_type *p = nullptr;
+    const int r = upload(&p, v, nullptr);
+    if (p) tab->mem.push_back(p);
+    bytes += v.size() * sizeof(*p);
+    *d = p;
+    return r;
+  };
+  for (TetraPacked &k : pk) {
+    if ((rc = put(k.words, (const void **)&k.s.words))) return rc;
+    if (T == PLG_F64) rc = put(k.coef, &k.s.coef);
+    else rc = put(std::vector<float>(k.coef.begin(), k.coef.end()), &k.s.coef);
+    if (rc) return rc;
+    tab->s.push_back(k.s);
+  }
+  out = tab;
+  if (bytes > PACK_BYTES) return PLG_OK;
   std::lock_guard<std::mutex> lk(g_pack_mu);
   if (g_pack_cache.size() >= PACK_CACHE) g_pack_cache.erase(g_pack_cache.begin());
-  g_pack_cache.emplace_back(h, std::move(pk));
+  g_pack_cache.emplace_back(h, std::move(tab));
   return PLG_OK;
 }
 
@@ -1669,26 +1700,26 @@ static int tetra_run(const plg_prop *const views[4], const int16_t *idxs, const 
   if (!idxs || !col_contr || !vals || !counts || nops <= 0) return fail(PLG_ERR_INVALID, "empty table");
   for (int i = 0; i < 4; i++)
     if (!views[i]) return fail(PLG_ERR_INVALID, "NULL propagator view");
-  TetraPacked pk;
-  rc = tetra_pack_cached(idxs, col_contr, vals, counts, nops, pk);
+  const int prec = mode == PLG_MODE_F64 ? PLG_F64 : PLG_F32;
+  std::shared_ptr<const TetraTable> tab;  // held until the stream is synchronised
+  rc = tetra_pack_cached(idxs, col_contr, vals, counts, nops, prec, tab);
   if (rc == PLG_ERR_INVALID) return fail(rc, "spin or colour index outside 0..3");
+  if (rc == PLG_ERR_HIP) return rc;
   if (rc)
     return fail(rc, "table outside the supported form (64 operators; colour slots a permutation of the four "
                     "sums, closing as <P1,P3><P2,P4>, Tr[(P3^dag P1)(P4^dag P2)], <P1,P4><P2,P3> or "
                     "Tr[(P4^dag P1)(P3^dag P2)]; 65536 distinct coefficients)");
-  const bool two_sets = !pk.terms[1].empty();
   int lt;
   if ((rc = plg_window(source, totalT, nullptr, nullptr, &lt))) return rc;
   const Window w = window_of(g_ctx.L, source, totalT);
   const int T = g_ctx.L[3];
   const int64_t inner = space == PLG_MOMENTUM_SPACE ? (int64_t)nmom : g_ctx.V3;
-  hipStream_t hs = (hipStream_t)stream;
   Plan P;
   P.kind = -1;
   P.mode = mode;
   P.terms = PLG_SPLIT_BF16X6;
   P.space = space;
-  P.T = mode == PLG_MODE_F64 ? PLG_F64 : PLG_F32;
+  P.T = prec;
   for (int i = 0; i < 4; i++) P.props.push_back(*views[i]);
   P.nmom = space == PLG_MOMENTUM_SPACE ? nmom : 0;
   if (P.nmom) P.moms.assign(moms, moms + 3 * P.nmom);
@@ -1700,9 +1731,7 @@ static int tetra_run(const plg_prop *const views[4], const int16_t *idxs, const 
     for (const plg_prop &v : P.props)
       if ((rc = check_prop(v, P.T, t))) return rc;
     P.rows.push_back({t, 0, 1, 0, 2});
-    P.rows4.push_back({t, {0, 1, 2, 3}});
   }
-  for (int j = 0; j < lt; j++) P.rows4.push_back({P.rows[j].t, {0, 1, 3, 2}});  // set 1's views
   for (int k = 0; k < nops; k++)
     for (int j = 0; j < lt; j++) {
       const int t = P.rows[j].t;
@@ -1725,51 +1754,11 @@ static int tetra_run(const plg_prop *const views[4], const int16_t *idxs, const 
   P.m_stride = 1;
   P.out_elems = (int64_t)(d0 + nops) * lt * inner;
   P.nsites = (int64_t)lt * g_ctx.V3;
-  // set 0 writes every operator (zero where it has no terms), set 1 adds
-  P.launches.push_back({Launch::TETRA, 0, false, false, 0, 0});
-  if (two_sets) P.launches.push_back({Launch::TETRA, 1, false, false, 0, 0});
-  TetraTerm *d_terms[2] = {nullptr, nullptr};
-  float *d_coef = nullptr;
-  auto free_tables = [&] {
-    for (TetraTerm *p : d_terms) hipFree(p);
-    hipFree(d_coef);
-  };
-  for (int h = 0; h < (two_sets ? 2 : 1) && !rc; h++) rc = upload(&d_terms[h], pk.terms[h], hs);
-  if (!rc) rc = upload(&d_coef, pk.coef, hs);
-  if (rc) {
-    hipStreamSynchronize(hs);
-    free_tables();
-    return rc;
-  }
-  for (int h = 0; h < 2; h++) {
-    TetraSched &S = h ? P.tetra2 : P.tetra;
-    S.ncoef = (int)pk.coef.size() / 2;
-    S.nops = nops;
-    for (int k = 0; k < nops; k++) {
-      S.first[k] = pk.first[h][k];
-      S.count[k] = pk.count[h][k];
-      S.ndirect[k] = pk.ndirect[h][k];
-    }
-    S.terms = d_terms[h];
-    S.coef = d_coef;
-    S.accumulate = h;
-  }
+  P.tetra = tab->s;
+  for (int i = 0, k = 0; i < (int)P.tetra.size(); k += P.tetra[i++].nops)
+    P.launches.push_back({Launch::TETRA, i, false, false, 0, k});
   choose_tiles(P);
-  P.tpb = 64;  // sites per workgroup of the kernel
-  if (!(rc = upload_plan(P, hs)) && !(rc = upload(&P.d_rows4, P.rows4, hs))) {
-    std::lock_guard<std::mutex> wl(g_ws_mu);  // until the stream is synchronised below
-    {
-      std::lock_guard<std::mutex> lk(g_mu);
-      if (!(rc = ensure(&g_ctx.ws_c, &g_ctx.ws_c_bytes, c_bytes(P))))
-        rc = ensure(&g_ctx.ws_part, &g_ctx.ws_part_bytes, part_bytes(P));
-    }
-    if (!rc) rc = enqueue(P, g_ctx.ws_c, g_ctx.ws_part, out, out_precision, hs);
-    const hipError_t se = hipStreamSynchronize(hs);  // also after an error
-    if (!rc && se != hipSuccess) rc = fail(PLG_ERR_HIP, "tetraquark table sync failed");
-  }
-  hipStreamSynchronize(hs);  // no launch may still read the terms
-  free_tables();
-  return rc;
+  return plan_run(P, out, out_precision, (hipStream_t)stream, nullptr);
 }
 
 int plg_tetraquark_table(const plg_prop *p1, const plg_prop *p2, const plg_prop *p3, const plg_prop *p4,

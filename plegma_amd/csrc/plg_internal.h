@@ -139,40 +139,35 @@ int udsc_schedule_terms(const UdscTerm *terms, const int *first, const int *coun
 
 // four-propagator table contractions (tetraquark table format)
 constexpr int TETRA_MAXOPS = 64;
-// A term, 32 bits: the (P1, P3) spin pair p = 16 s1 + s3 (bits 0-7), the
-// (P2, P4) pair q = 16 s2 + s4 (bits 8-15) and the coefficient index (bits
-// 16-31), with the 4-bit spin pairs s1 = 4 i0 + i1, s2 = 4 i2 + i3,
-// s3 = 4 (i5+2) + (i4+2), s4 = 4 (i7+2) + (i6+2) (indices mod 4).  An
-// operator's terms are its direct ones (<P1,P3><P2,P4>) first, then its
-// crossed ones (Tr[(P3^dag P1)(P4^dag P2)]).
-typedef uint32_t TetraTerm;
-constexpr int TETRA_MAXCOEF = 65536;
+constexpr int TETRA_MAXCOEF = 65536;  // distinct coefficients
+constexpr int TT_WAVES = 8;           // waves of a workgroup
+// A table as the walk of the kernel's waves: nsteps steps from word word0 and
+// coefficient vector coef0.  Step, two words: four pairs p = s1 << 4 | s3 (a
+// byte each); groups of crossed (bits 0-7) and of direct products (8-15), set
+// (16).  Group, crossed ones first: four s2 (4 bits each) and the products
+// (16-).  Product: four s4 (4 bits each) and the operator blocks with a real
+// (16-19) and an imaginary (20-23) coefficient vector, each [quarter][operator
+// of the block], in this order.  Spin pairs s1 = 4 i0 + i1, s2 = 4 i2 + i3,
+// s3 = 4 (i5+2) + (i4+2), s4 = 4 (i7+2) + (i6+2) (indices mod 4).
 struct TetraSched {
   int nops;
-  int first[TETRA_MAXOPS], count[TETRA_MAXOPS], ndirect[TETRA_MAXOPS];
-  const TetraTerm *terms;
-  const float *coef;  // re, im of each distinct coefficient
-  int ncoef;
-  int accumulate;     // add the operators to the site correlator instead of writing them
+  int word0[TT_WAVES], nsteps[TT_WAVES], coef0[TT_WAVES];
+  const uint32_t *words;
+  const void *coef;  // in the precision of the contraction
 };
-struct RowDev4 {
-  int t;
-  int p[4];
-};
-// The terms of a table in two sets.  Set 0 pairs the colours of P1 with P3
-// and of P2 with P4 (the two structures above); set 1 pairs P1 with P4 and
-// P2 with P3 (<P1,P4><P2,P3> and Tr[(P4^dag P1)(P3^dag P2)]), which are the
-// same structures on the views P1, P2, P4, P3, and is packed for those views.
+// operators of one launch: all in FP32; in FP64 the sums of more than two
+// blocks of 16 do not fit the registers beside the products
+template <typename T> constexpr int TT_OPS = sizeof(T) == 4 ? TETRA_MAXOPS : 32;
 struct TetraPacked {
-  std::vector<TetraTerm> terms[2];
-  std::vector<int> first[2], count[2], ndirect[2];
-  std::vector<float> coef;  // shared by both sets
+  TetraSched s{};
+  std::vector<uint32_t> words;
+  std::vector<double> coef;
 };
-int tetra_pack(const int16_t *idxs, const int16_t *cols, const float *vals, const int16_t *counts, int nops,
-               TetraPacked &out);
+int tetra_pack(const int16_t *idxs, const int16_t *cols, const float *vals, const int16_t *counts, int nops, int per,
+               std::vector<TetraPacked> &out);
 template <typename T>
-int launch_tetra(const TetraSched &S, const PropDev<T> *props, const RowDev4 *rows, int nrows, cx<T> *out,
-                 int64_t V3, int T_lat, int nch_total, int spw, hipStream_t st);
+int launch_tetra(const TetraSched &S, const PropDev<T> *props, const RowDev *rows, int nrows, cx<T> *out,
+                 int64_t V3, int T_lat, int nch_total, int ch0, hipStream_t st);
 int udsc_products();
 const char *udsc_flavours(int prod);
 int udsc_nops(int prod);

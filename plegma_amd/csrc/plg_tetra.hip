@@ -12,375 +12,395 @@
 //   direct  (c0 = c5, c1 = c4, c2 = c7, c3 = c6):  <B1, B3> <B2, B4>,   <X, Y> = sum X conj(Y)
 //   crossed (c0 = c5, c1 = c6, c2 = c7, c3 = c4):  Tr[(B3^dag B1)(B4^dag B2)]
 // Terms that pair P1 with P4 and P2 with P3 instead (the bcud tables) close
-// into the same two structures on the views P1, P2, P4, P3; the host packs them
-// as a second set, contracted by a second launch that adds to the first.
+// into the same two structures on the views P1, P2, P4, P3: a second set.
 // The host classifies every term; a table with another structure is refused.
 //
-// Both structures factor through the spin pairs p = (B1, B3) and
-// q = (B2, B4), 256 of each per site: per site the workgroup builds the
-// tables <B1,B3>, B3^dag B1 (over p) and <B2,B4>, B4^dag B2 (over q), 36
-// complex products per entry, and then a direct term costs one complex
-// product of two table entries and a crossed term the trace of a product of
-// two (9 products), instead of 19 and 63 from the blocks.  The terms of the
-// reference's tables use every p and q, about 50 terms per entry.
-//
-// A workgroup of 4 waves stages 64-byte lines of the four propagators (8
-// FP32 or 4 FP64 consecutive sites) in LDS; per site, each thread builds one
-// p entry and one q entry of the tables, then each wave takes every fourth
-// operator, its lanes splitting the operator's terms, and a wave reduction.
-// In FP32 a spin pair's entries are ten (the 3x3 product, then the scalar
-// product), read as five 16-byte pairs: 83.0 -> 76.3 ms on the benchmark's
-// table against nine entries read one by one.
+// Terms of one structure with the same four spin pairs are one product with a
+// coefficient per operator: the 12.7 k terms of the heavy-light tables are
+// 3648 products, the 63 k of the bcud table 10496.  With M = B3^dag B1 of the
+// spin pairs p = (s1, s3), both structures are scalar products with B4:
+//   crossed: <X, B4>, X = B2 M;    direct: <X, B4>, X = Tr(M) B2,
+// so the products are walked as p, then s2 (X in registers), then s4.
 #include "plg_internal.h"
 
 #include <algorithm>
+#include <array>
 #include <cstring>
 #include <map>
+#include <numeric>
 
 namespace plg {
 
-constexpr int TETRA_TB = 12;      // terms per lane loaded together
-constexpr int TETRA_LDS_COEF = 256;  // coefficients kept in LDS
-
-template <typename T> struct TetraGeom {
-  static constexpr int G = 64 / (int)sizeof(cx<T>);  // sites per staged line
-  static constexpr int SPAD = 577;                   // LDS stride of a site (576 + 1)
+// A workgroup of 8 waves stages the four propagators of 16 consecutive sites
+// in LDS, entries outermost (a row of 16 sites is 128 or 256 bytes).  The lane
+// of site s and quarter q = lane / 16 takes its quarter's spin pairs of every
+// step, so that the walk is uniform over the wave and a product's 64 values
+// (16 sites, 4 sets of spin pairs) are, as they lie in the registers, the B
+// operand of a 16x16x4 matrix product with the coefficients of 16 operators.
+// A wave reads its walk 64 words at a time and hands them out by lane reads;
+// the coefficients are loaded two products ahead.  The waves' sums meet in LDS
+// at the end.
+// Bound by the vector unit: M 108 FMAs, X 108 (crossed) or 36, a product 36
+// and its matrix instructions.
+// Of 2.64 M cycles on 16^3 x 24 sites with the udbb table, FP32, the FMAs take
+// 1.5 M, the matrix instructions 0.35 M, LDS is busy 1.4 M.  Term by term from
+// tables of B3^dag B1 and B4^dag B2 in LDS, a site at a time, the same took
+// 3.65 ms, bound by the 160 bytes of LDS a term reads; this 1.26 ms.
+template <typename T> struct TtAcc;
+template <> struct TtAcc<float> {
+  typedef float v4 __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ v4 mma(float a, float b, v4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane >> 4) + r; }
+};
+template <> struct TtAcc<double> {
+  typedef double v4 __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ v4 mma(double a, double b, v4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int lane, int r) { return 4 * r + (lane >> 4); }
 };
 
-template <typename T>
-__global__ __launch_bounds__(256) void k_tetra(TetraSched S, const PropDev<T> *__restrict__ props,
-                                               const RowDev4 *__restrict__ rows, cx<T> *__restrict__ out,
-                                               int64_t V3, int T_lat, int nch_total, int groups_per_block) {
-  constexpr int G = TetraGeom<T>::G, SPAD = TetraGeom<T>::SPAD;
-  __shared__ cx<T> sp[G * SPAD];                 // [site][f][m01][a b]
-  // per spin pair: the 9 entries of (B3^dag B1)[z][y] (over p) or
-  // (B4^dag B2)[y][z] (over q) at z*3+y; in FP32 then <B1,B3> or <B2,B4>,
-  // ten entries, so that entry pairs are 16-byte reads (in FP64 an entry is
-  // one, and nine entries keep the spin pairs on distinct banks)
-  constexpr bool F32 = sizeof(T) == 4;
-  constexpr int SPP = F32 ? 10 : 9;
-  __shared__ __align__(16) cx<T> m13[256 * SPP], n24[256 * SPP];
-  __shared__ cx<T> d13[F32 ? 1 : 256], d24[F32 ? 1 : 256];  // FP64: <B1,B3> over p, <B2,B4> over q
-  __shared__ cx<T> scoef[TETRA_LDS_COEF];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const RowDev4 row = rows[blockIdx.y];
-  const PropDev<T> P0 = props[row.p[0]], P1 = props[row.p[1]], P2 = props[row.p[2]], P3 = props[row.p[3]];
-  auto plane_base = [&](const PropDev<T> &Q) {
-    int plane = row.t - Q.t_first;
-    plane += plane < 0 ? T_lat : 0;
-    return Q.data + (int64_t)plane * V3;
-  };
-  const cx<T> *b0 = plane_base(P0), *b1 = plane_base(P1), *b2 = plane_base(P2), *b3 = plane_base(P3);
-  const T sg = prop_sign(P0, row.t) * prop_sign(P1, row.t) * prop_sign(P2, row.t) * prop_sign(P3, row.t);
-  const int rot_any = P0.rot | P1.rot | P2.rot | P3.rot;
-  const int64_t ncols = (int64_t)gridDim.y * nch_total, col0 = (int64_t)blockIdx.y * nch_total;
-  // the coefficients in LDS when they fit (the reference's tables have six)
-  const bool coef_lds = S.ncoef <= TETRA_LDS_COEF;
-  if (coef_lds)
-    for (int i = tid; i < S.ncoef; i += 256) scoef[i] = cmake<T>((T)S.coef[2 * i], (T)S.coef[2 * i + 1]);
-
-  for (int gi = 0; gi < groups_per_block; gi++) {
-    const int64_t x0 = ((int64_t)blockIdx.x * groups_per_block + gi) * G;
-    if (x0 >= V3) break;  // uniform over the workgroup
-    __syncthreads();      // the previous group's sites are done
-    for (int idx = tid; idx < 576 * G; idx += 256) {
-      const int comp = idx / G, s = idx - comp * G;
-      const int f = comp / 144, cl = comp - f * 144;
-      const cx<T> *b = f == 0 ? b0 : (f == 1 ? b1 : (f == 2 ? b2 : b3));
-      const int64_t cs = f == 0 ? P0.cs : (f == 1 ? P1.cs : (f == 2 ? P2.cs : P3.cs));
-      const int64_t x = x0 + s;
-      sp[s * SPAD + comp] = x < V3 ? gload(b + (int64_t)cl * cs + x) : cmake<T>(0, 0);
+// NB: blocks of 16 operators
+template <typename T, int NB>
+__global__ __launch_bounds__(64 * TT_WAVES, sizeof(T) == 4 ? 4 : 2) void k_tetra(
+    TetraSched S, const PropDev<T> *__restrict__ props, const RowDev *__restrict__ rows, cx<T> *__restrict__ out,
+    int64_t V3, int T_lat, int nch_total, int ch0) {
+  typedef typename TtAcc<T>::v4 v4;
+  constexpr int NT = 64 * TT_WAVES;
+  __shared__ cx<T> sp[4 * 144 * 16];  // [propagator][m01][a b][site]
+  __shared__ T red[TT_WAVES][256];    // the waves' sums of 16 operators, real or imaginary
+  const int tid = threadIdx.x, lane = tid & 63, s = tid & 15, kq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const RowDev row = rows[blockIdx.y];
+  const int64_t x0 = (int64_t)blockIdx.x * 16;
+  T sg = 1;
+  int rot_any = 0;
+  {
+    const bool xin = x0 + s < V3;
+#pragma unroll
+    for (int f = 0; f < 4; f++) {
+      const PropDev<T> Q = props[f];
+      sg *= prop_sign(Q, row.t);
+      rot_any |= Q.rot;
+      int plane = row.t - Q.t_first;
+      plane += plane < 0 ? T_lat : 0;
+      const cx<T> *b = Q.data + (int64_t)plane * V3 + x0 + s;
+#pragma unroll
+      for (int i = 0; i < (144 * 16 + NT - 1) / NT; i++) {
+        const int c = i * (NT / 16) + (tid >> 4);
+        if (c < 144) sp[(f * 144 + c) * 16 + s] = xin ? gload(b + (int64_t)c * Q.cs) : cmake<T>(0, 0);
+      }
+    }
+  }
+  __syncthreads();
+  if (rot_any) {  // rotation to the physical basis, per (site, propagator, colour pair)
+    for (int k = tid; k < 4 * 9 * 16; k += NT) {
+      const int f = k / 144, cc = (k >> 4) % 9, rot = props[f].rot;
+      if (rot) {
+        cx<T> *b = sp + (f * 144 + cc) * 16 + (k & 15);
+        cx<T> w[16];
+#pragma unroll
+        for (int m = 0; m < 16; m++) w[m] = b[m * 9 * 16];
+        rot_spins(w, rot);
+#pragma unroll
+        for (int m = 0; m < 16; m++) b[m * 9 * 16] = w[m];
+      }
     }
     __syncthreads();
-    if (rot_any) {  // rotation to the physical basis, per (site, propagator, colour pair)
-      for (int k = tid; k < G * 36; k += 256) {
-        const int s = k / 36, f = (k % 36) / 9, cc = k % 9;
-        const int rot = f == 0 ? P0.rot : (f == 1 ? P1.rot : (f == 2 ? P2.rot : P3.rot));
-        if (rot) {
-          cx<T> *b = sp + s * SPAD + f * 144 + cc;
-          cx<T> v[16];
+  }
+  v4 ar[NB], ai[NB];
 #pragma unroll
-          for (int m = 0; m < 16; m++) v[m] = b[m * 9];
-          rot_spins(v, rot);
-#pragma unroll
-          for (int m = 0; m < 16; m++) b[m * 9] = v[m];
-        }
-      }
-      __syncthreads();
+  for (int b = 0; b < NB; b++) ar[b] = ai[b] = (v4)(T)0;
+  // the wave's words, 64 at a time and the next 64 on the way
+  const uint32_t *wp = S.words + S.word0[wave] + lane;
+  uint32_t wcur = wp[0], wnext = wp[64];
+  int wpos = 0;
+  auto word = [&]() -> uint32_t {
+    if (wpos == 64) {
+      wcur = wnext;
+      wp += 64;
+      wnext = wp[64];
+      wpos = 0;
     }
-    for (int s = 0; s < G; s++) {
-      const int64_t x = x0 + s;
-      if (x >= V3) break;  // uniform
-      const cx<T> *spx = sp + s * SPAD;
-      // tables of the site: thread tid = 16 hi + lo builds entry tid of both
+    return (uint32_t)__builtin_amdgcn_readlane((int)wcur, wpos++);
+  };
+  const T *cp = (const T *)S.coef + (int64_t)S.coef0[wave] * 64 + lane;
+  T c0 = cp[0], c1 = cp[64];
+  cp += 128;
+  for (int st = 0; st < S.nsteps[wave]; st++) {
+    const uint32_t pw = word(), fw = word();
+    const int p = (pw >> (8 * kq)) & 255;
+    const cx<T> *P3 = sp + ((fw >> 16) & 1 ? 3 : 2) * 2304 + s, *P4 = sp + ((fw >> 16) & 1 ? 2 : 3) * 2304 + s;
+    cx<T> m[9];  // (B3^dag B1)[z][y] at z * 3 + y
+    {
+      const cx<T> *A = sp + s + (p >> 4) * 144, *B = P3 + (p & 15) * 144;
+      cx<T> a[9], b[9];
+#pragma unroll
+      for (int j = 0; j < 9; j++) {
+        a[j] = A[j * 16];
+        b[j] = B[j * 16];
+      }
+#pragma unroll
+      for (int z = 0; z < 3; z++)
+#pragma unroll
+        for (int y = 0; y < 3; y++) {
+          m[z * 3 + y] = cmake<T>(0, 0);
+#pragma unroll
+          for (int w = 0; w < 3; w++) cfma_conj(m[z * 3 + y], a[w * 3 + y], b[w * 3 + z]);
+        }
+    }
+    const int ncr = fw & 255, ng = ncr + ((fw >> 8) & 255);
+    for (int g = 0; g < ng; g++) {
+      const uint32_t gw = word();
+      cx<T> X[9];
       {
-        const int hi = tid >> 4, lo = tid & 15;
-        cx<T> a[9], b[9];
+        const cx<T> *B2 = sp + 2304 + s + ((gw >> (4 * kq)) & 15) * 144;
+        cx<T> b[9];
 #pragma unroll
-        for (int j = 0; j < 9; j++) {
-          a[j] = spx[hi * 9 + j];          // B1 = P1 block s1 = hi
-          b[j] = spx[288 + lo * 9 + j];    // B3 = P3 block s3 = lo
+        for (int j = 0; j < 9; j++) b[j] = B2[j * 16];
+        if (g < ncr) {
+#pragma unroll
+          for (int w = 0; w < 3; w++)
+#pragma unroll
+            for (int y = 0; y < 3; y++) {
+              X[w * 3 + y] = cmake<T>(0, 0);
+#pragma unroll
+              for (int z = 0; z < 3; z++) cfma(X[w * 3 + y], b[w * 3 + z], m[z * 3 + y]);
+            }
+        } else {
+          const cx<T> d = m[0] + m[4] + m[8];  // <B1, B3>
+#pragma unroll
+          for (int j = 0; j < 9; j++) X[j] = d * b[j];
         }
-        cx<T> d = cmake<T>(0, 0);
+      }
+      const int nt = (int)(gw >> 16);
+      for (int e = 0; e < nt; e++) {
+        const uint32_t uw = word();
+        const cx<T> *B4 = P4 + ((uw >> (4 * kq)) & 15) * 144;
+        cx<T> t = cmake<T>(0, 0);
 #pragma unroll
-        for (int j = 0; j < 9; j++) cfma_conj(d, a[j], b[j]);
-        if constexpr (F32) m13[tid * SPP + 9] = d;
-        else d13[tid] = d;
+        for (int j = 0; j < 9; j++) cfma_conj(t, X[j], B4[j * 16]);
+        // O[k] += V[k] t in the operator blocks the products have coefficients in
 #pragma unroll
-        for (int z = 0; z < 3; z++)
-#pragma unroll
-          for (int y = 0; y < 3; y++) {
-            cx<T> m = cmake<T>(0, 0);
-#pragma unroll
-            for (int w = 0; w < 3; w++) cfma_conj(m, a[w * 3 + y], b[w * 3 + z]);
-            m13[tid * SPP + z * 3 + y] = m;
+        for (int b = 0; b < NB; b++)
+          if (uw >> (16 + b) & 1) {
+            const T v = c0;
+            c0 = c1;
+            c1 = *cp;
+            cp += 64;
+            ar[b] = TtAcc<T>::mma(v, t.re, ar[b]);
+            ai[b] = TtAcc<T>::mma(v, t.im, ai[b]);
           }
+        if (uw >> 20) {
 #pragma unroll
-        for (int j = 0; j < 9; j++) {
-          a[j] = spx[144 + hi * 9 + j];    // B2 = P2 block s2 = hi
-          b[j] = spx[432 + lo * 9 + j];    // B4 = P4 block s4 = lo
+          for (int b = 0; b < NB; b++)
+            if (uw >> (20 + b) & 1) {
+              const T v = c0;
+              c0 = c1;
+              c1 = *cp;
+              cp += 64;
+              ar[b] = TtAcc<T>::mma(v, -t.im, ar[b]);
+              ai[b] = TtAcc<T>::mma(v, t.re, ai[b]);
+            }
         }
-        d = cmake<T>(0, 0);
+      }
+    }
+  }
+  // the waves' sums
+  const int64_t ncols = (int64_t)gridDim.y * nch_total, col0 = (int64_t)blockIdx.y * nch_total + ch0;
 #pragma unroll
-        for (int j = 0; j < 9; j++) cfma_conj(d, a[j], b[j]);
-        if constexpr (F32) n24[tid * SPP + 9] = d;
-        else d24[tid] = d;
+  for (int b = 0; b < NB; b++) {
+    T o[2];
 #pragma unroll
-        for (int z = 0; z < 3; z++)
+    for (int h = 0; h < 2; h++) {
 #pragma unroll
-          for (int y = 0; y < 3; y++) {
-            cx<T> m = cmake<T>(0, 0);
+      for (int r = 0; r < 4; r++) red[wave][r * 64 + lane] = h ? ai[b][r] : ar[b][r];
+      __syncthreads();
+      if (tid < 256) {
+        T v = red[0][tid];
 #pragma unroll
-            for (int w = 0; w < 3; w++) cfma_conj(m, a[w * 3 + z], b[w * 3 + y]);
-            n24[tid * SPP + z * 3 + y] = m;
-          }
+        for (int w = 1; w < TT_WAVES; w++) v += red[w][tid];
+        o[h] = v;
       }
       __syncthreads();
-      // one term of the tables: direct <B1,B3><B2,B4> or crossed trace
-      auto term = [&](uint32_t u, bool crossed) {
-        const int p = u & 255, q = (u >> 8) & 255, ci = (int)(u >> 16);
-        cx<T> v;
-        if constexpr (F32) {
-          // 16-byte reads: entry pairs (0,1) .. (6,7), then (8, the <,> value)
-          typedef float f4 __attribute__((ext_vector_type(4)));
-          const f4 *a = reinterpret_cast<const f4 *>(m13 + p * SPP);
-          const f4 *b = reinterpret_cast<const f4 *>(n24 + q * SPP);
-          if (!crossed) {
-            const f4 x = a[4], y = b[4];
-            v = cmake<T>(x[2], x[3]) * cmake<T>(y[2], y[3]);
-          } else {
-            v = cmake<T>(0, 0);
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-              const f4 x = a[k], y = b[k];
-              cfma(v, cmake<T>(x[0], x[1]), cmake<T>(y[0], y[1]));
-              cfma(v, cmake<T>(x[2], x[3]), cmake<T>(y[2], y[3]));
-            }
-            const f4 x = a[4], y = b[4];
-            cfma(v, cmake<T>(x[0], x[1]), cmake<T>(y[0], y[1]));
-          }
-        } else {
-          if (!crossed) {
-            v = d13[p] * d24[q];
-          } else {
-            v = cmake<T>(0, 0);
-#pragma unroll
-            for (int j = 0; j < 9; j++) cfma(v, m13[p * SPP + j], n24[q * SPP + j]);
-          }
-        }
-        const cx<T> c = coef_lds ? scoef[ci] : cmake<T>((T)S.coef[2 * ci], (T)S.coef[2 * ci + 1]);
-        return c * v;
-      };
-      auto emit = [&](int k, cx<T> acc) {
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) {
-          acc.re += __shfl_xor(acc.re, off);
-          acc.im += __shfl_xor(acc.im, off);
-        }
-        if (lane == 0) {
-          cx<T> *o = out + ctile_idx(col0 + k, x, ncols);
-          cx<T> v = cmake<T>(sg * acc.re, sg * acc.im);
-          if (S.accumulate) v = v + gload(o);  // the set written by the previous launch
-          gstore(o, v);
-        }
-      };
-      // wave w takes the operators k = w, w + 4, ...; its lanes split an
-      // operator's terms, TETRA_TB terms per lane loaded together, the next
-      // batch (of this operator or the wave's next one) in flight while one
-      // is summed
-      int k = wave, base = 0;
-      uint32_t u[TETRA_TB];
-      auto fetch = [&](int kk, int b, uint32_t *dst) {
-        const int n = kk < S.nops ? S.count[kk] : 0;
-        const TetraTerm *E = S.terms + (kk < S.nops ? S.first[kk] : 0);
-#pragma unroll
-        for (int i = 0; i < TETRA_TB; i++) {
-          const int t = b + lane + 64 * i;
-          dst[i] = t < n ? E[t] : 0u;
-        }
-      };
-      fetch(k, 0, u);
-      cx<T> acc = cmake<T>(0, 0);
-      while (k < S.nops) {
-        const int n = S.count[k], nd = S.ndirect[k];
-        // the batch after this one
-        int k2 = k, b2 = base + 64 * TETRA_TB;
-        if (b2 >= n) {
-          k2 = k + 4;
-          b2 = 0;
-        }
-        uint32_t v[TETRA_TB];
-        fetch(k2, b2, v);
-#pragma unroll
-        for (int i = 0; i < TETRA_TB; i++) {
-          const int t = base + lane + 64 * i;
-          if (t < n) acc = acc + term(u[i], t >= nd);
-        }
-        if (k2 != k) {
-          emit(k, acc);
-          acc = cmake<T>(0, 0);
-        }
-        k = k2;
-        base = b2;
-#pragma unroll
-        for (int i = 0; i < TETRA_TB; i++) u[i] = v[i];
-      }
-      __syncthreads();  // the tables may be rebuilt for the next site
     }
+    const int k = 16 * b + TtAcc<T>::row(lane, wave);
+    if (tid < 256 && k < S.nops && x0 + s < V3)
+      gstore(out + ctile_idx(col0 + k, x0 + s, ncols), cmake<T>(sg * o[0], sg * o[1]));
   }
 }
 
 template <typename T>
-int launch_tetra(const TetraSched &S, const PropDev<T> *props, const RowDev4 *rows, int nrows, cx<T> *out,
-                 int64_t V3, int T_lat, int nch_total, int spw, hipStream_t st) {
-  constexpr int G = TetraGeom<T>::G;
-  const int gpb = std::max(1, spw / G);
-  const int64_t ngroups = (V3 + G - 1) / G;
-  dim3 block(256), grid((unsigned)((ngroups + gpb - 1) / gpb), (unsigned)nrows);
-  k_tetra<T><<<grid, block, 0, st>>>(S, props, rows, out, V3, T_lat, nch_total, gpb);
+int launch_tetra(const TetraSched &S, const PropDev<T> *props, const RowDev *rows, int nrows, cx<T> *out,
+                 int64_t V3, int T_lat, int nch_total, int ch0, hipStream_t st) {
+  dim3 block(64 * TT_WAVES), grid((unsigned)((V3 + 15) / 16), (unsigned)nrows);
+  switch ((S.nops + 15) / 16) {
+  case 1: k_tetra<T, 1><<<grid, block, 0, st>>>(S, props, rows, out, V3, T_lat, nch_total, ch0); break;
+  case 2: k_tetra<T, 2><<<grid, block, 0, st>>>(S, props, rows, out, V3, T_lat, nch_total, ch0); break;
+  case 3:
+    if constexpr (TT_OPS<T> > 32) k_tetra<T, 3><<<grid, block, 0, st>>>(S, props, rows, out, V3, T_lat, nch_total, ch0);
+    else return PLG_ERR_UNSUPPORTED;
+    break;
+  case 4:
+    if constexpr (TT_OPS<T> > 48) k_tetra<T, 4><<<grid, block, 0, st>>>(S, props, rows, out, V3, T_lat, nch_total, ch0);
+    else return PLG_ERR_UNSUPPORTED;
+    break;
+  default: return PLG_ERR_UNSUPPORTED;
+  }
   return hipGetLastError() == hipSuccess ? PLG_OK : PLG_ERR_HIP;
 }
 
-template int launch_tetra<double>(const TetraSched &, const PropDev<double> *, const RowDev4 *, int, cx<double> *,
+template int launch_tetra<double>(const TetraSched &, const PropDev<double> *, const RowDev *, int, cx<double> *,
                                   int64_t, int, int, int, hipStream_t);
-template int launch_tetra<float>(const TetraSched &, const PropDev<float> *, const RowDev4 *, int, cx<float> *,
+template int launch_tetra<float>(const TetraSched &, const PropDev<float> *, const RowDev *, int, cx<float> *,
                                  int64_t, int, int, int, hipStream_t);
 
-// Order of an operator's terms of one structure.  The kernel's lanes take
-// consecutive terms, and the 16 lanes of a row read LDS together, each a table
-// entry p * 9 + j (or q * 9 + j): two different spin pairs with the same
-// residue mod 16 in one run of 16 fall on one bank, and the read takes as many
-// passes as the largest number of distinct spin pairs on a bank (equal pairs
-// broadcast).  The host therefore builds runs of 16 (the first one filling the
-// 16-term group the previous structure's terms end in) with distinct residues
-// of p and of q where the table allows (the order was fitted to 8-byte
-// reads; for the FP32 16-byte pair reads an order of runs of 8 with distinct
-// residues mod 8 measured the same): each slot takes a term from the
-// (p mod 16, q mod 16) bucket whose residues are still free in the run,
-// preferring the residues with most terms left; then pairwise swaps between
-// runs that do not raise the two runs' summed passes.  On the reference's
-// tables the passes per read drop from 1.6 (a Latin-square walk over the
-// buckets) to 1.3.  The sum is the same up to rounding.
-static int run_passes(const TetraTerm *r, int n) {
-  uint16_t mp[16] = {0}, mq[16] = {0};  // distinct spin pairs per residue (bit s1 / s2)
-  for (int i = 0; i < n; i++) {
-    const int p = r[i] & 255, q = (r[i] >> 8) & 255;
-    mp[p & 15] |= (uint16_t)(1u << (p >> 4));
-    mq[q & 15] |= (uint16_t)(1u << (q >> 4));
-  }
-  int dp = 0, dq = 0;
-  for (int k = 0; k < 16; k++) {
-    dp = std::max(dp, __builtin_popcount(mp[k]));
-    dq = std::max(dq, __builtin_popcount(mq[k]));
-  }
-  return dp + dq;
-}
+// a product: its coefficient per operator
+struct TetraProd {
+  std::vector<std::pair<int, std::array<double, 2>>> v;
+};
 
-static void order_runs(std::vector<TetraTerm> &v, int first_run) {
-  const int n = (int)v.size();
-  if (n <= 1) return;
-  std::vector<TetraTerm> bucket[256];
-  int cp[16] = {0}, cq[16] = {0};
-  for (TetraTerm u : v) {
-    const int pr = (u & 255) & 15, qr = ((u >> 8) & 255) & 15;
-    bucket[pr * 16 + qr].push_back(u);
-    cp[pr]++;
-    cq[qr]++;
-  }
-  std::vector<int> start;  // run boundaries in the output
-  std::vector<TetraTerm> out;
-  out.reserve(n);
-  int sz = first_run > 0 ? first_run : 16;
-  while ((int)out.size() < n) {
-    start.push_back((int)out.size());
-    unsigned usedp = 0, usedq = 0;
-    for (int slot = 0; slot < sz && (int)out.size() < n; slot++) {
-      int best = -1, bs = -1;
-      for (int b = 0; b < 256; b++) {
-        if (bucket[b].empty()) continue;
-        const int pr = b >> 4, qr = b & 15;
-        const int sc = ((usedp >> pr & 1) ? 0 : 1 << 22) + ((usedq >> qr & 1) ? 0 : 1 << 22) + cp[pr] + cq[qr];
-        if (sc > bs) {
-          bs = sc;
-          best = b;
-        }
-      }
-      const int pr = best >> 4, qr = best & 15;
-      out.push_back(bucket[best].back());
-      bucket[best].pop_back();
-      cp[pr]--;
-      cq[qr]--;
-      usedp |= 1u << pr;
-      usedq |= 1u << qr;
-    }
-    sz = 16;
-  }
-  start.push_back(n);
-  const int nr = (int)start.size() - 1;
-  if (nr > 1) {
-    std::vector<int> cost(nr);
-    for (int r = 0; r < nr; r++) cost[r] = run_passes(&out[start[r]], start[r + 1] - start[r]);
-    uint64_t st = 0x9e3779b97f4a7c15ull ^ (uint64_t)n;  // fixed seed: a table always packs alike
-    auto rnd = [&](uint64_t m) {
-      st = st * 6364136223846793005ull + 1442695040888963407ull;
-      return (int)((st >> 33) % m);
-    };
-    for (int it = 0; it < 16 * n; it++) {
-      const int a = rnd(nr), b = rnd(nr);
-      if (a == b) continue;
-      const int i = start[a] + rnd(start[a + 1] - start[a]), j = start[b] + rnd(start[b + 1] - start[b]);
-      std::swap(out[i], out[j]);
-      const int ca = run_passes(&out[start[a]], start[a + 1] - start[a]);
-      const int cb = run_passes(&out[start[b]], start[b + 1] - start[b]);
-      if (ca + cb <= cost[a] + cost[b]) {
-        cost[a] = ca;
-        cost[b] = cb;
-      } else {
-        std::swap(out[i], out[j]);
-      }
-    }
-  }
-  v.swap(out);
-}
-
-// host: classify and pack the terms of a table (reference format)
-int tetra_pack(const int16_t *idxs, const int16_t *cols, const float *vals, const int16_t *counts, int nops,
-               TetraPacked &out) {
-  if (nops <= 0 || nops > TETRA_MAXOPS) return PLG_ERR_UNSUPPORTED;
+// the walk of operators k0 .. k0 + nops - 1; index: the product of each
+// set << 17 | structure << 16 | p << 8 | q (structure 0 crossed, 1 direct)
+static void tetra_walk(const std::vector<TetraProd> &prods, const std::vector<int> &index, int k0, int nops,
+                       TetraPacked &out) {
   out = TetraPacked{};
-  for (int h = 0; h < 2; h++) {
-    out.first[h].assign(nops, 0);
-    out.count[h].assign(nops, 0);
-    out.ndirect[h].assign(nops, 0);
+  auto used = [&](int id) {
+    return id >= 0 && std::any_of(prods[id].v.begin(), prods[id].v.end(),
+                                  [&](const auto &kv) { return kv.first >= k0 && kv.first < k0 + nops; });
+  };
+  // per (set, p): its groups of one structure and s2, most products first
+  struct Group {
+    int s2;
+    std::vector<std::pair<int, int>> e;  // s4, product
+  };
+  struct Item {
+    int p;
+    std::array<std::vector<Group>, 2> g;  // crossed, direct
+    std::vector<int> sig;
+    int n = 0;
+  };
+  struct Step {
+    int set;
+    std::array<const Item *, 4> it;
+    int cost;
+  };
+  std::array<std::vector<Item>, 2> items;
+  std::vector<Step> steps;
+  for (int set = 0; set < 2; set++) {
+    for (int p = 0; p < 256; p++) {
+      Item I;
+      I.p = p;
+      for (int ty = 0; ty < 2; ty++) {
+        for (int s2 = 0; s2 < 16; s2++) {
+          Group G;
+          G.s2 = s2;
+          for (int s4 = 0; s4 < 16; s4++) {
+            const int id = index[set << 17 | ty << 16 | p << 8 | s2 * 16 + s4];
+            if (used(id)) G.e.push_back({s4, id});
+          }
+          I.n += (int)G.e.size();
+          if (!G.e.empty()) I.g[ty].push_back(G);
+        }
+        std::stable_sort(I.g[ty].begin(), I.g[ty].end(),
+                         [](const Group &a, const Group &b) { return a.e.size() > b.e.size(); });
+        for (const Group &G : I.g[ty]) I.sig.push_back((int)G.e.size());
+        I.sig.push_back(0);
+      }
+      if (I.n) items[set].push_back(I);
+    }
+    // steps of four spin pairs p with like groups
+    std::stable_sort(items[set].begin(), items[set].end(),
+                     [](const Item &a, const Item &b) { return a.n != b.n ? a.n > b.n : a.sig > b.sig; });
+    for (size_t i = 0; i < items[set].size(); i += 4) {
+      Step st;
+      st.set = set;
+      st.cost = 4;
+      for (size_t j = 0; j < 4; j++) {
+        st.it[j] = i + j < items[set].size() ? &items[set][i + j] : nullptr;
+        if (st.it[j])
+          st.cost = std::max(st.cost, 4 + 2 * st.it[j]->n + 4 * (int)st.it[j]->g[0].size() + 2 * (int)st.it[j]->g[1].size());
+      }
+      steps.push_back(st);
+    }
   }
-  std::map<std::pair<uint32_t, uint32_t>, uint32_t> cidx;  // coefficient bits -> index
-  cidx.emplace(std::make_pair(0u, 0u), 0u);                 // entry 0: zero
-  out.coef.push_back(0.0f);
-  out.coef.push_back(0.0f);
+  std::stable_sort(steps.begin(), steps.end(), [](const Step &a, const Step &b) { return a.cost > b.cost; });
+  std::array<std::vector<const Step *>, TT_WAVES> mine;
+  std::array<int, TT_WAVES> load{};
+  for (const Step &st : steps) {
+    const int w = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+    load[w] += st.cost;
+    mine[w].push_back(&st);
+  }
+  const int NB = (nops + 15) / 16;
+  for (int w = 0; w < TT_WAVES; w++) {
+    out.s.word0[w] = (int)out.words.size();
+    out.s.coef0[w] = (int)(out.coef.size() / 64);
+    out.s.nsteps[w] = (int)mine[w].size();
+    for (const Step *st : mine[w]) {
+      uint32_t pw = 0;
+      size_t ng[2] = {0, 0};
+      for (int j = 0; j < 4; j++)
+        if (st->it[j]) {
+          pw |= (uint32_t)st->it[j]->p << (8 * j);
+          for (int ty = 0; ty < 2; ty++) ng[ty] = std::max(ng[ty], st->it[j]->g[ty].size());
+        }
+      out.words.push_back(pw);
+      out.words.push_back((uint32_t)ng[0] | (uint32_t)ng[1] << 8 | (uint32_t)st->set << 16);
+      for (int ty = 0; ty < 2; ty++)
+        for (size_t g = 0; g < ng[ty]; g++) {
+          uint32_t gw = 0;
+          size_t nt = 0;
+          const Group *G[4];
+          for (int j = 0; j < 4; j++) {
+            G[j] = st->it[j] && g < st->it[j]->g[ty].size() ? &st->it[j]->g[ty][g] : nullptr;
+            if (!G[j]) continue;
+            gw |= (uint32_t)G[j]->s2 << (4 * j);
+            nt = std::max(nt, G[j]->e.size());
+          }
+          out.words.push_back(gw | (uint32_t)nt << 16);
+          for (size_t e = 0; e < nt; e++) {
+            uint32_t uw = 0;
+            double V[2][4][64] = {};  // [real, imaginary][operator block][quarter * 16 + operator]
+            for (int j = 0; j < 4; j++) {
+              if (!G[j] || e >= G[j]->e.size()) continue;
+              uw |= (uint32_t)G[j]->e[e].first << (4 * j);
+              for (const auto &kv : prods[G[j]->e[e].second].v) {
+                const int k = kv.first - k0;
+                if (k < 0 || k >= nops) continue;
+                for (int h = 0; h < 2; h++) V[h][k / 16][16 * j + k % 16] = kv.second[h];
+              }
+            }
+            for (int h = 0; h < 2; h++)
+              for (int b = 0; b < NB; b++)
+                if (std::any_of(V[h][b], V[h][b] + 64, [](double v) { return v != 0; })) {
+                  uw |= 1u << (16 + 4 * h + b);
+                  out.coef.insert(out.coef.end(), V[h][b], V[h][b] + 64);
+                }
+            out.words.push_back(uw);
+          }
+        }
+    }
+    out.words.resize((out.words.size() + 63) / 64 * 64 + 128, 0u);  // the reads ahead
+  }
+  out.coef.resize(out.coef.size() + 3 * 64, 0.0);
+  out.s.nops = nops;
+}
+
+// host: classify the terms of a table (reference format) and lay out the
+// walks, one per `per` operators
+int tetra_pack(const int16_t *idxs, const int16_t *cols, const float *vals, const int16_t *counts, int nops, int per,
+               std::vector<TetraPacked> &out) {
+  if (nops <= 0 || nops > TETRA_MAXOPS) return PLG_ERR_UNSUPPORTED;
+  std::map<std::pair<uint32_t, uint32_t>, int> cidx;  // distinct coefficients, zero among them
+  cidx.emplace(std::make_pair(0u, 0u), 0);
+  std::vector<TetraProd> prods;
+  std::vector<int> index(1 << 18, -1);
   size_t t = 0;
   for (int k = 0; k < nops; k++) {
     if (counts[k] < 0) return PLG_ERR_INVALID;
-    std::vector<TetraTerm> direct[2], crossed[2];
     for (int i = 0; i < counts[k]; i++, t++) {
       const int16_t *m = idxs + 8 * t, *c = cols + 8 * t;
       for (int j = 0; j < 8; j++)
@@ -389,43 +409,36 @@ int tetra_pack(const int16_t *idxs, const int16_t *cols, const float *vals, cons
       for (int a = 0; a < 4; a++)
         for (int b = a + 1; b < 4; b++) perm &= c[a] != c[b];
       if (!perm) return PLG_ERR_UNSUPPORTED;
-      const uint32_t s1 = m[0] * 4 + m[1], s2 = m[2] * 4 + m[3];
-      const uint32_t s3 = ((m[5] + 2) & 3) * 4 + ((m[4] + 2) & 3), s4 = ((m[7] + 2) & 3) * 4 + ((m[6] + 2) & 3);
+      const int s1 = m[0] * 4 + m[1], s2 = m[2] * 4 + m[3];
+      const int s3 = ((m[5] + 2) & 3) * 4 + ((m[4] + 2) & 3), s4 = ((m[7] + 2) & 3) * 4 + ((m[6] + 2) & 3);
       uint32_t re, im;
       std::memcpy(&re, vals + 2 * t, 4);
       std::memcpy(&im, vals + 2 * t + 1, 4);
-      auto it = cidx.find({re, im});
-      uint32_t ci;
-      if (it != cidx.end()) {
-        ci = it->second;
-      } else {
-        ci = (uint32_t)cidx.size();
-        if (ci >= (uint32_t)TETRA_MAXCOEF) return PLG_ERR_UNSUPPORTED;
-        cidx.emplace(std::make_pair(re, im), ci);
-        out.coef.push_back(vals[2 * t]);
-        out.coef.push_back(vals[2 * t + 1]);
-      }
+      if (cidx.emplace(std::make_pair(re, im), 0).second && (int)cidx.size() > TETRA_MAXCOEF)
+        return PLG_ERR_UNSUPPORTED;
       // set 0 on (P1, P2, P3, P4); set 1 on (P1, P2, P4, P3): P4's spin pair
       // takes the third place and P3's the fourth
-      const TetraTerm u0 = (s1 * 16 + s3) | ((s2 * 16 + s4) << 8) | (ci << 16);
-      const TetraTerm u1 = (s1 * 16 + s4) | ((s2 * 16 + s3) << 8) | (ci << 16);
-      if (c[0] == c[5] && c[1] == c[4] && c[2] == c[7] && c[3] == c[6]) direct[0].push_back(u0);
-      else if (c[0] == c[5] && c[1] == c[6] && c[2] == c[7] && c[3] == c[4]) crossed[0].push_back(u0);
-      else if (c[0] == c[7] && c[1] == c[6] && c[2] == c[5] && c[3] == c[4]) direct[1].push_back(u1);
-      else if (c[0] == c[7] && c[1] == c[4] && c[2] == c[5] && c[3] == c[6]) crossed[1].push_back(u1);
+      const int u0 = (s1 * 16 + s3) << 8 | (s2 * 16 + s4), u1 = (s1 * 16 + s4) << 8 | (s2 * 16 + s3);
+      int key;
+      if (c[0] == c[5] && c[1] == c[4] && c[2] == c[7] && c[3] == c[6]) key = 1 << 16 | u0;
+      else if (c[0] == c[5] && c[1] == c[6] && c[2] == c[7] && c[3] == c[4]) key = u0;
+      else if (c[0] == c[7] && c[1] == c[6] && c[2] == c[5] && c[3] == c[4]) key = 3 << 16 | u1;
+      else if (c[0] == c[7] && c[1] == c[4] && c[2] == c[5] && c[3] == c[6]) key = 2 << 16 | u1;
       else return PLG_ERR_UNSUPPORTED;
+      if (index[key] < 0) {
+        index[key] = (int)prods.size();
+        prods.emplace_back();
+      }
+      auto &v = prods[index[key]].v;
+      if (v.empty() || v.back().first != k) v.push_back({k, {0.0, 0.0}});
+      v.back().second[0] += (double)vals[2 * t];
+      v.back().second[1] += (double)vals[2 * t + 1];
     }
-    for (int h = 0; h < 2; h++) {
-      std::vector<TetraTerm> &terms = out.terms[h];
-      out.first[h][k] = (int)terms.size();
-      order_runs(direct[h], 16);
-      // the crossed terms start in the 16-term group the direct ones end in
-      order_runs(crossed[h], (int)(16 - direct[h].size() % 16));
-      terms.insert(terms.end(), direct[h].begin(), direct[h].end());
-      terms.insert(terms.end(), crossed[h].begin(), crossed[h].end());
-      out.ndirect[h][k] = (int)direct[h].size();
-      out.count[h][k] = (int)terms.size() - out.first[h][k];
-    }
+  }
+  out.clear();
+  for (int k0 = 0; k0 < nops; k0 += per) {
+    out.emplace_back();
+    tetra_walk(prods, index, k0, std::min(per, nops - k0), out.back());
   }
   return PLG_OK;
 }
