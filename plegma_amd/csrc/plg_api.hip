@@ -679,9 +679,10 @@ static std::string launch_name(const Plan &P, const Launch &l) {
 template <typename T> static int launch_contract_t(const Plan &P, const Launch &l, void *c, hipStream_t st) {
   auto *pd = (const PropDev<T> *)P.d_props;
   const int nrows = (int)P.rows.size();
+  const bool rot = std::any_of(P.props.begin(), P.props.end(), [](const plg_prop &v) { return v.rotate_sign != 0; });
   switch (l.what) {
   case Launch::MESON:
-    return launch_meson<T>(l.set, pd, P.d_rows, nrows, (cx<T> *)c, g_ctx.V3, g_ctx.L[3], P.nch_c, l.ch0, st);
+    return launch_meson<T>(l.set, pd, P.d_rows, nrows, (cx<T> *)c, g_ctx.V3, g_ctx.L[3], P.nch_c, l.ch0, rot, st);
   case Launch::MESMES:
     return launch_mesmes<T>(pd, P.d_rows, nrows, (cx<T> *)c, g_ctx.V3, g_ctx.L[3], P.nch_c, l.ch0, P.tpb, st);
   case Launch::UDSC:

@@ -181,7 +181,7 @@ int launch_udsc_all(const UdscAll &S, const PropDev<T> *props, const RowDev *row
 
 template <typename T>
 int launch_meson(int set, const PropDev<T> *props, const RowDev *rows, int nrows, cx<T> *out,
-                 int64_t V3, int T_lat, int nch_total, int ch0, hipStream_t st);
+                 int64_t V3, int T_lat, int nch_total, int ch0, bool rot, hipStream_t st);
 template <typename T>
 int launch_mesmes(const PropDev<T> *props, const RowDev *rows, int nrows, cx<T> *out, int64_t V3, int T_lat,
                   int nch_total, int ch0, int tiles_per_block, hipStream_t st);
