@@ -1,5 +1,5 @@
 // plg_baryon.hip -- baryon two-point contractions (and the fused meson +
-// baryon kernel of the mixed path) on gfx950.
+// baryon two-point kernel) on gfx950.
 //
 // Replaces PLEGMA_baryons_NtoN.cu:6-46 (proton, Cg5 x Cg5) and
 // PLEGMA_baryons_deltas.cu:61-110 (Delta iso-3/2, Cg_k x g4 (Cg_k)^dag g4)

@@ -14,8 +14,8 @@
 //                   reads site x0+i of one spin-colour component.
 //  k_meson_all      PLEGMA_mesonsAll.cuh:27-83: four lanes per site.
 //
-//  The baryon contractions (and the fused meson + baryon kernel of the mixed
-//  path) are in plg_baryon.hip.
+//  The baryon contractions and the fused meson + baryon kernel are in
+//  plg_baryon.hip.
 #include "plg_tile.h"
 
 namespace plg {
