@@ -6,6 +6,7 @@ fallback.  torch supplies device memory and streams only.
 from __future__ import annotations
 
 import ctypes as C
+import itertools
 import os
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -153,6 +154,17 @@ def ivec(v):
     return (C.c_int * len(v))(*[int(x) for x in v])
 
 
+def _flat(moms):
+    """momentum triples as a C int array, None for an empty list"""
+    v = list(itertools.chain.from_iterable(moms))
+    if not v:
+        return None
+    try:
+        return (C.c_int * len(v))(*v)
+    except TypeError:  # floats and the like
+        return ivec(v)
+
+
 def _stream(s):
     if s is None:
         return None
@@ -203,18 +215,18 @@ def prop_view(tensor, precision, t_first=0, nt=None, V3=None, T=None):
 
 def correlator(kind, mask, p1, p2, source, totalT, moms, mode, space, out_prec, out,
                stream=None):
-    flat = [int(v) for m in moms for v in m]
+    flat = _flat(moms)
     check(lib().plg_correlator(kind, mask, C.byref(p1), C.byref(p2) if p2 is not None else None,
-                               ivec(source), totalT, ivec(flat) if flat else None, len(moms), mode,
+                               ivec(source), totalT, flat, len(moms), mode,
                                space, out_prec, C.c_void_p(out.data_ptr()), _stream(stream)))
 
 
 def correlator_static(kind, mask, p1, p2, source, totalT, moms, mode, space, out_prec, out,
                       stream=None):
     """plg_correlator without device allocation (the library's static scratch)"""
-    flat = [int(v) for m in moms for v in m]
+    flat = _flat(moms)
     check(lib().plg_correlator_static(kind, mask, C.byref(p1), C.byref(p2) if p2 is not None else None,
-                                      ivec(source), totalT, ivec(flat) if flat else None, len(moms), mode,
+                                      ivec(source), totalT, flat, len(moms), mode,
                                       space, out_prec, C.c_void_p(out.data_ptr()), _stream(stream)))
 
 
@@ -230,8 +242,8 @@ def ft_apply(field, precision, dof, nt, moms, sign, out, out_prec=F64, accumulat
             and moms.flags.c_contiguous:
         mp, n = moms.ctypes.data_as(C.POINTER(C.c_int)), moms.shape[0]
     else:
-        flat = [int(v) for m in moms for v in m]
-        mp, n = ivec(flat), len(flat) // 3
+        flat = _flat(moms)
+        mp, n = flat, len(flat) // 3 if flat else 0
     check(lib().plg_ft_apply(C.c_void_p(field.data_ptr()), precision, dof, nt, mp, n, sign,
                              int(accumulate), C.c_void_p(out.data_ptr()), out_prec, _stream(stream)))
 
@@ -270,21 +282,21 @@ def udsc_select(up, dn, st, ch, only_st=False, only_ch=False):
 def baryons_udsc(up, dn, st, ch, source, totalT, moms, mode, space, out_prec, out, only_st=False, only_ch=False,
                  stream=None):
     """contractBaryonsUDSC: views up/dn/st/ch (None = absent) -> out [dataset][j][m]"""
-    flat = [int(v) for m in moms for v in m]
+    flat = _flat(moms)
     check(lib().plg_baryons_udsc(_ref(up), _ref(dn), _ref(st), _ref(ch), int(only_st), int(only_ch),
-                                 ivec(source), totalT, ivec(flat) if flat else None, len(moms), mode, space,
+                                 ivec(source), totalT, flat, len(moms), mode, space,
                                  out_prec, C.c_void_p(out.data_ptr()), _stream(stream)))
 
 
 def baryons_udsc_profile(up, dn, st, ch, source, totalT, moms, mode, space, out_prec, out, only_st=False,
                          only_ch=False, stream=None, cap=16):
     """one baryons_udsc pass with events between stages: {stage: ms summed over products}"""
-    flat = [int(v) for m in moms for v in m]
+    flat = _flat(moms)
     n = C.c_int()
     ms = (C.c_double * cap)()
     names = C.create_string_buffer(32 * cap)
     check(lib().plg_baryons_udsc_profile(_ref(up), _ref(dn), _ref(st), _ref(ch), int(only_st), int(only_ch),
-                                         ivec(source), totalT, ivec(flat) if flat else None, len(moms), mode, space,
+                                         ivec(source), totalT, flat, len(moms), mode, space,
                                          out_prec, C.c_void_p(out.data_ptr()), _stream(stream), cap, C.byref(n), ms,
                                          names))
     raw = names.raw
@@ -299,10 +311,10 @@ def baryons_table(p1, p2, p3, idxs, vals, counts, source, totalT, moms, mode, sp
     idxs = np.ascontiguousarray(idxs, dtype=np.int16)
     vals = np.ascontiguousarray(vals, dtype=np.float32)
     counts = np.ascontiguousarray(counts, dtype=np.int16)
-    flat = [int(v) for m in moms for v in m]
+    flat = _flat(moms)
     check(lib().plg_baryons_table(C.byref(p1), C.byref(p2), C.byref(p3), idxs.ctypes.data, vals.ctypes.data,
                                   counts.ctypes.data, len(counts), ivec(source), totalT,
-                                  ivec(flat) if flat else None, len(moms), mode, space, out_prec,
+                                  flat, len(moms), mode, space, out_prec,
                                   C.c_void_p(out.data_ptr()), _stream(stream)))
 
 
@@ -316,10 +328,10 @@ def tetraquark_table(p1, p2, p3, p4, idxs, cols, vals, counts, source, totalT, m
     cols = np.ascontiguousarray(cols, dtype=np.int16)
     vals = np.ascontiguousarray(vals, dtype=np.float32)
     counts = np.ascontiguousarray(counts, dtype=np.int16)
-    flat = [int(v) for m in moms for v in m]
+    flat = _flat(moms)
     check(lib().plg_tetraquark_table(C.byref(p1), C.byref(p2), C.byref(p3), C.byref(p4), idxs.ctypes.data,
                                      cols.ctypes.data, vals.ctypes.data, counts.ctypes.data, len(counts),
-                                     ivec(source), totalT, ivec(flat) if flat else None, len(moms), mode, space,
+                                     ivec(source), totalT, flat, len(moms), mode, space,
                                      out_prec, C.c_void_p(out.data_ptr()), _stream(stream)))
 
 
@@ -375,9 +387,9 @@ def tetraquarks(lt, st, ch, bt, source, totalT, moms, mode, space, out_prec, out
                 stream=None, family="heavy-light"):
     """contractTetraquarks (family "heavy-light") or contractTetraquarksBCUD
     (family "bcud"): views lt/st/ch/bt (None = absent) -> out [dataset][j][m]"""
-    flat = [int(v) for m in moms for v in m]
+    flat = _flat(moms)
     check(_tf("plg_tetraquarks", family)(_ref(lt), _ref(st), _ref(ch), _ref(bt), int(only_st), int(only_ch),
-                                         ivec(source), totalT, ivec(flat) if flat else None, len(moms), mode,
+                                         ivec(source), totalT, flat, len(moms), mode,
                                          space, out_prec, C.c_void_p(out.data_ptr()), _stream(stream)))
 
 
@@ -408,9 +420,9 @@ class Batch:
             J[i].prop = prop
             J[i].prop2 = job[4] if len(job) > 4 else -1
             J[i].out_offset = off
-        flat = [int(v) for m in moms for v in m]
+        flat = _flat(moms)
         h = C.c_void_p()
-        check(lib().plg_batch_create(kind, mask, P, len(props), J, len(jobs), ivec(flat),
+        check(lib().plg_batch_create(kind, mask, P, len(props), J, len(jobs), flat,
                                      len(moms), mode, split, flags, C.byref(h)))
         self.h = h
         self._keep = (P, J)

@@ -56,6 +56,8 @@ struct Context {
   size_t ws_c_bytes = 0;
   void *ws_part = nullptr;
   size_t ws_part_bytes = 0;
+  void *ws_tab = nullptr;        // the tables of a plan that lives for one call
+  size_t ws_tab_bytes = 0;
 };
 static Context g_ctx;
 // g_mu guards the context (tables, workspace sizes, udsc schedules).
@@ -922,21 +924,24 @@ struct FtTables {
 };
 static FtTables g_ft;
 
+static void key_add(std::string &k, const void *v, size_t n) { k.append((const char *)v, n); }
+template <typename... A> static void key_put(std::string &k, const A &...v) { (key_add(k, &v, sizeof v), ...); }
+
+// the call as a byte string (its integers and addresses, then the settings
+// read from the environment)
 static std::string single_key(int kind, int mask, const std::vector<plg_prop> &props, const int src[4], int totalT,
                               const int *moms, int nmom, int mode, int space) {
-  std::ostringstream k;
-  k << kind << ' ' << mask << ' ' << mode << ' ' << space << ' ' << totalT;
-  for (int i = 0; i < 4; i++) k << ' ' << src[i];
+  std::string k;
+  k.reserve(256 + 12 * (size_t)std::max(nmom, 0));
+  key_put(k, kind, mask, mode, space, totalT, nmom);
+  key_add(k, src, 4 * sizeof(int));
   for (const plg_prop &p : props)
-    k << " | " << p.data << ' ' << p.precision << ' ' << p.t_first << ' ' << p.nt << ' ' << p.comp_stride << ' '
-      << (const void *)p.plane_exp << ' ' << p.rotate_sign << ' ' << p.bc_t0;
-  k << " | " << nmom;
-  if (moms && space == PLG_MOMENTUM_SPACE)
-    for (int i = 0; i < 3 * nmom; i++) k << ' ' << moms[i];
+    key_put(k, p.data, p.precision, p.t_first, p.nt, p.comp_stride, p.plane_exp, p.rotate_sign, p.bc_t0);
+  if (moms && space == PLG_MOMENTUM_SPACE && nmom > 0) key_add(k, moms, 3 * (size_t)nmom * sizeof(int));
   // a pinned projection tile (PLG_PROJ_CODE) is part of the plan
-  if (const char *e = std::getenv("PLG_PROJ_CODE")) k << " code=" << e;
-  if (const char *e = std::getenv("PLG_PROJ_SEP")) k << " sep=" << e;
-  return k.str();
+  if (const char *e = std::getenv("PLG_PROJ_CODE")) k += std::string(" code=") + e;
+  if (const char *e = std::getenv("PLG_PROJ_SEP")) k += std::string(" sep=") + e;
+  return k;
 }
 
 static Plan *single_lookup(const std::string &key) {
@@ -1004,8 +1009,9 @@ static int put_async(ScratchCarver &sc, A **dst, const std::vector<A> &v, hipStr
   return PLG_OK;
 }
 
-// the device tables of a plan that lives in the static scratch: pointers
-// into the array, cleared before the plan is destroyed (it owns none of them)
+// the device tables of a plan that lives in the static scratch or in the
+// context's table buffer: pointers into the array, cleared before the plan is
+// destroyed (it owns none of them)
 static void release_static(Plan &P) {
   P.d_props = nullptr;
   P.d_rows = nullptr;
@@ -1170,7 +1176,7 @@ static void finalize_locked() {
   g_single.clear();
   g_ft.release();
   tetra_tables_clear();
-  for (void *p : {(void *)g_ctx.d_cos, (void *)g_ctx.d_sin, (void *)g_ctx.d_wtab, g_ctx.ws_c, g_ctx.ws_part})
+  for (void *p : {(void *)g_ctx.d_cos, (void *)g_ctx.d_sin, (void *)g_ctx.d_wtab, g_ctx.ws_c, g_ctx.ws_part, g_ctx.ws_tab})
     if (p) hipFree(p);
   for (void *p : g_ctx.udsc_mem) hipFree(p);
   g_ctx = Context();
@@ -1434,19 +1440,59 @@ static int udsc_check_args(const void *out, const int *source, int out_precision
   return PLG_OK;
 }
 
-// tables, workspace and launches of a plan of a single call, waited for
+// Tables, workspace and launches of a plan that lives for one call, waited
+// for.  The tables go up as one copy into the context's table buffer: a device
+// allocation, copy and free for each of the nine took 200 us of every call.
 static int plan_run(Plan &P, void *out, int out_precision, hipStream_t hs, std::map<std::string, double> *stage_ms) {
   int rc;
-  if ((rc = upload_plan(P, hs))) return rc;
+  std::vector<unsigned char> blob;
+  auto add = [&](const void *v, size_t n) {
+    const size_t off = (blob.size() + 255) / 256 * 256;
+    blob.resize(off + std::max<size_t>(n, 1));
+    if (n) std::memcpy(blob.data() + off, v, n);
+    return off;
+  };
+  auto addv = [&](const auto &v) { return add(v.data(), v.size() * sizeof(v[0])); };
+  size_t o_props;
+  if (P.T == PLG_F64) {
+    std::vector<PropDev<double>> pd;
+    fill_propdev(P.props, pd);
+    o_props = addv(pd);
+  } else {
+    std::vector<PropDev<float>> pd;
+    fill_propdev(P.props, pd);
+    o_props = addv(pd);
+  }
+  const size_t o_rows = addv(P.rows), o_orows = addv(P.orows), o_csel = addv(P.csel), o_choff = addv(P.ch_off);
+  const size_t o_ms = addv(P.ms), o_pair = addv(P.pair_ms), o_mom = addv(P.mom_pair);
+  const bool sep = plan_sep(P), pidx = !sep && P.npairs > 0 && P.T == PLG_F32;
+  const size_t o_sep = sep ? addv(P.sep.blob) : 0, o_pidx = (blob.size() + 255) / 256 * 256;
   std::lock_guard<std::mutex> wl(g_ws_mu);  // until the stream is synchronised below
   {
     std::lock_guard<std::mutex> lk(g_mu);
     if ((rc = ensure(&g_ctx.ws_c, &g_ctx.ws_c_bytes, c_bytes(P)))) return rc;
     if ((rc = ensure(&g_ctx.ws_part, &g_ctx.ws_part_bytes, part_bytes(P)))) return rc;
+    if ((rc = ensure(&g_ctx.ws_tab, &g_ctx.ws_tab_bytes,
+                     o_pidx + (pidx ? phase_index_bytes(g_ctx.V3, P.npairs) : 0))))
+      return rc;
   }
+  unsigned char *d = (unsigned char *)g_ctx.ws_tab;
+  HIPCHK(hipMemcpyAsync(d, blob.data(), blob.size(), hipMemcpyHostToDevice, hs));
+  P.d_props = d + o_props;
+  P.d_rows = (RowDev *)(d + o_rows);
+  P.d_orows = (OutRowDev *)(d + o_orows);
+  P.d_csel = (int *)(d + o_csel);
+  P.d_choff = (int64_t *)(d + o_choff);
+  P.d_ms = (int *)(d + o_ms);
+  P.d_pair_ms = (int *)(d + o_pair);
+  P.d_mom_pair = (int *)(d + o_mom);
+  if (sep) P.d_sep = d + o_sep;
+  if (pidx) P.d_pidx = (uint16_t *)(d + o_pidx);
+  rc = pidx ? launch_phase_index(plan_geom(P), P.d_pidx, hs) : PLG_OK;
+  if (rc) rc = fail(rc, "phase index launch failed");
   StageLog log;
-  rc = enqueue(P, g_ctx.ws_c, g_ctx.ws_part, out, out_precision, hs, stage_ms ? &log : nullptr);
-  // the plan's tables are freed on return: wait for every launch, also after an error
+  if (!rc) rc = enqueue(P, g_ctx.ws_c, g_ctx.ws_part, out, out_precision, hs, stage_ms ? &log : nullptr);
+  // the tables are the next call's after this: wait for every launch, also after an error
   const hipError_t se = hipStreamSynchronize(hs);
   if (!rc && se != hipSuccess) rc = fail(PLG_ERR_HIP, "synchronisation failed");
   for (size_t i = 0; i + 1 < log.ev.size(); i++) {
@@ -1455,6 +1501,7 @@ static int plan_run(Plan &P, void *out, int out_precision, hipStream_t hs, std::
     (*stage_ms)[log.name[i + 1]] += t;
   }
   for (hipEvent_t e : log.ev) hipEventDestroy(e);
+  release_static(P);
   return rc;
 }
 
@@ -1608,8 +1655,8 @@ static int udsc_run(const plg_prop *up, const plg_prop *dn, const plg_prop *st, 
 
 // Packed tables by content (laying out a table takes milliseconds per ten
 // thousand terms): the last few tables, with their device arrays, keyed by a
-// 64-bit hash of the counts, spins, colour slots and coefficients and by the
-// precision.  A table whose device arrays are large is not kept.
+// 64-bit hash of the counts, spins, colour slots and coefficients (a built-in
+// table by its number) and by the precision.  A table whose device arrays are large is not kept.
 struct TetraTable {
   std::vector<TetraSched> s;  // one per launch
   std::vector<void *> mem;
@@ -1639,19 +1686,24 @@ static uint64_t hash_bytes(const void *data, size_t n, uint64_t h) {
   return h;
 }
 
+// builtin: the number of a built-in table, which needs no hash (a read of
+// 0.5 to 2.5 MB); -1: a caller's table
 static int tetra_pack_cached(const int16_t *idxs, const int16_t *cols, const float *vals, const int16_t *counts,
-                             int nops, int T, std::shared_ptr<const TetraTable> &out) {
+                             int nops, int builtin, int T, std::shared_ptr<const TetraTable> &out) {
   if (nops <= 0 || nops > TETRA_MAXOPS) return PLG_ERR_UNSUPPORTED;
   size_t nt = 0;
   for (int k = 0; k < nops; k++) {
     if (counts[k] < 0) return PLG_ERR_INVALID;
     nt += (size_t)counts[k];
   }
-  uint64_t h = 0xcbf29ce484222325ull ^ (uint64_t)nops ^ (uint64_t)T << 32;
-  h = hash_bytes(counts, nops * sizeof(int16_t), h);
-  h = hash_bytes(idxs, nt * 8 * sizeof(int16_t), h);
-  h = hash_bytes(cols, nt * 8 * sizeof(int16_t), h);
-  h = hash_bytes(vals, nt * 2 * sizeof(float), h);
+  uint64_t h = (uint64_t)(2 * builtin + (T == PLG_F64 ? 1 : 0));
+  if (builtin < 0) {
+    h = 0xcbf29ce484222325ull ^ (uint64_t)nops ^ (uint64_t)T << 32;
+    h = hash_bytes(counts, nops * sizeof(int16_t), h);
+    h = hash_bytes(idxs, nt * 8 * sizeof(int16_t), h);
+    h = hash_bytes(cols, nt * 8 * sizeof(int16_t), h);
+    h = hash_bytes(vals, nt * 2 * sizeof(float), h);
+  }
   {
     std::lock_guard<std::mutex> lk(g_pack_mu);
     for (auto &e : g_pack_cache)
@@ -1692,8 +1744,8 @@ static int tetra_pack_cached(const int16_t *idxs, const int16_t *cols, const flo
 // one four-propagator table (views P1..P4), its operators written as datasets
 // d0 .. d0 + nops - 1 of the output
 static int tetra_run(const plg_prop *const views[4], const int16_t *idxs, const int16_t *col_contr, const float *vals,
-                     const int16_t *counts, int nops, int d0, const int source[4], int totalT, const int *moms,
-                     int nmom, int mode, int space, int out_precision, void *out, void *stream) {
+                     const int16_t *counts, int nops, int builtin, int d0, const int source[4], int totalT,
+                     const int *moms, int nmom, int mode, int space, int out_precision, void *out, void *stream) {
   int rc;
   if ((rc = udsc_check_args(out, source, out_precision, mode, space, moms, nmom))) return rc;
   if (!idxs || !col_contr || !vals || !counts || nops <= 0) return fail(PLG_ERR_INVALID, "empty table");
@@ -1701,7 +1753,7 @@ static int tetra_run(const plg_prop *const views[4], const int16_t *idxs, const 
     if (!views[i]) return fail(PLG_ERR_INVALID, "NULL propagator view");
   const int prec = mode == PLG_MODE_F64 ? PLG_F64 : PLG_F32;
   std::shared_ptr<const TetraTable> tab;  // held until the stream is synchronised
-  rc = tetra_pack_cached(idxs, col_contr, vals, counts, nops, prec, tab);
+  rc = tetra_pack_cached(idxs, col_contr, vals, counts, nops, builtin, prec, tab);
   if (rc == PLG_ERR_INVALID) return fail(rc, "spin or colour index outside 0..3");
   if (rc == PLG_ERR_HIP) return rc;
   if (rc)
@@ -1765,7 +1817,7 @@ int plg_tetraquark_table(const plg_prop *p1, const plg_prop *p2, const plg_prop 
                          int nops, const int source[4], int totalT, const int *moms, int nmom, int mode, int space,
                          int out_precision, void *out, void *stream) {
   const plg_prop *views[4] = {p1, p2, p3, p4};
-  return tetra_run(views, idxs, col_contr, vals, counts, nops, 0, source, totalT, moms, nmom, mode, space,
+  return tetra_run(views, idxs, col_contr, vals, counts, nops, -1, 0, source, totalT, moms, nmom, mode, space,
                    out_precision, out, stream);
 }
 
@@ -1871,8 +1923,9 @@ static int tetra_products(const TetraSet &ts, const plg_prop *lt, const plg_prop
     const char *f = ts.prod[prod];
     const plg_prop *views[4];
     for (int i = 0; i < 4; i++) views[i] = fl[TT_VIEW_OF[std::find(TT_LETTERS, TT_LETTERS + 5, f[i]) - TT_LETTERS]];
-    if ((rc = tetra_run(views, ts.idx[prod], ts.col[prod], ts.val[prod], ts.count[prod], ts.nops[prod], d0, source,
-                        totalT, moms, nmom, mode, space, out_precision, out, stream)))
+    if ((rc = tetra_run(views, ts.idx[prod], ts.col[prod], ts.val[prod], ts.count[prod], ts.nops[prod],
+                        (&ts == &TETRA_BCUD ? TT_NPROD : 0) + prod, d0, source, totalT, moms, nmom, mode, space,
+                        out_precision, out, stream)))
       return rc;
     d0 += ts.nops[prod];
   }
@@ -2023,10 +2076,10 @@ int plg_ft_apply(const void *field, int precision, int dof, int nt, const int *m
   const char *sep_env = std::getenv("PLG_PROJ_SEP");
   // the separable sums read the field with 16-byte loads
   const bool sep_off = (sep_env && std::string(sep_env) == "0") || ((uintptr_t)field & 15);
-  std::ostringstream key;
-  key << precision << ' ' << dof << ' ' << nt << ' ' << sep_off;
-  for (int i = 0; i < 4; i++) key << ' ' << g_ctx.L[i];
-  for (int v : ms) key << ' ' << v;
+  std::string key;
+  key_put(key, precision, dof, nt, sep_off);
+  key_add(key, g_ctx.L, sizeof g_ctx.L);
+  key_add(key, ms.data(), ms.size() * sizeof(int));
   // the tables and the shared workspace are this call's until the stream is
   // synchronised below
   std::unique_lock<std::mutex> wl(g_ws_mu);
@@ -2040,7 +2093,7 @@ int plg_ft_apply(const void *field, int precision, int dof, int nt, const int *m
   g.cos_tab = g_ctx.d_cos;
   g.sin_tab = g_ctx.d_sin;
   int rc = PLG_OK;
-  if (F.key != key.str()) {
+  if (F.key != key) {
     F.release();
     std::vector<int> pair_ms, mom_pair;
     F.npairs = make_pairs(ms, g_ctx.M, pair_ms, mom_pair, &F.zero_pair);
@@ -2050,7 +2103,7 @@ int plg_ft_apply(const void *field, int precision, int dof, int nt, const int *m
     if (!rc) rc = upload(&F.d_pair_ms, pair_ms, st);
     if (!rc) rc = upload(&F.d_mom_pair, mom_pair, st);
     if (!rc && F.sh.ok) rc = upload(&F.d_sep, F.sh.blob, st);
-    F.key = key.str();
+    F.key = key;
   }
   const int npairs = F.npairs, zero_pair = F.zero_pair;
   const SepHost &sh = F.sh;
