@@ -345,12 +345,19 @@ struct SepGeom {
   const int *xs;           // [NAP][2]: residue slot of +a and of -a (or -1)
   const int *slot;         // [NXR][NBP][2]: pair index of (n_x, +b) and (n_x, -b), or -1
   const int *sl_m, *sl_rz; // [NS][NZP]: momentum index (or -1) and n_z residue of a pair's momenta
+  // matrix form (mm): NF functions f(x) and NG functions g(y), the cosines
+  // and sines of the classes a and b
+  int mm, NF, NG;
+  const double *pha;       // [step][64]: f_i of the site a lane holds, row i = lane % 16 (rows >= NF zero)
+  const double *ph2f;      // [Ly][5, 7 or 9]: g_j(y)
+  const int *slq;          // [NS][6]: cos and sin function of n_x (-1: none), sign of n_x, the same of n_y
 };
 // host description of a plan's separable projection
 struct SepHost {
   bool ok = false;
   SepGeom g{};                     // scalars (pointers set by sep_geom)
   std::vector<unsigned char> blob;  // the device tables, uploaded as one piece
+  size_t off_pha = 0, off_ph2f = 0, off_slq = 0;
   size_t off_ph1 = 0, off_ph1p = 0, off_ph2 = 0, off_ph3 = 0, off_xs = 0, off_slot = 0, off_slm = 0,
          off_slrz = 0;
 };
