@@ -26,7 +26,7 @@
 //            written.
 //            Where a line is whole groups of 4 sites and the momenta are few,
 //            k_sep_xy_mm does the same without the LDS (below).
-//  k_sep_z   thread = column, workgroup row = (n_x, n_y) pair: the sums over
+//  k_sep_z   lane = column, workgroup row = (n_x, n_y) pair: the sums over
 //            z of the pair's momenta, written momentum-major for the
 //            finalize kernel.
 //
@@ -346,19 +346,26 @@ __global__ __launch_bounds__(256, 3) void k_sep_xy_mm(SepGeom s, const cx<T> *__
     }
 }
 
+// A workgroup holds 64 columns, its four waves every fourth plane each: with
+// a thread per column and all its planes a call of 1024 columns had 784 waves
+// on the chip, each a serial chain of loads: 15 -> 9 us.
 template <int MAXZ>
 __global__ __launch_bounds__(256) void k_sep_z(SepGeom s, const cx<double> *__restrict__ H,
                                                cx<double> *__restrict__ part) {
-  const int64_t col = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  __shared__ cx<double> sum[MAXZ][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t col = (int64_t)blockIdx.x * 64 + lane;
   const int sl = blockIdx.y;
-  if (col >= s.ncols) return;
+  const bool in = col < s.ncols;
+  const cx<double> *Hc = H + (int64_t)sl * s.ncols + (in ? col : s.ncols - 1);
   // the pair's momenta, padded to MAXZ (padding: n_z residue 0, momentum -1)
   const int *rz = s.sl_rz + sl * MAXZ, *mm = s.sl_m + sl * MAXZ;
   cx<double> acc[MAXZ];
 #pragma unroll
   for (int j = 0; j < MAXZ; j++) acc[j] = cmake<double>(0, 0);
-  for (int z = 0; z < s.Lz; z++) {
-    const cx<double> h = gload(H + ((int64_t)z * s.NS + sl) * s.ncols + col);
+#pragma unroll 2
+  for (int z = wave; z < s.Lz; z += 4) {
+    const cx<double> h = gload(Hc + (int64_t)z * s.NS * s.ncols);
 #pragma unroll
     for (int j = 0; j < MAXZ; j++) {  // (cos - i sin) h
       const cx<double> ph = s.ph3[rz[j] * s.Lz + z];
@@ -368,9 +375,16 @@ __global__ __launch_bounds__(256) void k_sep_z(SepGeom s, const cx<double> *__re
       acc[j].im -= ph.im * h.re;
     }
   }
+  for (int w = 3; w > 0; w--) {
+    if (wave == w)
 #pragma unroll
-  for (int j = 0; j < MAXZ; j++)
-    if (mm[j] >= 0) gstore(part + (int64_t)mm[j] * s.ncols + col, acc[j]);
+      for (int j = 0; j < MAXZ; j++) sum[j][lane] = w == 3 ? acc[j] : sum[j][lane] + acc[j];
+    __syncthreads();
+  }
+  if (wave == 0 && in)
+#pragma unroll
+    for (int j = 0; j < MAXZ; j++)
+      if (mm[j] >= 0) gstore(part + (int64_t)mm[j] * s.ncols + col, acc[j] + sum[j][lane]);
 }
 
 // ------------------------------------------------------------------ host
@@ -631,7 +645,7 @@ int launch_project_sep(const SepGeom &g, const void *c, int c_prec, double *part
     rc = g.small ? launch_xy<float, 5, 5>(g, (const cx<float> *)c, H, st)
                  : launch_xy<float, 8, 8>(g, (const cx<float> *)c, H, st);
   if (rc) return rc;
-  dim3 block(256), grid((unsigned)((g.ncols + 255) / 256), (unsigned)g.NS);
+  dim3 block(256), grid((unsigned)((g.ncols + 63) / 64), (unsigned)g.NS);
   if (g.small) k_sep_z<9><<<grid, block, 0, st>>>(g, H, P);
   else k_sep_z<16><<<grid, block, 0, st>>>(g, H, P);
   return hipGetLastError() == hipSuccess ? PLG_OK : PLG_ERR_HIP;
