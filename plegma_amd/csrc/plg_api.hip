@@ -184,7 +184,7 @@ static int kind_shape(int kind, int mask, int &ng, int &nd, int &nch) {
 
 // ------------------------------------------------------------------ plans
 struct Launch {
-  enum { MESON, BARYON, MESMES, UDSC, TETRA, UDSC_ALL } what;
+  enum { MESON, BARYON, MESMES, UDSC, TETRA, TETRA_TERMS, UDSC_ALL } what;
   int set;          // meson set
   bool two, mes;    // baryon
   int gmask;
@@ -237,6 +237,7 @@ struct Plan {
   UdscAll udsc_all{};
   // four-propagator tables (device arrays kept by the caller of the plan)
   std::vector<TetraSched> tetra;
+  std::vector<TetraTermsSched> tetra_terms;
   // batch-owned workspace (single calls use the context workspace)
   void *c = nullptr, *part = nullptr;
   size_t c_bytes = 0, part_bytes = 0;
@@ -672,7 +673,7 @@ static std::string launch_name(const Plan &P, const Launch &l) {
   if (l.what == Launch::MESON) return "contract_mesons_" + t;
   if (l.what == Launch::MESMES) return "contract_mesmes_" + t;
   if (l.what == Launch::UDSC || l.what == Launch::UDSC_ALL) return "contract_udsc_" + t;
-  if (l.what == Launch::TETRA) return "contract_tetra_" + t;
+  if (l.what == Launch::TETRA || l.what == Launch::TETRA_TERMS) return "contract_tetra_" + t;
   return std::string(l.mes ? "contract_twopt_" : "contract_baryons_") + t;
 }
 
@@ -691,6 +692,9 @@ template <typename T> static int launch_contract_t(const Plan &P, const Launch &
     return launch_udsc_all<T>(P.udsc_all, pd, P.d_rows, nrows, (cx<T> *)c, g_ctx.V3, g_ctx.L[3], P.nch_c, st);
   case Launch::TETRA:
     return launch_tetra<T>(P.tetra[l.set], pd, P.d_rows, nrows, (cx<T> *)c, g_ctx.V3, g_ctx.L[3], P.nch_c, l.ch0, st);
+  case Launch::TETRA_TERMS:
+    return launch_tetra_terms<T>(P.tetra_terms[l.set], pd, P.d_rows, nrows, (cx<T> *)c, g_ctx.V3, g_ctx.L[3], P.nch_c,
+                                 P.tpb, st);
   default:
     return launch_baryon<T>(l.two, l.mes, l.gmask, pd, P.d_rows, nrows, (cx<T> *)c, g_ctx.V3, g_ctx.L[3],
                             P.nch_c, l.ch0, P.tpb, st);
@@ -1659,6 +1663,7 @@ static int udsc_run(const plg_prop *up, const plg_prop *dn, const plg_prop *st, 
 // table by its number) and by the precision.  A table whose device arrays are large is not kept.
 struct TetraTable {
   std::vector<TetraSched> s;  // one per launch
+  std::vector<TetraTermsSched> terms;  // or, term by term, one per set
   std::vector<void *> mem;
   ~TetraTable() {
     for (void *p : mem) hipFree(p);
@@ -1714,7 +1719,8 @@ static int tetra_pack_cached(const int16_t *idxs, const int16_t *cols, const flo
   }
   std::vector<TetraPacked> pk;
   const int per = T == PLG_F64 ? TT_OPS<double> : TT_OPS<float>;
-  int rc = tetra_pack(idxs, cols, vals, counts, nops, per, pk);
+  bool by_terms = false;
+  int rc = tetra_pack(idxs, cols, vals, counts, nops, per, pk, by_terms);
   if (rc) return rc;
   auto tab = std::make_shared<TetraTable>();
   size_t bytes = 0;
@@ -1726,6 +1732,27 @@ static int tetra_pack_cached(const int16_t *idxs, const int16_t *cols, const flo
     *d = p;
     return r;
   };
+  if (by_terms) {
+    pk.clear();
+    TetraTermsPacked tp;
+    if ((rc = tetra_pack_terms(idxs, cols, vals, counts, nops, tp))) return rc;
+    const void *coef = nullptr;
+    if ((rc = put(tp.coef, &coef))) return rc;
+    for (int h = 0; h < (tp.terms[1].empty() ? 1 : 2); h++) {
+      TetraTermsSched S{};
+      S.nops = nops;
+      S.ncoef = (int)tp.coef.size() / 2;
+      S.set = h;
+      for (int k = 0; k < nops; k++) {
+        S.first[k] = tp.first[h][k];
+        S.count[k] = tp.count[h][k];
+        S.ndirect[k] = tp.ndirect[h][k];
+      }
+      if ((rc = put(tp.terms[h], (const void **)&S.terms))) return rc;
+      S.coef = (const float *)coef;
+      tab->terms.push_back(S);
+    }
+  }
   for (TetraPacked &k : pk) {
     if ((rc = put(k.words, (const void **)&k.s.words))) return rc;
     if (T == PLG_F64) rc = put(k.coef, &k.s.coef);
@@ -1808,7 +1835,11 @@ static int tetra_run(const plg_prop *const views[4], const int16_t *idxs, const 
   P.tetra = tab->s;
   for (int i = 0, k = 0; i < (int)P.tetra.size(); k += P.tetra[i++].nops)
     P.launches.push_back({Launch::TETRA, i, false, false, 0, k});
+  P.tetra_terms = tab->terms;
+  for (int i = 0; i < (int)P.tetra_terms.size(); i++)
+    P.launches.push_back({Launch::TETRA_TERMS, i, false, false, 0, 0});
   choose_tiles(P);
+  P.tpb = 64;  // sites per workgroup, term by term
   return plan_run(P, out, out_precision, (hipStream_t)stream, nullptr);
 }
 

@@ -160,14 +160,42 @@ struct TetraSched {
 template <typename T> constexpr int TT_OPS = sizeof(T) == 4 ? TETRA_MAXOPS : 32;
 struct TetraPacked {
   TetraSched s{};
+  int64_t cost = 0;  // FMAs of a lane per 16 sites, a matrix instruction counted as 13
   std::vector<uint32_t> words;
   std::vector<double> coef;
 };
+// by_terms: the table is better contracted term by term
 int tetra_pack(const int16_t *idxs, const int16_t *cols, const float *vals, const int16_t *counts, int nops, int per,
-               std::vector<TetraPacked> &out);
+               std::vector<TetraPacked> &out, bool &by_terms);
 template <typename T>
 int launch_tetra(const TetraSched &S, const PropDev<T> *props, const RowDev *rows, int nrows, cx<T> *out,
                  int64_t V3, int T_lat, int nch_total, int ch0, hipStream_t st);
+
+// The same tables term by term, for tables whose terms share little.
+// A term, 32 bits: the (P1, P3) spin pair p = 16 s1 + s3 (bits 0-7), the
+// (P2, P4) pair q = 16 s2 + s4 (bits 8-15) and the coefficient index (bits
+// 16-31).  An operator's terms are its direct ones first, then its crossed
+// ones; set 1 is packed for the views P1, P2, P4, P3, and its launch adds to
+// set 0's.
+typedef uint32_t TetraTerm;
+struct TetraTermsSched {
+  int nops;
+  int first[TETRA_MAXOPS], count[TETRA_MAXOPS], ndirect[TETRA_MAXOPS];
+  const TetraTerm *terms;
+  const float *coef;  // re, im of each distinct coefficient
+  int ncoef;
+  int set;
+};
+struct TetraTermsPacked {
+  std::vector<TetraTerm> terms[2];
+  std::vector<int> first[2], count[2], ndirect[2];
+  std::vector<float> coef;  // shared by both sets
+};
+int tetra_pack_terms(const int16_t *idxs, const int16_t *cols, const float *vals, const int16_t *counts, int nops,
+                     TetraTermsPacked &out);
+template <typename T>
+int launch_tetra_terms(const TetraTermsSched &S, const PropDev<T> *props, const RowDev *rows, int nrows, cx<T> *out,
+                       int64_t V3, int T_lat, int nch_total, int spw, hipStream_t st);
 int udsc_products();
 const char *udsc_flavours(int prod);
 int udsc_nops(int prod);

@@ -348,6 +348,7 @@ static void tetra_walk(const std::vector<TetraProd> &prods, const std::vector<in
           for (int ty = 0; ty < 2; ty++) ng[ty] = std::max(ng[ty], st->it[j]->g[ty].size());
         }
       out.words.push_back(pw);
+      out.cost += 108 + 108 * (int64_t)ng[0] + 36 * (int64_t)ng[1];
       out.words.push_back((uint32_t)ng[0] | (uint32_t)ng[1] << 8 | (uint32_t)st->set << 16);
       for (int ty = 0; ty < 2; ty++)
         for (size_t g = 0; g < ng[ty]; g++) {
@@ -380,6 +381,7 @@ static void tetra_walk(const std::vector<TetraProd> &prods, const std::vector<in
                   out.coef.insert(out.coef.end(), V[h][b], V[h][b] + 64);
                 }
             out.words.push_back(uw);
+            out.cost += 36 + 26 * __builtin_popcount(uw >> 16);
           }
         }
     }
@@ -392,12 +394,13 @@ static void tetra_walk(const std::vector<TetraProd> &prods, const std::vector<in
 // host: classify the terms of a table (reference format) and lay out the
 // walks, one per `per` operators
 int tetra_pack(const int16_t *idxs, const int16_t *cols, const float *vals, const int16_t *counts, int nops, int per,
-               std::vector<TetraPacked> &out) {
+               std::vector<TetraPacked> &out, bool &by_terms) {
   if (nops <= 0 || nops > TETRA_MAXOPS) return PLG_ERR_UNSUPPORTED;
   std::map<std::pair<uint32_t, uint32_t>, int> cidx;  // distinct coefficients, zero among them
   cidx.emplace(std::make_pair(0u, 0u), 0);
   std::vector<TetraProd> prods;
   std::vector<int> index(1 << 18, -1);
+  int64_t ndirect = 0;
   size_t t = 0;
   for (int k = 0; k < nops; k++) {
     if (counts[k] < 0) return PLG_ERR_INVALID;
@@ -425,6 +428,7 @@ int tetra_pack(const int16_t *idxs, const int16_t *cols, const float *vals, cons
       else if (c[0] == c[7] && c[1] == c[6] && c[2] == c[5] && c[3] == c[4]) key = 3 << 16 | u1;
       else if (c[0] == c[7] && c[1] == c[4] && c[2] == c[5] && c[3] == c[6]) key = 2 << 16 | u1;
       else return PLG_ERR_UNSUPPORTED;
+      ndirect += key >> 16 & 1;
       if (index[key] < 0) {
         index[key] = (int)prods.size();
         prods.emplace_back();
@@ -440,6 +444,15 @@ int tetra_pack(const int16_t *idxs, const int16_t *cols, const float *vals, cons
     out.emplace_back();
     tetra_walk(prods, index, k0, std::min(per, nops - k0), out.back());
   }
+  // The walk against the terms one by one (plg_tetra_terms.hip), in ns per
+  // site of a full chip: the walk 0.116 per unit of its cost (the udbb table
+  // 12.8, 110 k units), the terms 4 per thousand crossed and 1 per thousand
+  // direct ones and 5 for their spin-pair tables (udbb 37; 12.3 k random terms
+  // with complex coefficients 37, by the walk 42).  Ties go to the walk.
+  int64_t cost = 0;
+  for (const TetraPacked &P : out) cost += P.cost;
+  const double walk = 0.116e-3 * (double)cost, terms = 5 + 4e-3 * (double)((int64_t)t - ndirect) + 1e-3 * (double)ndirect;
+  by_terms = walk > terms;
   return PLG_OK;
 }
 

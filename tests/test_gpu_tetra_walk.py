@@ -1,6 +1,7 @@
-"""Four-propagator tables (k_tetra): edges of its 16-site tiles, of its blocks
-of 16 operators (FP64 takes 32 per launch) and of its walk -- operators
-without terms, duplicate terms, one term, every spin quad -- against the CPU
+"""Four-propagator tables: edges of the walk's 16-site tiles (k_tetra), of its
+blocks of 16 operators (FP64 takes 32 per launch) and of its steps --
+operators without terms, duplicate terms, one term, every spin quad -- and
+large irregular tables, which go term by term (k_tetra_terms), against the CPU
 oracle.  Tolerances: FP64 1e-12 normwise, mixed 1e-6 (the paths' bounds)."""
 import numpy as np
 import pytest
@@ -17,7 +18,8 @@ PATTERNS = [(0, 2, 1, 3, 2, 0, 3, 1), (0, 3, 1, 2, 3, 0, 2, 1), (0, 2, 1, 3, 3, 
 COEFS = [1, -1, 2, 1j, -0.5, 0.25 + 0.5j]
 # lattice, operators, terms of an operator, real coefficients only
 CASES = [([2, 2, 2, 4], 1, 1, True), ([3, 3, 3, 4], 16, 30, True), ([17, 1, 1, 4], 17, 12, False),
-         ([4, 4, 1, 4], 33, 9, False), ([5, 3, 3, 4], 64, 8, False), ([3, 3, 3, 4], 3, 900, False)]
+         ([4, 4, 1, 4], 33, 9, False), ([5, 3, 3, 4], 64, 8, False), ([3, 3, 3, 4], 3, 900, False),
+         ([3, 3, 3, 4], 7, 1500, False), ([5, 1, 1, 4], 16, 700, False)]  # these term by term
 
 
 @pytest.mark.parametrize("case", range(len(CASES)))
