@@ -1595,6 +1595,9 @@ static int udsc_run(const plg_prop *up, const plg_prop *dn, const plg_prop *st, 
       }
   UdscAll S;
   const int prec = mode == PLG_MODE_F64 ? PLG_F64 : PLG_F32;
+  for (int j = 0; j < lt; j++)
+    for (const plg_prop &v : props)
+      if ((rc = check_prop(v, prec, row_time(g_ctx.L, source, w, j)))) return rc;
   if ((rc = udsc_device_schedule(prods, fidx, (int)props.size(), prec, S))) return rc;
   // The products of a call share one launch; the site correlator holds all
   // their operators, so the time slices are taken in pieces that keep it
@@ -1602,9 +1605,10 @@ static int udsc_run(const plg_prop *up, const plg_prop *dn, const plg_prop *st, 
   const int64_t row_bytes = (int64_t)nd_total * ctile_sites(V3) * (prec == PLG_F64 ? 16 : 8);
   int64_t per = std::max<int64_t>((int64_t)1 << 30, row_bytes / nd_total * 16 * lt) / row_bytes;
   per = std::max<int64_t>(1, std::min<int64_t>({per, lt, 32768 / nd_total}));
-  const int npiece = (int)((lt + per - 1) / per);
-  for (int ip = 0; ip < npiece; ip++) {
-    const int j0 = lt * ip / npiece, j1 = lt * (ip + 1) / npiece;
+  const int64_t npiece = (lt + per - 1) / per;
+  per = (lt + npiece - 1) / npiece;
+  for (int j0 = 0, j1; j0 < lt;) {
+    j1 = (int)std::min<int64_t>(lt, j0 + per);
     Plan P;
     P.kind = -1;
     P.mode = mode;
@@ -1617,12 +1621,7 @@ static int udsc_run(const plg_prop *up, const plg_prop *dn, const plg_prop *st, 
     P.ms = scaled_moms(P.moms.data(), P.nmom, 1);
     if (P.nmom > 0) P.npairs = make_pairs(P.ms, g_ctx.M, P.pair_ms, P.mom_pair, &P.zero_pair);
     P.nch_c = nd_total;
-    for (int j = j0; j < j1; j++) {
-      const int t = row_time(g_ctx.L, source, w, j);
-      for (const plg_prop &v : P.props)
-        if ((rc = check_prop(v, P.T, t))) return rc;
-      P.rows.push_back({t, 0, 0, 0, 0});
-    }
+    for (int j = j0; j < j1; j++) P.rows.push_back({row_time(g_ctx.L, source, w, j), 0, 0, 0, 0});
     int d0 = 0;
     for (int prod : prods) {
       const char *f = udsc_flavours(prod);
@@ -1652,7 +1651,14 @@ static int udsc_run(const plg_prop *up, const plg_prop *dn, const plg_prop *st, 
     P.launches.push_back({Launch::UDSC_ALL, 0, false, false, 0, 0});
     P.udsc_all = S;
     choose_tiles(P);
-    if ((rc = plan_run(P, out, out_precision, (hipStream_t)stream, stage_ms))) return rc;
+    rc = plan_run(P, out, out_precision, (hipStream_t)stream, stage_ms);
+    if (rc == PLG_ERR_ALLOC && per > 1) {  // nothing was launched: fewer slices at a time
+      (void)hipGetLastError();
+      per = (per + 1) / 2;
+      continue;
+    }
+    if (rc) return rc;
+    j0 = j1;
   }
   return PLG_OK;
 }

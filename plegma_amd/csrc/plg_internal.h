@@ -66,7 +66,7 @@ __device__ __forceinline__ double row_scale(const OutRowDev &R) {
   return ldexp(1.0, e);
 }
 
-// udsc baryons: chunked schedule of one flavour product's term tables.
+// three-propagator tables: chunked schedule of a caller's table.
 // Chunk c holds up to 64 (m0m1, m2m3) quads, one per lane; lane l's quad has
 // up to UD_TPQ distinct terms, kept in the chunk-local slots e*64 + l.
 // Operator k owns the lanes [op_lo[k], op_lo[k] + op_n[k]) (all 64 lanes are
