@@ -1724,9 +1724,8 @@ static int tetra_pack_cached(const int16_t *idxs, const int16_t *cols, const flo
       }
   }
   std::vector<TetraPacked> pk;
-  const int per = T == PLG_F64 ? TT_OPS<double> : TT_OPS<float>;
   bool by_terms = false;
-  int rc = tetra_pack(idxs, cols, vals, counts, nops, per, pk, by_terms);
+  int rc = tetra_pack(idxs, cols, vals, counts, nops, TT_OPS, pk, by_terms);
   if (rc) return rc;
   auto tab = std::make_shared<TetraTable>();
   size_t bytes = 0;

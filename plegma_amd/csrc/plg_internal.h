@@ -155,9 +155,9 @@ struct TetraSched {
   const uint32_t *words;
   const void *coef;  // in the precision of the contraction
 };
-// operators of one launch: all in FP32; in FP64 the sums of more than two
-// blocks of 16 do not fit the registers beside the products
-template <typename T> constexpr int TT_OPS = sizeof(T) == 4 ? TETRA_MAXOPS : 32;
+// operators of one launch: the sums of more than two blocks of 16, in two
+// levels, do not fit the registers beside the products
+constexpr int TT_OPS = 32;
 struct TetraPacked {
   TetraSched s{};
   int64_t cost = 0;  // FMAs of a lane per 16 sites, a matrix instruction counted as 13

@@ -110,9 +110,21 @@ __global__ __launch_bounds__(64 * TT_WAVES, sizeof(T) == 4 ? 4 : 2) void k_tetra
     }
     __syncthreads();
   }
-  v4 ar[NB], ai[NB];
+  // the sums, and those of the last few products: sums of sums round less
+  // than one long sum
+  v4 tr[NB], ti[NB], ar[NB], ai[NB];
+  int nsum = 0;
 #pragma unroll
-  for (int b = 0; b < NB; b++) ar[b] = ai[b] = (v4)(T)0;
+  for (int b = 0; b < NB; b++) tr[b] = ti[b] = ar[b] = ai[b] = (v4)(T)0;
+  auto flush = [&]() {
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+      tr[b] += ar[b];
+      ti[b] += ai[b];
+      ar[b] = ai[b] = (v4)(T)0;
+    }
+    nsum = 0;
+  };
   // the wave's words, 64 at a time and the next 64 on the way
   const uint32_t *wp = S.words + S.word0[wave] + lane;
   uint32_t wcur = wp[0], wnext = wp[64];
@@ -206,8 +218,11 @@ __global__ __launch_bounds__(64 * TT_WAVES, sizeof(T) == 4 ? 4 : 2) void k_tetra
             }
         }
       }
+      nsum += nt;
+      if (nsum >= 6) flush();
     }
   }
+  flush();
   // the waves' sums
   const int64_t ncols = (int64_t)gridDim.y * nch_total, col0 = (int64_t)blockIdx.y * nch_total + ch0;
 #pragma unroll
@@ -216,13 +231,17 @@ __global__ __launch_bounds__(64 * TT_WAVES, sizeof(T) == 4 ? 4 : 2) void k_tetra
 #pragma unroll
     for (int h = 0; h < 2; h++) {
 #pragma unroll
-      for (int r = 0; r < 4; r++) red[wave][r * 64 + lane] = h ? ai[b][r] : ar[b][r];
+      for (int r = 0; r < 4; r++) red[wave][r * 64 + lane] = h ? ti[b][r] : tr[b][r];
       __syncthreads();
       if (tid < 256) {
-        T v = red[0][tid];
+        T v[TT_WAVES];
 #pragma unroll
-        for (int w = 1; w < TT_WAVES; w++) v += red[w][tid];
-        o[h] = v;
+        for (int w = 0; w < TT_WAVES; w++) v[w] = red[w][tid];
+#pragma unroll
+        for (int n = TT_WAVES / 2; n > 0; n /= 2)  // pairwise
+#pragma unroll
+          for (int w = 0; w < n; w++) v[w] += v[w + n];
+        o[h] = v[0];
       }
       __syncthreads();
     }
@@ -239,14 +258,6 @@ int launch_tetra(const TetraSched &S, const PropDev<T> *props, const RowDev *row
   switch ((S.nops + 15) / 16) {
   case 1: k_tetra<T, 1><<<grid, block, 0, st>>>(S, props, rows, out, V3, T_lat, nch_total, ch0); break;
   case 2: k_tetra<T, 2><<<grid, block, 0, st>>>(S, props, rows, out, V3, T_lat, nch_total, ch0); break;
-  case 3:
-    if constexpr (TT_OPS<T> > 32) k_tetra<T, 3><<<grid, block, 0, st>>>(S, props, rows, out, V3, T_lat, nch_total, ch0);
-    else return PLG_ERR_UNSUPPORTED;
-    break;
-  case 4:
-    if constexpr (TT_OPS<T> > 48) k_tetra<T, 4><<<grid, block, 0, st>>>(S, props, rows, out, V3, T_lat, nch_total, ch0);
-    else return PLG_ERR_UNSUPPORTED;
-    break;
   default: return PLG_ERR_UNSUPPORTED;
   }
   return hipGetLastError() == hipSuccess ? PLG_OK : PLG_ERR_HIP;

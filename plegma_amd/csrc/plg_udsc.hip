@@ -682,6 +682,7 @@ __global__ __launch_bounds__(64 * UD_WAVES, sizeof(T) == 4 ? 4 : 2) void k_udsc_
           const uint64_t pw = (uint64_t)S.units[2 * un] | (uint64_t)S.units[2 * un + 1] << 32;
           const int pl = (int)(pw >> (16 * kq)) & 0xffff;
           const v4 cn = coef[(un + 1) * 64];  // the next unit's
+          v4 ur = (v4)(T)0, ui = (v4)(T)0;    // the unit's sums: sums of sums round less than one long sum
 #pragma unroll
           for (int e = 0; e < 4; e++) {
             if (e0 + e >= nt) break;
@@ -689,9 +690,11 @@ __global__ __launch_bounds__(64 * UD_WAVES, sizeof(T) == 4 ? 4 : 2) void k_udsc_
             cx<T> t = cmake<T>(0, 0);
 #pragma unroll
             for (int c = 0; c < 9; c++) cfma(t, d[c], Cp[c * 16]);
-            ar[j] = UdAcc<T>::mma(cf[e], t.re, ar[j]);
-            ai[j] = UdAcc<T>::mma(cf[e], t.im, ai[j]);
+            ur = UdAcc<T>::mma(cf[e], t.re, ur);
+            ui = UdAcc<T>::mma(cf[e], t.im, ui);
           }
+          ar[j] += ur;
+          ai[j] += ui;
           cf = cn;
         }
       }
@@ -708,10 +711,14 @@ __global__ __launch_bounds__(64 * UD_WAVES, sizeof(T) == 4 ? 4 : 2) void k_udsc_
         for (int r = 0; r < 4; r++) red[wave][r * 64 + lane] = h ? ai[j][r] : ar[j][r];
         __syncthreads();
         if (tid < 256) {
-          T v = red[0][tid];
+          T v[UD_WAVES];
 #pragma unroll
-          for (int w = 1; w < UD_WAVES; w++) v += red[w][tid];
-          o[h] = v;
+        for (int w = 0; w < UD_WAVES; w++) v[w] = red[w][tid];
+#pragma unroll
+        for (int n = UD_WAVES / 2; n > 0; n /= 2)  // pairwise
+#pragma unroll
+          for (int w = 0; w < n; w++) v[w] += v[w + n];
+        o[h] = v[0];
         }
         __syncthreads();
       }

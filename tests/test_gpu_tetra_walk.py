@@ -1,5 +1,5 @@
 """Four-propagator tables: edges of the walk's 16-site tiles (k_tetra), of its
-blocks of 16 operators (FP64 takes 32 per launch) and of its steps --
+blocks of 16 operators (32 per launch) and of its steps --
 operators without terms, duplicate terms, one term, every spin quad -- and
 large irregular tables, which go term by term (k_tetra_terms), against the CPU
 oracle.  Tolerances: FP64 1e-12 normwise, mixed 1e-6 (the paths' bounds)."""
