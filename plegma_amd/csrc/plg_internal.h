@@ -120,7 +120,7 @@ constexpr int UD_MAXGROUPS = 6;   // uu, dd, ss, cc, ud, sc
 struct UdscGroup {
   int pa, pb, nprod;
   int third[UD_NJ], nops[UD_NJ], ch0[UD_NJ];
-  int step0[UD_WAVES], nsteps[UD_WAVES], unit0[UD_WAVES];
+  int step0[UD_WAVES], nsteps[UD_WAVES], npair[UD_WAVES], unit0[UD_WAVES], coef0[UD_WAVES];
 };
 struct UdscAll {
   int ngroups, nprops;

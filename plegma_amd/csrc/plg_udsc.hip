@@ -263,75 +263,132 @@ int udsc_groups(const std::vector<int> &prods, const int fidx[4], UdscAllHost &h
         for (auto e = T.begin(); e != T.end();)
           e = std::all_of(e->second.begin(), e->second.end(), [](double v) { return v == 0; }) ? T.erase(e)
                                                                                               : std::next(e);
-    // steps of four quads with like term counts, most terms first
+    // the spin pairs of the third propagator a quad has terms with, per product
     typedef std::pair<const int, std::array<Terms, UD_NJ>> Quad;
-    std::vector<const Quad *> order;
-    for (const Quad &q : quads) order.push_back(&q);
-    auto nterms = [](const Quad *q) {
-      size_t n = 0;
-      for (auto &T : q->second) n += T.size();
+    struct Item {  // the quads of a quarter of a step: one, or two that share reads of the third propagator
+      const Quad *q[2];
+      std::array<uint32_t, UD_NJ> set;
+      int n;
+    };
+    auto sets = [](const Quad &q) {
+      std::array<uint32_t, UD_NJ> m{};
+      for (int j = 0; j < UD_NJ; j++)
+        for (auto &e : q.second[j]) m[j] |= 1u << e.first;
+      return m;
+    };
+    auto count = [](const std::array<uint32_t, UD_NJ> &m) {
+      int n = 0;
+      for (uint32_t v : m) n += __builtin_popcount(v);
       return n;
     };
-    std::stable_sort(order.begin(), order.end(), [&](const Quad *a, const Quad *b) {
-      const size_t na = nterms(a), nb = nterms(b);
-      if (na != nb) return na > nb;
-      for (int j = 0; j < UD_NJ; j++)
-        if (a->second[j].size() != b->second[j].size()) return a->second[j].size() > b->second[j].size();
-      return false;
-    });
-    const int nsteps = ((int)order.size() + 3) / 4;
-    auto step_count = [&](int st, int j) {
-      size_t n = 0;
-      for (int i = 4 * st; i < std::min(4 * st + 4, (int)order.size()); i++) n = std::max(n, order[i]->second[j].size());
-      return (int)n;
+    std::vector<Item> single, pairs;
+    for (const Quad &q : quads) {
+      const auto m = sets(q);
+      single.push_back({{&q, nullptr}, m, count(m)});
+    }
+    auto more = [](const Item &x, const Item &y) { return x.n != y.n ? x.n > y.n : x.set > y.set; };
+    std::stable_sort(single.begin(), single.end(), more);
+    // as many steps of two as leave the waves even: whole rounds of the
+    // waves, then two quads per quarter where the rest exceeds one round
+    const int half = ((int)single.size() + 3) / 4, rest = half % (2 * UD_WAVES);
+    const size_t npairs = 4 * (size_t)((half - rest) / 2 + (rest > UD_WAVES ? rest / 2 : 0));
+    while (pairs.size() < npairs && single.size() > 1) {
+      // the quad with most terms and the one that shares most of its spin pairs
+      size_t best = 1;
+      int bw = 1 << 30;
+      for (size_t i = 1; i < single.size(); i++) {
+        std::array<uint32_t, UD_NJ> u;
+        for (int j = 0; j < UD_NJ; j++) u[j] = single[0].set[j] | single[i].set[j];
+        const int waste = 2 * count(u) - single[0].n - single[i].n;
+        if (waste < bw) {
+          bw = waste;
+          best = i;
+        }
+      }
+      Item P = single[0];
+      P.q[1] = single[best].q[0];
+      for (int j = 0; j < UD_NJ; j++) P.set[j] |= single[best].set[j];
+      P.n = count(P.set);
+      pairs.push_back(P);
+      single.erase(single.begin() + best);
+      single.erase(single.begin());
+    }
+    std::stable_sort(pairs.begin(), pairs.end(), more);
+    // steps of four items, to the wave with the least work so far
+    struct Step {
+      const Item *it[4];
+      int cnt[UD_NJ];
+      int cost;
+      bool two;
     };
-    // the steps go to the wave with the least work so far
-    std::vector<std::vector<int>> mine(UD_WAVES);
+    std::vector<Step> steps;
+    for (int two = 1; two >= 0; two--) {
+      const std::vector<Item> &v = two ? pairs : single;
+      for (size_t i = 0; i < v.size(); i += 4) {
+        Step S{};
+        S.two = two;
+        S.cost = two ? 9 : 5;  // a diquark costs four terms, and its loads
+        for (size_t k = 0; k < 4; k++) S.it[k] = i + k < v.size() ? &v[i + k] : nullptr;
+        for (int j = 0; j < UD_NJ; j++) {
+          for (int k = 0; k < 4; k++)
+            if (S.it[k]) S.cnt[j] = std::max(S.cnt[j], __builtin_popcount(S.it[k]->set[j]));
+          S.cost += S.cnt[j] * (two ? 2 : 1);
+        }
+        steps.push_back(S);
+      }
+    }
+    std::vector<std::vector<const Step *>> mine(UD_WAVES);
     int load[UD_WAVES] = {0};
-    for (int st = 0; st < nsteps; st++) {
-      int cost = 5;  // a diquark costs four terms, and its loads
-      for (int j = 0; j < UD_NJ; j++) cost += step_count(st, j);
+    for (const Step &S : steps) {
       const int w = (int)(std::min_element(load, load + UD_WAVES) - load);
-      load[w] += cost;
-      mine[w].push_back(st);
+      load[w] += S.cost;
+      mine[w].push_back(&S);  // steps of two first, as they come
     }
     for (int w = 0; w < UD_WAVES; w++) {
-      G.step0[w] = (int)h.steps.size() / 2;
+      G.step0[w] = (int)h.steps.size() / 3;
       G.nsteps[w] = (int)mine[w].size();
+      G.npair[w] = (int)std::count_if(mine[w].begin(), mine[w].end(), [](const Step *S) { return S->two; });
       G.unit0[w] = (int)h.units.size() / 2;
-      for (int st : mine[w]) {
-        uint32_t qw = 0, cw = 0;
+      G.coef0[w] = (int)h.coef.size() / 256;
+      for (const Step *S : mine[w]) {
+        uint32_t qw[2] = {0, 0}, cw = 0;
         for (int i = 0; i < 4; i++)
-          if (4 * st + i < (int)order.size()) qw |= (uint32_t)order[4 * st + i]->first << (8 * i);
-        for (int j = 0; j < UD_NJ; j++) cw |= (uint32_t)step_count(st, j) << (8 * j);
-        h.steps.push_back(qw);
-        h.steps.push_back(cw);
-        for (int j = 0; j < UD_NJ; j++) {
-          const int n = step_count(st, j);
-          for (int e0 = 0; e0 < n; e0 += 4) {  // a unit: four terms of each of the step's quads
+          for (int b = 0; b < 2; b++)
+            if (S->it[i] && S->it[i]->q[b]) qw[b] |= (uint32_t)S->it[i]->q[b]->first << (8 * i);
+        for (int j = 0; j < UD_NJ; j++) cw |= (uint32_t)S->cnt[j] << (8 * j);
+        h.steps.insert(h.steps.end(), {qw[0], qw[1], cw});
+        for (int j = 0; j < UD_NJ; j++)
+          for (int e0 = 0; e0 < S->cnt[j]; e0 += 4) {  // a unit: four terms of each quarter's quads
             uint64_t pw = 0;
             const size_t c0 = h.coef.size();
-            h.coef.resize(c0 + 256, 0.0);
+            h.coef.resize(c0 + (S->two ? 512 : 256), 0.0);
             for (int i = 0; i < 4; i++) {
-              if (4 * st + i >= (int)order.size()) continue;
-              const Terms &T = order[4 * st + i]->second[j];
-              auto e = T.begin();
-              for (int u = 0; u < e0 && e != T.end(); u++) ++e;
-              for (int u = 0; u < 4 && e != T.end(); u++, ++e) {
-                pw |= (uint64_t)e->first << (16 * i + 4 * u);
-                for (int k = 0; k < UD_MAXOPS; k++) h.coef[c0 + (i * 16 + k) * 4 + u] = e->second[k];
+              if (!S->it[i]) continue;
+              int u = 0;  // the quarter's spin pairs in order
+              for (int sp = 0; sp < 16; sp++) {
+                if (!(S->it[i]->set[j] >> sp & 1)) continue;
+                if (u >= e0 && u < e0 + 4) {
+                  pw |= (uint64_t)sp << (16 * i + 4 * (u - e0));
+                  for (int b = 0; b < 2; b++) {
+                    if (!S->it[i]->q[b]) continue;
+                    auto e = S->it[i]->q[b]->second[j].find(sp);
+                    if (e == S->it[i]->q[b]->second[j].end()) continue;
+                    for (int k = 0; k < UD_MAXOPS; k++)
+                      h.coef[c0 + b * 256 + (i * 16 + k) * 4 + (u - e0)] = e->second[k];
+                  }
+                }
+                u++;
               }
             }
             h.units.push_back((uint32_t)pw);
             h.units.push_back((uint32_t)(pw >> 32));
           }
-        }
       }
     }
   }
   // the kernel loads a wave's next unit ahead of its use
   h.units.resize(h.units.size() + 2, 0u);
-  h.coef.resize(h.coef.size() + 256, 0.0);
+  h.coef.resize(h.coef.size() + 4 * 256, 0.0);
   return PLG_OK;
 }
 
@@ -579,12 +636,15 @@ template int launch_udsc<float>(const UdscSched &, const PropDev<float> *, const
 // operators: O[k][site] += sum_q V[k][term of quad q] T[q][site], for the
 // real and the imaginary part.  The waves share a group's steps and their
 // sums meet in LDS at the group's end.
+// Where the quads pair up, a quarter takes two at a time whose terms have like
+// spin pairs of the third propagator: one read of it serves both.
 // Bound by the vector unit and LDS (a term is 36 FMAs, two matrix instructions
-// and 9 reads; of 9.2 M cycles the FMAs take 4.5 M, the matrix instructions
-// 1.9 M, LDS is busy 5.5 M).  20 products on 24^3 x 16 sites, FP32: 20 launches
-// of k_udsc, 0.5 ms each -> 4.2 ms, the call 14.5 -> 4.4 ms.  k_udsc reads the
-// terms, coefficients and entry indexes of its operator sums and every
-// diquark's blocks from LDS 20 times per site, and is bound there.
+// and 9 reads; one quad at a time the FMAs took 4.5 M of 9.2 M cycles, the
+// matrix instructions 1.9 M, LDS was busy 5.5 M).  20 products on 24^3 x 16
+// sites, FP32, whole calls: 20 launches of k_udsc 14.6 ms, here one quad at a
+// time 4.16 ms, two 3.89 ms.  k_udsc reads the terms, coefficients and entry
+// indexes of its operator sums and every diquark's blocks from LDS 20 times
+// per site, and is bound there.
 template <typename T> struct UdAcc;
 template <> struct UdAcc<float> {
   typedef float v4 __attribute__((ext_vector_type(4)));
@@ -657,48 +717,66 @@ __global__ __launch_bounds__(64 * UD_WAVES, sizeof(T) == 4 ? 4 : 2) void k_udsc_
     for (int j = 0; j < UD_NJ; j++) ar[j] = ai[j] = (v4)(T)0;
     const cx<T> *A = sp + G.pa * 2304 + s, *B = sp + G.pb * 2304 + s;
     const int st0 = G.step0[wave], nst = G.nsteps[wave];
-    int un = G.unit0[wave];
-    v4 cf = coef[un * 64];
-    for (int st = st0; st < st0 + nst; st++) {
-      const uint32_t qw = S.steps[2 * st], cw = S.steps[2 * st + 1];
-      const int q = (qw >> (8 * kq)) & 255;
-      cx<T> d[9];
-      {
+    int un = G.unit0[wave], ci = G.coef0[wave];
+    v4 cf[2] = {coef[ci * 64], coef[(ci + 1) * 64]};
+    // a step: two quads of each quarter (N = 2, the terms' reads of the third
+    // propagator serve both), or one
+    auto step = [&](auto N, int st) {
+      const uint32_t cw = S.steps[3 * st + 2];
+      cx<T> d[N.value][9];
+#pragma unroll
+      for (int b = 0; b < N.value; b++) {
+        const int q = (S.steps[3 * st + b] >> (8 * kq)) & 255;
         const cx<T> *Aq = A + (q & 15) * 144, *Bq = B + (q >> 4) * 144;
-        cx<T> a[9], b[9];
+        cx<T> x[9], y[9];
 #pragma unroll
         for (int j = 0; j < 9; j++) {
-          a[j] = Aq[j * 16];
-          b[j] = Bq[j * 16];
+          x[j] = Aq[j * 16];
+          y[j] = Bq[j * 16];
         }
-        udsc_diquark(a, b, d);
+        udsc_diquark(x, y, d[b]);
       }
 #pragma unroll
       for (int j = 0; j < UD_NJ; j++) {
         const int nt = (cw >> (8 * j)) & 255;
         if (nt == 0) continue;
         const cx<T> *C = sp + G.third[j] * 2304 + s;
-        for (int e0 = 0; e0 < nt; e0 += 4, un++) {
+        for (int e0 = 0; e0 < nt; e0 += 4, un++, ci += N.value) {
           const uint64_t pw = (uint64_t)S.units[2 * un] | (uint64_t)S.units[2 * un + 1] << 32;
           const int pl = (int)(pw >> (16 * kq)) & 0xffff;
-          const v4 cn = coef[(un + 1) * 64];  // the next unit's
+          v4 cn[N.value];  // the next unit's
+#pragma unroll
+          for (int b = 0; b < N.value; b++) cn[b] = coef[(ci + N.value + b) * 64];
           v4 ur = (v4)(T)0, ui = (v4)(T)0;    // the unit's sums: sums of sums round less than one long sum
 #pragma unroll
           for (int e = 0; e < 4; e++) {
             if (e0 + e >= nt) break;
             const cx<T> *Cp = C + ((pl >> (4 * e)) & 15) * 144;
-            cx<T> t = cmake<T>(0, 0);
+            cx<T> t[N.value];
 #pragma unroll
-            for (int c = 0; c < 9; c++) cfma(t, d[c], Cp[c * 16]);
-            ur = UdAcc<T>::mma(cf[e], t.re, ur);
-            ui = UdAcc<T>::mma(cf[e], t.im, ui);
+            for (int b = 0; b < N.value; b++) t[b] = cmake<T>(0, 0);
+#pragma unroll
+            for (int c = 0; c < 9; c++) {
+              const cx<T> v = Cp[c * 16];
+#pragma unroll
+              for (int b = 0; b < N.value; b++) cfma(t[b], d[b][c], v);
+            }
+#pragma unroll
+            for (int b = 0; b < N.value; b++) {
+              ur = UdAcc<T>::mma(cf[b][e], t[b].re, ur);
+              ui = UdAcc<T>::mma(cf[b][e], t[b].im, ui);
+            }
           }
           ar[j] += ur;
           ai[j] += ui;
-          cf = cn;
+#pragma unroll
+          for (int b = 0; b < N.value; b++) cf[b] = cn[b];
         }
       }
-    }
+    };
+    const int mid = st0 + G.npair[wave];
+    for (int st = st0; st < mid; st++) step(std::integral_constant<int, 2>{}, st);
+    for (int st = mid; st < st0 + nst; st++) step(std::integral_constant<int, 1>{}, st);
     // the waves' sums
     const T sgp = prop_sign(props[G.pa], row.t) * prop_sign(props[G.pb], row.t);
 #pragma unroll
