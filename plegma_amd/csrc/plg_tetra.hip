@@ -53,6 +53,7 @@ template <> struct TtAcc<float> {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
   }
   static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane >> 4) + r; }
+  static __device__ __forceinline__ int slot(int k, int s) { return (k & 3) * 64 + (k >> 2) * 16 + s; }  // r * 64 + lane
 };
 template <> struct TtAcc<double> {
   typedef double v4 __attribute__((ext_vector_type(4)));
@@ -60,6 +61,7 @@ template <> struct TtAcc<double> {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
   static __device__ __forceinline__ int row(int lane, int r) { return 4 * r + (lane >> 4); }
+  static __device__ __forceinline__ int slot(int k, int s) { return (k >> 2) * 64 + (k & 3) * 16 + s; }
 };
 
 // NB: blocks of 16 operators
@@ -112,142 +114,209 @@ __global__ __launch_bounds__(64 * TT_WAVES, sizeof(T) == 4 ? 4 : 2) void k_tetra
   }
   // the sums, and those of the last few products: sums of sums round less
   // than one long sum
-  v4 tr[NB], ti[NB], ar[NB], ai[NB];
-  int nsum = 0;
+  v4 tr[NB], ti[NB];
+  // SAFE: values that are not finite stay out of the matrix products, where a
+  // zero coefficient would spread them over the operators of a block, and go
+  // one by one to those that have a coefficient, in spec
+  T *spec = &red[0][0];  // [operator block][real, imaginary][as a wave's sums lie in red]
+  static_assert(2 * NB <= TT_WAVES, "spec fits red");
+  auto walk = [&](auto SAFE) {
+    constexpr bool safe = SAFE.value;
+    v4 ar[NB], ai[NB];
+    int nsum = 0;
 #pragma unroll
-  for (int b = 0; b < NB; b++) tr[b] = ti[b] = ar[b] = ai[b] = (v4)(T)0;
-  auto flush = [&]() {
+    for (int b = 0; b < NB; b++) tr[b] = ti[b] = ar[b] = ai[b] = (v4)(T)0;
+    auto flush = [&]() {
 #pragma unroll
-    for (int b = 0; b < NB; b++) {
-      tr[b] += ar[b];
-      ti[b] += ai[b];
-      ar[b] = ai[b] = (v4)(T)0;
-    }
-    nsum = 0;
-  };
-  // the wave's words, 64 at a time and the next 64 on the way
-  const uint32_t *wp = S.words + S.word0[wave] + lane;
-  uint32_t wcur = wp[0], wnext = wp[64];
-  int wpos = 0;
-  auto word = [&]() -> uint32_t {
-    if (wpos == 64) {
-      wcur = wnext;
-      wp += 64;
-      wnext = wp[64];
-      wpos = 0;
-    }
-    return (uint32_t)__builtin_amdgcn_readlane((int)wcur, wpos++);
-  };
-  const T *cp = (const T *)S.coef + (int64_t)S.coef0[wave] * 64 + lane;
-  T c0 = cp[0], c1 = cp[64];
-  cp += 128;
-  for (int st = 0; st < S.nsteps[wave]; st++) {
-    const uint32_t pw = word(), fw = word();
-    const int p = (pw >> (8 * kq)) & 255;
-    const cx<T> *P3 = sp + ((fw >> 16) & 1 ? 3 : 2) * 2304 + s, *P4 = sp + ((fw >> 16) & 1 ? 2 : 3) * 2304 + s;
-    cx<T> m[9];  // (B3^dag B1)[z][y] at z * 3 + y
-    {
-      const cx<T> *A = sp + s + (p >> 4) * 144, *B = P3 + (p & 15) * 144;
-      cx<T> a[9], b[9];
-#pragma unroll
-      for (int j = 0; j < 9; j++) {
-        a[j] = A[j * 16];
-        b[j] = B[j * 16];
+      for (int b = 0; b < NB; b++) {
+        tr[b] += ar[b];
+        ti[b] += ai[b];
+        ar[b] = ai[b] = (v4)(T)0;
       }
-#pragma unroll
-      for (int z = 0; z < 3; z++)
-#pragma unroll
-        for (int y = 0; y < 3; y++) {
-          m[z * 3 + y] = cmake<T>(0, 0);
-#pragma unroll
-          for (int w = 0; w < 3; w++) cfma_conj(m[z * 3 + y], a[w * 3 + y], b[w * 3 + z]);
-        }
-    }
-    const int ncr = fw & 255, ng = ncr + ((fw >> 8) & 255);
-    for (int g = 0; g < ng; g++) {
-      const uint32_t gw = word();
-      cx<T> X[9];
+      nsum = 0;
+    };
+    // the wave's words, 64 at a time and the next 64 on the way
+    const uint32_t *wp = S.words + S.word0[wave] + lane;
+    uint32_t wcur = wp[0], wnext = wp[64];
+    int wpos = 0;
+    auto word = [&]() -> uint32_t {
+      if (wpos == 64) {
+        wcur = wnext;
+        wp += 64;
+        wnext = wp[64];
+        wpos = 0;
+      }
+      return (uint32_t)__builtin_amdgcn_readlane((int)wcur, wpos++);
+    };
+    const T *cp = (const T *)S.coef + (int64_t)S.coef0[wave] * 64 + lane;
+    T c0 = cp[0], c1 = cp[64];
+    cp += 128;
+    for (int st = 0; st < S.nsteps[wave]; st++) {
+      const uint32_t pw = word(), fw = word();
+      const int p = (pw >> (8 * kq)) & 255;
+      const cx<T> *P3 = sp + ((fw >> 16) & 1 ? 3 : 2) * 2304 + s, *P4 = sp + ((fw >> 16) & 1 ? 2 : 3) * 2304 + s;
+      cx<T> m[9];  // (B3^dag B1)[z][y] at z * 3 + y
       {
-        const cx<T> *B2 = sp + 2304 + s + ((gw >> (4 * kq)) & 15) * 144;
-        cx<T> b[9];
+        const cx<T> *A = sp + s + (p >> 4) * 144, *B = P3 + (p & 15) * 144;
+        cx<T> a[9], b[9];
 #pragma unroll
-        for (int j = 0; j < 9; j++) b[j] = B2[j * 16];
-        if (g < ncr) {
-#pragma unroll
-          for (int w = 0; w < 3; w++)
-#pragma unroll
-            for (int y = 0; y < 3; y++) {
-              X[w * 3 + y] = cmake<T>(0, 0);
-#pragma unroll
-              for (int z = 0; z < 3; z++) cfma(X[w * 3 + y], b[w * 3 + z], m[z * 3 + y]);
-            }
-        } else {
-          const cx<T> d = m[0] + m[4] + m[8];  // <B1, B3>
-#pragma unroll
-          for (int j = 0; j < 9; j++) X[j] = d * b[j];
+        for (int j = 0; j < 9; j++) {
+          a[j] = A[j * 16];
+          b[j] = B[j * 16];
         }
-      }
-      const int nt = (int)(gw >> 16);
-      for (int e = 0; e < nt; e++) {
-        const uint32_t uw = word();
-        const cx<T> *B4 = P4 + ((uw >> (4 * kq)) & 15) * 144;
-        cx<T> t = cmake<T>(0, 0);
 #pragma unroll
-        for (int j = 0; j < 9; j++) cfma_conj(t, X[j], B4[j * 16]);
-        // O[k] += V[k] t in the operator blocks the products have coefficients in
+        for (int z = 0; z < 3; z++)
 #pragma unroll
-        for (int b = 0; b < NB; b++)
-          if (uw >> (16 + b) & 1) {
-            const T v = c0;
-            c0 = c1;
-            c1 = *cp;
-            cp += 64;
-            ar[b] = TtAcc<T>::mma(v, t.re, ar[b]);
-            ai[b] = TtAcc<T>::mma(v, t.im, ai[b]);
+          for (int y = 0; y < 3; y++) {
+            m[z * 3 + y] = cmake<T>(0, 0);
+#pragma unroll
+            for (int w = 0; w < 3; w++) cfma_conj(m[z * 3 + y], a[w * 3 + y], b[w * 3 + z]);
           }
-        if (uw >> 20) {
+      }
+      const int ncr = fw & 255, ng = ncr + ((fw >> 8) & 255);
+      for (int g = 0; g < ng; g++) {
+        const uint32_t gw = word();
+        cx<T> X[9];
+        {
+          const cx<T> *B2 = sp + 2304 + s + ((gw >> (4 * kq)) & 15) * 144;
+          cx<T> b[9];
+#pragma unroll
+          for (int j = 0; j < 9; j++) b[j] = B2[j * 16];
+          if (g < ncr) {
+#pragma unroll
+            for (int w = 0; w < 3; w++)
+#pragma unroll
+              for (int y = 0; y < 3; y++) {
+                X[w * 3 + y] = cmake<T>(0, 0);
+#pragma unroll
+                for (int z = 0; z < 3; z++) cfma(X[w * 3 + y], b[w * 3 + z], m[z * 3 + y]);
+              }
+          } else {
+            const cx<T> d = m[0] + m[4] + m[8];  // <B1, B3>
+#pragma unroll
+            for (int j = 0; j < 9; j++) X[j] = d * b[j];
+          }
+        }
+        const int nt = (int)(gw >> 16);
+        for (int e = 0; e < nt; e++) {
+          const uint32_t uw = word();
+          const cx<T> *B4 = P4 + ((uw >> (4 * kq)) & 15) * 144;
+          cx<T> t = cmake<T>(0, 0);
+#pragma unroll
+          for (int j = 0; j < 9; j++) cfma_conj(t, X[j], B4[j * 16]);
+          cx<T> u = cmake<T>(0, 0);  // what of t is not finite
+          bool odd = false;
+          if constexpr (safe) {
+            const bool fr = __builtin_isfinite(t.re), fi = __builtin_isfinite(t.im);
+            u = cmake<T>(fr ? (T)0 : t.re, fi ? (T)0 : t.im);
+            t = cmake<T>(fr ? t.re : (T)0, fi ? t.im : (T)0);
+            odd = __any(!fr || !fi);
+          }
+          // operators of block b that have a coefficient v: real sum += v re, imaginary sum += v im
+          auto apart = [&](int b, T v, T re, T im) {
+#pragma unroll 1
+            for (int k = 0; k < 16; k++) {
+              const T w = __shfl(v, 16 * kq + k);
+              T *d = spec + 512 * b + TtAcc<T>::slot(k, s);
+              if (w != 0 && !__builtin_isfinite(re)) atomicAdd(d, w * re);
+              if (w != 0 && !__builtin_isfinite(im)) atomicAdd(d + 256, w * im);
+            }
+          };
+          // O[k] += V[k] t in the operator blocks the products have coefficients in
 #pragma unroll
           for (int b = 0; b < NB; b++)
-            if (uw >> (20 + b) & 1) {
+            if (uw >> (16 + b) & 1) {
               const T v = c0;
               c0 = c1;
               c1 = *cp;
               cp += 64;
-              ar[b] = TtAcc<T>::mma(v, -t.im, ar[b]);
-              ai[b] = TtAcc<T>::mma(v, t.re, ai[b]);
+              ar[b] = TtAcc<T>::mma(v, t.re, ar[b]);
+              ai[b] = TtAcc<T>::mma(v, t.im, ai[b]);
+              if (safe && odd) apart(b, v, u.re, u.im);
             }
+          if (uw >> 20) {
+#pragma unroll
+            for (int b = 0; b < NB; b++)
+              if (uw >> (20 + b) & 1) {
+                const T v = c0;
+                c0 = c1;
+                c1 = *cp;
+                cp += 64;
+                ar[b] = TtAcc<T>::mma(v, -t.im, ar[b]);
+                ai[b] = TtAcc<T>::mma(v, t.re, ai[b]);
+                if (safe && odd) apart(b, v, -u.im, u.re);
+              }
+          }
         }
+        nsum += nt;
+        if (nsum >= 6) flush();
       }
-      nsum += nt;
-      if (nsum >= 6) flush();
+    }
+    flush();
+  };
+  // the waves' sums: thread tid < 256 holds operator row(lane, wave) of every block at its site
+  T o[NB][2];
+  auto reduce = [&]() {
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) red[wave][r * 64 + lane] = h ? ti[b][r] : tr[b][r];
+        __syncthreads();
+        if (tid < 256) {
+          T v[TT_WAVES];
+#pragma unroll
+          for (int w = 0; w < TT_WAVES; w++) v[w] = red[w][tid];
+#pragma unroll
+          for (int n = TT_WAVES / 2; n > 0; n /= 2)  // pairwise
+#pragma unroll
+            for (int w = 0; w < n; w++) v[w] += v[w + n];
+          o[b][h] = v[0];
+        }
+        __syncthreads();
+      }
+  };
+  walk(std::false_type{});
+  reduce();
+  {
+    // a sum that is not finite: its tile again, with the care of SAFE
+    bool bad = false;
+    if (tid < 256)
+#pragma unroll
+      for (int b = 0; b < NB; b++) bad = bad || !__builtin_isfinite(o[b][0]) || !__builtin_isfinite(o[b][1]);
+    int *flag = (int *)spec;
+    const int mine = __any(bad);
+    if (lane == 0) flag[wave] = mine;
+    __syncthreads();
+    int any = 0;
+#pragma unroll
+    for (int w = 0; w < 4; w++) any |= flag[w];
+    if (__builtin_amdgcn_readfirstlane(any)) {
+      __syncthreads();
+      for (int i = tid; i < 512 * NB; i += NT) spec[i] = 0;
+      __syncthreads();
+      walk(std::true_type{});
+      __syncthreads();
+      T apart[NB][2];
+#pragma unroll
+      for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) apart[b][h] = spec[512 * b + 256 * h + (tid & 255)];
+      __syncthreads();
+      reduce();
+#pragma unroll
+      for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) o[b][h] += apart[b][h];
     }
   }
-  flush();
-  // the waves' sums
   const int64_t ncols = (int64_t)gridDim.y * nch_total, col0 = (int64_t)blockIdx.y * nch_total + ch0;
 #pragma unroll
   for (int b = 0; b < NB; b++) {
-    T o[2];
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-#pragma unroll
-      for (int r = 0; r < 4; r++) red[wave][r * 64 + lane] = h ? ti[b][r] : tr[b][r];
-      __syncthreads();
-      if (tid < 256) {
-        T v[TT_WAVES];
-#pragma unroll
-        for (int w = 0; w < TT_WAVES; w++) v[w] = red[w][tid];
-#pragma unroll
-        for (int n = TT_WAVES / 2; n > 0; n /= 2)  // pairwise
-#pragma unroll
-          for (int w = 0; w < n; w++) v[w] += v[w + n];
-        o[h] = v[0];
-      }
-      __syncthreads();
-    }
     const int k = 16 * b + TtAcc<T>::row(lane, wave);
     if (tid < 256 && k < S.nops && x0 + s < V3)
-      gstore(out + ctile_idx(col0 + k, x0 + s, ncols), cmake<T>(sg * o[0], sg * o[1]));
+      gstore(out + ctile_idx(col0 + k, x0 + s, ncols), cmake<T>(sg * o[b][0], sg * o[b][1]));
   }
 }
 

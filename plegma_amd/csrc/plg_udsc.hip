@@ -652,6 +652,7 @@ template <> struct UdAcc<float> {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
   }
   static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane >> 4) + r; }
+  static __device__ __forceinline__ int slot(int k, int s) { return (k & 3) * 64 + (k >> 2) * 16 + s; }  // r * 64 + lane
 };
 template <> struct UdAcc<double> {
   typedef double v4 __attribute__((ext_vector_type(4)));
@@ -659,6 +660,7 @@ template <> struct UdAcc<double> {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
   static __device__ __forceinline__ int row(int lane, int r) { return 4 * r + (lane >> 4); }
+  static __device__ __forceinline__ int slot(int k, int s) { return (k >> 2) * 64 + (k & 3) * 16 + s; }
 };
 
 template <typename T>
@@ -713,97 +715,165 @@ __global__ __launch_bounds__(64 * UD_WAVES, sizeof(T) == 4 ? 4 : 2) void k_udsc_
   for (int gi = blockIdx.z * groups_per_block; gi < g1; gi++) {
     const UdscGroup &G = S.g[gi];
     v4 ar[UD_NJ], ai[UD_NJ];
-#pragma unroll
-    for (int j = 0; j < UD_NJ; j++) ar[j] = ai[j] = (v4)(T)0;
     const cx<T> *A = sp + G.pa * 2304 + s, *B = sp + G.pb * 2304 + s;
-    const int st0 = G.step0[wave], nst = G.nsteps[wave];
-    int un = G.unit0[wave], ci = G.coef0[wave];
-    v4 cf[2] = {coef[ci * 64], coef[(ci + 1) * 64]};
-    // a step: two quads of each quarter (N = 2, the terms' reads of the third
-    // propagator serve both), or one
-    auto step = [&](auto N, int st) {
-      const uint32_t cw = S.steps[3 * st + 2];
-      cx<T> d[N.value][9];
+    // SAFE: values that are not finite stay out of the matrix products, where
+    // a zero coefficient would spread them over the operators of a product,
+    // and go one by one to those that have a coefficient, in spec
+    T *spec = &red[0][0];  // [product][real, imaginary][as a wave's sums lie in red]
+    static_assert(2 * UD_NJ <= UD_WAVES, "spec fits red");
+    auto walk = [&](auto SAFE) {
+      constexpr bool safe = SAFE.value;
 #pragma unroll
-      for (int b = 0; b < N.value; b++) {
-        const int q = (S.steps[3 * st + b] >> (8 * kq)) & 255;
-        const cx<T> *Aq = A + (q & 15) * 144, *Bq = B + (q >> 4) * 144;
-        cx<T> x[9], y[9];
+      for (int j = 0; j < UD_NJ; j++) ar[j] = ai[j] = (v4)(T)0;
+      const int st0 = G.step0[wave], nst = G.nsteps[wave];
+      int un = G.unit0[wave], ci = G.coef0[wave];
+      v4 cf[2] = {coef[ci * 64], coef[(ci + 1) * 64]};
+      // a step: two quads of each quarter (N = 2, the terms' reads of the third
+      // propagator serve both), or one
+      auto step = [&](auto N, int st) {
+        const uint32_t cw = S.steps[3 * st + 2];
+        cx<T> d[N.value][9];
 #pragma unroll
-        for (int j = 0; j < 9; j++) {
-          x[j] = Aq[j * 16];
-          y[j] = Bq[j * 16];
+        for (int b = 0; b < N.value; b++) {
+          const int q = (S.steps[3 * st + b] >> (8 * kq)) & 255;
+          const cx<T> *Aq = A + (q & 15) * 144, *Bq = B + (q >> 4) * 144;
+          cx<T> x[9], y[9];
+#pragma unroll
+          for (int j = 0; j < 9; j++) {
+            x[j] = Aq[j * 16];
+            y[j] = Bq[j * 16];
+          }
+          udsc_diquark(x, y, d[b]);
         }
-        udsc_diquark(x, y, d[b]);
-      }
 #pragma unroll
-      for (int j = 0; j < UD_NJ; j++) {
-        const int nt = (cw >> (8 * j)) & 255;
-        if (nt == 0) continue;
-        const cx<T> *C = sp + G.third[j] * 2304 + s;
-        for (int e0 = 0; e0 < nt; e0 += 4, un++, ci += N.value) {
-          const uint64_t pw = (uint64_t)S.units[2 * un] | (uint64_t)S.units[2 * un + 1] << 32;
-          const int pl = (int)(pw >> (16 * kq)) & 0xffff;
-          v4 cn[N.value];  // the next unit's
-#pragma unroll
-          for (int b = 0; b < N.value; b++) cn[b] = coef[(ci + N.value + b) * 64];
-          v4 ur = (v4)(T)0, ui = (v4)(T)0;    // the unit's sums: sums of sums round less than one long sum
-#pragma unroll
-          for (int e = 0; e < 4; e++) {
-            if (e0 + e >= nt) break;
-            const cx<T> *Cp = C + ((pl >> (4 * e)) & 15) * 144;
-            cx<T> t[N.value];
-#pragma unroll
-            for (int b = 0; b < N.value; b++) t[b] = cmake<T>(0, 0);
-#pragma unroll
-            for (int c = 0; c < 9; c++) {
-              const cx<T> v = Cp[c * 16];
-#pragma unroll
-              for (int b = 0; b < N.value; b++) cfma(t[b], d[b][c], v);
-            }
+        for (int j = 0; j < UD_NJ; j++) {
+          const int nt = (cw >> (8 * j)) & 255;
+          if (nt == 0) continue;
+          const cx<T> *C = sp + G.third[j] * 2304 + s;
+          for (int e0 = 0; e0 < nt; e0 += 4, un++, ci += N.value) {
+            const uint64_t pw = (uint64_t)S.units[2 * un] | (uint64_t)S.units[2 * un + 1] << 32;
+            const int pl = (int)(pw >> (16 * kq)) & 0xffff;
+            v4 cn[N.value];  // the next unit's (SAFE: no loads ahead, for the registers)
 #pragma unroll
             for (int b = 0; b < N.value; b++) {
-              ur = UdAcc<T>::mma(cf[b][e], t[b].re, ur);
-              ui = UdAcc<T>::mma(cf[b][e], t[b].im, ui);
+              if constexpr (safe) cf[b] = coef[(ci + b) * 64];
+              else cn[b] = coef[(ci + N.value + b) * 64];
             }
-          }
-          ar[j] += ur;
-          ai[j] += ui;
+            v4 ur = (v4)(T)0, ui = (v4)(T)0;    // the unit's sums: sums of sums round less than one long sum
 #pragma unroll
-          for (int b = 0; b < N.value; b++) cf[b] = cn[b];
+            for (int e = 0; e < 4; e++) {
+              if (e0 + e >= nt) break;
+              const cx<T> *Cp = C + ((pl >> (4 * e)) & 15) * 144;
+              cx<T> t[N.value];
+#pragma unroll
+              for (int b = 0; b < N.value; b++) t[b] = cmake<T>(0, 0);
+#pragma unroll
+              for (int c = 0; c < 9; c++) {
+                const cx<T> v = Cp[c * 16];
+#pragma unroll
+                for (int b = 0; b < N.value; b++) cfma(t[b], d[b][c], v);
+              }
+#pragma unroll
+              for (int b = 0; b < N.value; b++) {
+                if constexpr (safe) {
+                  const bool fr = __builtin_isfinite(t[b].re), fi = __builtin_isfinite(t[b].im);
+                  if (__any(!fr || !fi)) {
+#pragma unroll 1
+                    for (int k = 0; k < 16; k++) {
+                      const T w = __shfl(cf[b][e], 16 * kq + k);
+                      T *o = spec + 512 * j + UdAcc<T>::slot(k, s);
+                      if (w != 0 && !fr) atomicAdd(o, w * t[b].re);
+                      if (w != 0 && !fi) atomicAdd(o + 256, w * t[b].im);
+                    }
+                    t[b] = cmake<T>(fr ? t[b].re : (T)0, fi ? t[b].im : (T)0);
+                  }
+                }
+                ur = UdAcc<T>::mma(cf[b][e], t[b].re, ur);
+                ui = UdAcc<T>::mma(cf[b][e], t[b].im, ui);
+              }
+            }
+            ar[j] += ur;
+            ai[j] += ui;
+            if constexpr (!safe)
+#pragma unroll
+              for (int b = 0; b < N.value; b++) cf[b] = cn[b];
+          }
+        }
+      };
+      const int mid = st0 + G.npair[wave];
+      for (int st = st0; st < mid; st++) step(std::integral_constant<int, 2>{}, st);
+      for (int st = mid; st < st0 + nst; st++) step(std::integral_constant<int, 1>{}, st);
+    };
+    walk(std::false_type{});
+    int tq = threadIdx.x;  // opaque: what derives from it is not kept across the walk
+    asm volatile("" : "+v"(tq));
+    const int ln = tq & 63;
+    // the waves' sums: thread tq < 256 holds operator row(ln, wave) of every product at its site
+    T o[UD_NJ][2];
+#pragma unroll
+    for (int j = 0; j < UD_NJ; j++) o[j][0] = o[j][1] = 0;
+    auto reduce = [&]() {
+#pragma unroll
+      for (int j = 0; j < UD_NJ; j++) {
+        if (j >= G.nprod) break;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+#pragma unroll
+          for (int r = 0; r < 4; r++) red[wave][r * 64 + ln] = h ? ai[j][r] : ar[j][r];
+          __syncthreads();
+          if (tq < 256) {
+            T v[UD_WAVES];
+#pragma unroll
+            for (int w = 0; w < UD_WAVES; w++) v[w] = red[w][tq];
+#pragma unroll
+            for (int n = UD_WAVES / 2; n > 0; n /= 2)  // pairwise
+#pragma unroll
+              for (int w = 0; w < n; w++) v[w] += v[w + n];
+            o[j][h] = v[0];
+          }
+          __syncthreads();
         }
       }
     };
-    const int mid = st0 + G.npair[wave];
-    for (int st = st0; st < mid; st++) step(std::integral_constant<int, 2>{}, st);
-    for (int st = mid; st < st0 + nst; st++) step(std::integral_constant<int, 1>{}, st);
-    // the waves' sums
+    reduce();
+    // a sum that is not finite: the group again, with the care of SAFE
+    bool bad = false;
+#pragma unroll
+    for (int j = 0; j < UD_NJ; j++) bad = bad || !__builtin_isfinite(o[j][0]) || !__builtin_isfinite(o[j][1]);
+    int *flag = (int *)spec;
+    const int mine = __any(bad);
+    if (ln == 0) flag[wave] = mine;
+    __syncthreads();
+    int any = 0;
+#pragma unroll
+    for (int w = 0; w < 4; w++) any |= flag[w];
+    __syncthreads();  // red is the next group's (or SAFE's) after this
+    if (__builtin_amdgcn_readfirstlane(any)) {
+      for (int i = tq; i < 512 * UD_NJ; i += NT) spec[i] = 0;
+      __syncthreads();
+      walk(std::true_type{});
+      __syncthreads();
+      T apart[UD_NJ][2];
+#pragma unroll
+      for (int j = 0; j < UD_NJ; j++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) apart[j][h] = spec[512 * j + 256 * h + (tq & 255)];
+      __syncthreads();
+      reduce();
+#pragma unroll
+      for (int j = 0; j < UD_NJ; j++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) o[j][h] += apart[j][h];
+    }
     const T sgp = prop_sign(props[G.pa], row.t) * prop_sign(props[G.pb], row.t);
+    const int k = UdAcc<T>::row(ln, wave);
+    const int64_t x = (int64_t)blockIdx.x * 16 + (tq & 15);
 #pragma unroll
     for (int j = 0; j < UD_NJ; j++) {
       if (j >= G.nprod) break;
-      T o[2];
-#pragma unroll
-      for (int h = 0; h < 2; h++) {
-#pragma unroll
-        for (int r = 0; r < 4; r++) red[wave][r * 64 + lane] = h ? ai[j][r] : ar[j][r];
-        __syncthreads();
-        if (tid < 256) {
-          T v[UD_WAVES];
-#pragma unroll
-        for (int w = 0; w < UD_WAVES; w++) v[w] = red[w][tid];
-#pragma unroll
-        for (int n = UD_WAVES / 2; n > 0; n /= 2)  // pairwise
-#pragma unroll
-          for (int w = 0; w < n; w++) v[w] += v[w + n];
-        o[h] = v[0];
-        }
-        __syncthreads();
-      }
-      const int k = UdAcc<T>::row(lane, wave);
-      if (tid < 256 && k < G.nops[j] && x0 + s < V3) {
+      if (tq < 256 && k < G.nops[j] && x < V3) {
         const T sg = sgp * prop_sign(props[G.third[j]], row.t);
-        gstore(out + ctile_idx(col0 + G.ch0[j] + k, x0 + s, ncols), cmake<T>(sg * o[0], sg * o[1]));
+        gstore(out + ctile_idx(col0 + G.ch0[j] + k, x, ncols), cmake<T>(sg * o[j][0], sg * o[j][1]));
       }
     }
   }
