@@ -223,7 +223,8 @@ constexpr int MF_WIDTH = 511;   // widest layer (products below 512 terms are on
 constexpr int MF_MAXL = 16;
 constexpr int MF_THREADS = 1024, MF_WAVES = MF_THREADS / 64;
 constexpr int MF_ZL = 2;        // hidden layers whose Z stays in LDS for the backward pass
-constexpr int MF_LD = 512 + 8;  // LDS row stride: the 16 rows of a fragment read start 4 banks apart
+// columns of the activations in LDS of a block of nw waves
+__host__ __device__ constexpr int mlp_cols(int nw) { return nw == 1 ? 32 : nw == 4 ? 64 : nw == 8 ? 192 : 512; }
 __host__ __device__ __forceinline__ int pad16(int n) { return (n + 15) / 16 * 16; }
 __host__ __device__ __forceinline__ int pad32(int n) { return (n + 31) / 32 * 32; }
 
@@ -270,29 +271,34 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // The rows [4 Q blockIdx.x, + 4 Q) through the whole network (Q rows a lane, 4 or
-// 2): every layer's outputs are column tiles of 16, one per wave in turn, the activations stay in
-// LDS.  BACK: the loss gradient 2 (y - t) scale and the chain of dX as well, with
+// 2; NW waves): every layer's outputs are column tiles of 16, one per wave in turn,
+// the activations stay in LDS.  BACK: the loss gradient 2 (y - t) scale and the chain of dX as well, with
 // the transposed operands of the weight gradients for k_mlp_update.  y (may be
 // NULL): outputs, [B][out].  coef (may be NULL): the step counter is advanced
 // and its bias corrections are written.
 // Bound by the chain of layers: eight rows a block (Q = 2, half of each MFMA's
 // rows unused) spread the learned workload's 2 048 rows over 256 CUs and halve
 // the activations' vector instructions of a wave (a 256-wide layer 2.6 -> 2.2
-// us); 16 rows where the batch fills the CUs.  A wave loads the weights of
+// us); 16 rows where the batch fills the CUs.  There a block has as many waves as
+// the widest layer has column tiles (two tiles a wave from 129 to 192 columns),
+// so that idle waves leave the CUs to other blocks: forward passes of 131 072
+// rows, 16 waves a block always / so, us: 17-11 47 / 12, 17-64-11 83 / 28,
+// 17-129-11 98 / 69 (launch by product 19, 75, 95).  A wave loads the weights of
 // its first tile of the next layer before this layer's stores.
 // 17-256-256-11 at 2 048 rows: 17 us (a 256 x 256 layer streams its 131 KB of
 // weights through the CU in about 2 us; the transposed outputs' stores are
 // 4 us), k_mlp_update 6 us; a step takes 28 us against 153 us in 23 launches.
-template <bool BACK, int Q>
-__global__ __launch_bounds__(MF_THREADS) void k_mlp_rows(MlpDev d, const float *__restrict__ x, const float *__restrict__ t,
+template <bool BACK, int Q, int NW>
+__global__ __launch_bounds__(64 * NW) void k_mlp_rows(MlpDev d, const float *__restrict__ x, const float *__restrict__ t,
                                                          float scale, float *__restrict__ y, int *__restrict__ step,
                                                          float *__restrict__ coef, float b1, float b2) {
-  __shared__ __align__(16) uint16_t act[2][16][MF_LD];
+  constexpr int LD = mlp_cols(NW) + 8;  // the 16 rows of a fragment read start on distinct banks
+  __shared__ __align__(16) uint16_t act[2][16][LD];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int row0 = blockIdx.x * 4 * Q, lc = lane & 15, lk = 8 * (lane >> 4);
   // the lane's rows: of the block, and of act (and of the MFMA)
   const int rq = Q * (lane >> 4), r4 = 4 * (lane >> 4);
-  __shared__ float zl_[MF_ZL][MF_THREADS * Q];  // Z of the waves' first tiles of the first hidden layers
+  __shared__ float zl_[MF_ZL][64 * NW * Q];  // Z of the waves' first tiles of the first hidden layers
   // eight fragments (256 terms) of rows [16 tile, + 16) of a padded matrix
   u16x8 w8[8];
   auto load = [&](const uint16_t *w, int KP, int tile, int k0) {
@@ -347,12 +353,22 @@ __global__ __launch_bounds__(MF_THREADS) void k_mlp_rows(MlpDev d, const float *
   float bias0 = bias_of(0, wave * 16 + lc), tv0[Q] = {};
   if (wave * 16 < d.dims[1]) load(d.wf[0], pad32(d.dims[0]), wave, 0);
   if (BACK) targets(wave * 16 + lc, tv0);
-  if (wave < 4 * Q) {  // 64 lanes a row
-    const int Ni = d.dims[0], KP = pad32(Ni), r = wave;
+  if (wave < 4 * Q) {  // 64 lanes a row, the wave's rows loaded together
+    constexpr int RW = (4 * Q + NW - 1) / NW;
+    const int Ni = d.dims[0], KP = pad32(Ni);
     for (int i = lane; i < KP; i += 64) {
-      const uint16_t b = (i < Ni && row0 + r < d.B) ? bf16_rne(x[(int64_t)(row0 + r) * Ni + i]) : (uint16_t)0;
-      act[0][r / Q * 4 + r % Q][i] = b;
-      if (BACK && i < Ni) d.xt[0][frag_idx(i, row0 + r, d.BT / 32)] = b;
+      uint16_t b[RW];
+#pragma unroll
+      for (int k = 0; k < RW; k++) {
+        const int r = wave + k * NW;
+        b[k] = (i < Ni && row0 + r < d.B) ? bf16_rne(x[(int64_t)(row0 + r) * Ni + i]) : (uint16_t)0;
+      }
+#pragma unroll
+      for (int k = 0; k < RW; k++) {
+        const int r = wave + k * NW;
+        act[0][r / Q * 4 + r % Q][i] = b[k];
+        if (BACK && i < Ni) d.xt[0][frag_idx(i, row0 + r, d.BT / 32)] = b[k];
+      }
     }
   }
   if (BACK && coef && blockIdx.x == 0 && tid == 0) {
@@ -377,7 +393,7 @@ __global__ __launch_bounds__(MF_THREADS) void k_mlp_rows(MlpDev d, const float *
     } else if (BACK && l > 0) {
       if (wave * 16 < Ni) load(d.wt[l], pad32(No), wave, 0);
     }
-    for (int tile = wave; tile < pad32(No) / 16; tile += MF_WAVES) {
+    for (int tile = wave; tile < pad32(No) / 16; tile += NW) {
       const int n = tile * 16 + lc;
       hv h = {};
       if (tile < NT) {
@@ -414,7 +430,7 @@ __global__ __launch_bounds__(MF_THREADS) void k_mlp_rows(MlpDev d, const float *
       if (!last || BACK) put(h, n, No, cur ^ 1, BACK ? (last ? d.dzt[l] : d.xt[l + 1]) : nullptr);
     }
     // (waves of several tiles have overwritten their prefetched weights)
-    if (wave + MF_WAVES < NT) {
+    if (wave + NW < NT) {
       if (!last) {
         if (wave * 16 < d.dims[l + 2]) load(d.wf[l + 1], pad32(No), wave, 0);
       } else if (BACK && l > 0) {
@@ -431,7 +447,7 @@ __global__ __launch_bounds__(MF_THREADS) void k_mlp_rows(MlpDev d, const float *
     f4 dx = {0, 0, 0, 0};
     if (wave < NT) dx = product(wl, pad32(No), wave, cur);
     if (l > 1 && wave * 16 < d.dims[l - 1]) load(d.wt[l - 1], pad32(Ni), wave, 0);
-    for (int tile = wave; tile < pad32(Ni) / 16; tile += MF_WAVES) {
+    for (int tile = wave; tile < pad32(Ni) / 16; tile += NW) {
       const int n = tile * 16 + lc;
       hv h = {};
       if (tile < NT) {
@@ -449,7 +465,7 @@ __global__ __launch_bounds__(MF_THREADS) void k_mlp_rows(MlpDev d, const float *
       }
       put(h, n, Ni, cur ^ 1, d.dzt[l - 1]);
     }
-    if (l > 1 && wave + MF_WAVES < NT && wave * 16 < d.dims[l - 1]) load(d.wt[l - 1], pad32(Ni), wave, 0);
+    if (l > 1 && wave + NW < NT && wave * 16 < d.dims[l - 1]) load(d.wt[l - 1], pad32(Ni), wave, 0);
     cur ^= 1;
     lds_barrier();
   }
@@ -503,15 +519,19 @@ __global__ __launch_bounds__(MF_THREADS) void k_mlp_update(MlpDev d, int ks, int
       const u16x8 *A = (const u16x8 *)d.dzt[l] + (int64_t)(m0 / 16) * KS * 64 + lane;
       const u16x8 *X = (const u16x8 *)d.xt[l] + (int64_t)(n0 / 16) * KS * 64 + lane;
       f4 acc[2][2] = {{{0, 0, 0, 0}, {0, 0, 0, 0}}, {{0, 0, 0, 0}, {0, 0, 0, 0}}};
+      // halves of the tile that are padding alone are not read: a batch of
+      // many rows and a small layer are bound by one CU's reads (17-11 at 1 M
+      // rows: a training step 2.29 -> 1.61 ms)
+      const bool a2 = m0 + 16 < No, b2 = n0 + 16 < Ni;
       for (int k0 = kb; k0 < ke; k0 += 128) {
-        u16x8 a[4][2], b[4][2];
+        u16x8 a[4][2] = {}, b[4][2] = {};
 #pragma unroll
         for (int i = 0; i < 4; i++)
           if (k0 + 32 * i < ke)
 #pragma unroll
             for (int q = 0; q < 2; q++) {
-              a[i][q] = A[(int64_t)(q * KS + k0 / 32 + i) * 64];
-              b[i][q] = X[(int64_t)(q * KS + k0 / 32 + i) * 64];
+              if (q == 0 || a2) a[i][q] = A[(int64_t)(q * KS + k0 / 32 + i) * 64];
+              if (q == 0 || b2) b[i][q] = X[(int64_t)(q * KS + k0 / 32 + i) * 64];
             }
 #pragma unroll
         for (int i = 0; i < 4; i++)
@@ -661,16 +681,19 @@ static int rows_pass(plg_mlp_s *net, const float *x, const float *t, int B, floa
   const MlpDev d = rows_dev(net, B);
   const float scale = 1.0f / (float)((int64_t)B * net->dims[net->L]);
   float *coef = count ? net->d_coef : nullptr;
-  // eight rows a block while 16 would leave CUs of the 256 without one
-  if (pad32(B) / 8 <= 256) {
-    const int grid = pad32(B) / 8;
-    if (t) k_mlp_rows<true, 2><<<grid, MF_THREADS, 0, st>>>(d, x, t, scale, y, net->d_step, coef, MG_B1, MG_B2);
-    else k_mlp_rows<false, 2><<<grid, MF_THREADS, 0, st>>>(d, x, nullptr, 0.0f, y, nullptr, nullptr, MG_B1, MG_B2);
-  } else {
-    const int grid = pad32(B) / 16;
-    if (t) k_mlp_rows<true, 4><<<grid, MF_THREADS, 0, st>>>(d, x, t, scale, y, net->d_step, coef, MG_B1, MG_B2);
-    else k_mlp_rows<false, 4><<<grid, MF_THREADS, 0, st>>>(d, x, nullptr, 0.0f, y, nullptr, nullptr, MG_B1, MG_B2);
-  }
+  auto launch = [&](auto Q, auto NW) {
+    const dim3 grid(pad32(B) / (4 * Q.value)), block(64 * NW.value);
+    if (t) k_mlp_rows<true, Q.value, NW.value><<<grid, block, 0, st>>>(d, x, t, scale, y, net->d_step, coef, MG_B1, MG_B2);
+    else k_mlp_rows<false, Q.value, NW.value><<<grid, block, 0, st>>>(d, x, nullptr, 0.0f, y, nullptr, nullptr, MG_B1, MG_B2);
+  };
+  // eight rows a block while 16 would leave CUs of the 256 without one; the
+  // waves of the blocks of 16 by the widest layer (k_mlp_rows has the times)
+  const int out = *std::max_element(net->dims.begin() + 1, net->dims.end()), all = std::max(out, net->dims[0]);
+  if (pad32(B) / 8 <= 256) launch(ic<2>{}, ic<16>{});
+  else if (out <= 16 && all <= mlp_cols(1)) launch(ic<4>{}, ic<1>{});
+  else if (out <= 64 && all <= mlp_cols(4)) launch(ic<4>{}, ic<4>{});
+  else if (out <= 192 && all <= mlp_cols(8)) launch(ic<4>{}, ic<8>{});
+  else launch(ic<4>{}, ic<16>{});
   return hipGetLastError() == hipSuccess ? PLG_OK : fail(PLG_ERR_HIP, "MLP rows launch failed");
 }
 // gradients of the last rows_pass: into net->g, or (adam) applied
