@@ -749,6 +749,11 @@ static std::string tune_cache_path() {
   return std::string(h && *h ? h : "/tmp") + "/.plegma_amd_tunecache";
 }
 
+// The forms of the kernels that tuning times, part of every key: a kernel whose
+// best tiles may differ from those of the form before it takes a new name here,
+// so that choices made for the old one are not taken over.
+static const char *const TUNE_FORMS = "baryon.quad mesmes.quad sep.mfma";
+
 static std::string tune_key(const Plan &P) {
   hipDeviceProp_t prop;
   hipGetDeviceProperties(&prop, g_ctx.device);
@@ -756,7 +761,7 @@ static std::string tune_key(const Plan &P) {
   k << prop.gcnArchName << " L=" << g_ctx.L[0] << "x" << g_ctx.L[1] << "x" << g_ctx.L[2] << "x" << g_ctx.L[3]
     << " nmom=" << P.nmom << " cols=" << P.rows.size() * P.nch_c << " rows=" << P.rows.size() << " mode=" << P.mode
     << " npairs=" << P.npairs << " terms=" << P.terms << " kind=" << P.kind << " mask=" << P.mask
-    << " proj=pair32z.sep" << (P.sep.ok ? 1 : 0);
+    << " proj=pair32z.sep" << (P.sep.ok ? 1 : 0) << " kernels=" << TUNE_FORMS << ",";
   for (auto &l : P.launches) k << " L" << l.what << "." << l.set << "." << l.two << l.mes << "." << l.gmask;
   std::string s = k.str();
   for (char &ch : s)
