@@ -1673,6 +1673,7 @@ static int udsc_run(const plg_prop *up, const plg_prop *dn, const plg_prop *st, 
 // 64-bit hash of the counts, spins, colour slots and coefficients (a built-in
 // table by its number) and by the precision.  A table whose device arrays are large is not kept.
 struct TetraTable {
+  TetraCost cost;
   std::vector<TetraSched> s;  // one per launch
   std::vector<TetraTermsSched> terms;  // or, term by term, one per set
   std::vector<void *> mem;
@@ -1703,9 +1704,9 @@ static uint64_t hash_bytes(const void *data, size_t n, uint64_t h) {
 }
 
 // builtin: the number of a built-in table, which needs no hash (a read of
-// 0.5 to 2.5 MB); -1: a caller's table
+// 0.5 to 2.5 MB); -1: a caller's table.  In the form for nrows slices.
 static int tetra_pack_cached(const int16_t *idxs, const int16_t *cols, const float *vals, const int16_t *counts,
-                             int nops, int builtin, int T, std::shared_ptr<const TetraTable> &out) {
+                             int nops, int builtin, int T, int nrows, std::shared_ptr<const TetraTable> &out) {
   if (nops <= 0 || nops > TETRA_MAXOPS) return PLG_ERR_UNSUPPORTED;
   size_t nt = 0;
   for (int k = 0; k < nops; k++) {
@@ -1723,16 +1724,17 @@ static int tetra_pack_cached(const int16_t *idxs, const int16_t *cols, const flo
   {
     std::lock_guard<std::mutex> lk(g_pack_mu);
     for (auto &e : g_pack_cache)
-      if (e.first == h) {
+      if (e.first == h && tetra_by_terms(e.second->cost, g_ctx.V3, nrows) == !e.second->terms.empty()) {
         out = e.second;
         return PLG_OK;
       }
   }
-  std::vector<TetraPacked> pk;
-  bool by_terms = false;
-  int rc = tetra_pack(idxs, cols, vals, counts, nops, TT_OPS, pk, by_terms);
+  TetraProds prods;
+  int rc = tetra_products(idxs, cols, vals, counts, nops, prods);
   if (rc) return rc;
   auto tab = std::make_shared<TetraTable>();
+  TetraWalks walks;
+  tab->cost = tetra_cost(prods, TT_OPS, T == PLG_F64, walks);
   size_t bytes = 0;
   auto put = [&](const auto &v, const void **d) {
     typename std::decay_t<decltype(v)>::value_type *p = nullptr;
@@ -1742,8 +1744,10 @@ static int tetra_pack_cached(const int16_t *idxs, const int16_t *cols, const flo
     *d = p;
     return r;
   };
-  if (by_terms) {
-    pk.clear();
+  std::vector<TetraPacked> pk;
+  if (!tetra_by_terms(tab->cost, g_ctx.V3, nrows)) {
+    tetra_pack(prods, walks, pk);
+  } else {
     TetraTermsPacked tp;
     if ((rc = tetra_pack_terms(idxs, cols, vals, counts, nops, tp))) return rc;
     const void *coef = nullptr;
@@ -1788,17 +1792,18 @@ static int tetra_run(const plg_prop *const views[4], const int16_t *idxs, const 
   if (!idxs || !col_contr || !vals || !counts || nops <= 0) return fail(PLG_ERR_INVALID, "empty table");
   for (int i = 0; i < 4; i++)
     if (!views[i]) return fail(PLG_ERR_INVALID, "NULL propagator view");
+  int lt = 1;
+  const int wrc = plg_window(source, totalT, nullptr, nullptr, &lt);  // (a bad table is reported first)
   const int prec = mode == PLG_MODE_F64 ? PLG_F64 : PLG_F32;
   std::shared_ptr<const TetraTable> tab;  // held until the stream is synchronised
-  rc = tetra_pack_cached(idxs, col_contr, vals, counts, nops, builtin, prec, tab);
+  rc = tetra_pack_cached(idxs, col_contr, vals, counts, nops, builtin, prec, lt, tab);
   if (rc == PLG_ERR_INVALID) return fail(rc, "spin or colour index outside 0..3");
   if (rc == PLG_ERR_HIP) return rc;
   if (rc)
     return fail(rc, "table outside the supported form (64 operators; colour slots a permutation of the four "
                     "sums, closing as <P1,P3><P2,P4>, Tr[(P3^dag P1)(P4^dag P2)], <P1,P4><P2,P3> or "
                     "Tr[(P4^dag P1)(P3^dag P2)]; 65536 distinct coefficients)");
-  int lt;
-  if ((rc = plg_window(source, totalT, nullptr, nullptr, &lt))) return rc;
+  if (wrc) return plg_window(source, totalT, nullptr, nullptr, &lt);
   const Window w = window_of(g_ctx.L, source, totalT);
   const int T = g_ctx.L[3];
   const int64_t inner = space == PLG_MOMENTUM_SPACE ? (int64_t)nmom : g_ctx.V3;

@@ -5,6 +5,7 @@
 #include "plg_common.h"
 
 #include <array>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -160,13 +161,34 @@ struct TetraSched {
 constexpr int TT_OPS = 32;
 struct TetraPacked {
   TetraSched s{};
-  int64_t cost = 0;  // FMAs of a lane per 16 sites, a matrix instruction counted as 13
   std::vector<uint32_t> words;
   std::vector<double> coef;
 };
-// by_terms: the table is better contracted term by term
-int tetra_pack(const int16_t *idxs, const int16_t *cols, const float *vals, const int16_t *counts, int nops, int per,
-               std::vector<TetraPacked> &out, bool &by_terms);
+// a table's terms, merged into products (terms of one structure on the same
+// four spin pairs) with a coefficient per operator
+struct TetraProd {
+  std::vector<std::pair<int, std::array<double, 2>>> v;
+};
+struct TetraProds {
+  int nops = 0;
+  std::vector<TetraProd> prods;
+  std::vector<int> index;  // set << 17 | structure << 16 | p << 8 | q -> product or -1 (structure 0 crossed, 1 direct)
+  std::vector<std::array<int, 2>> terms[2];  // per set and operator: terms before the merging, crossed and direct
+};
+int tetra_products(const int16_t *idxs, const int16_t *cols, const float *vals, const int16_t *counts, int nops,
+                   TetraProds &out);
+// us of the two forms on a full chip (slots workgroups, of 16 sites by the
+// walk, of 64 term by term), and the choice for nrows slices of V3 sites
+struct TetraCost {
+  double walk = 0, terms = 0;
+  int slots = 0;
+};
+bool tetra_by_terms(const TetraCost &c, int64_t V3, int64_t nrows);
+// the walks of a table, one per `per` operators, their cost, and their packed form
+struct TetraWalk;
+typedef std::vector<std::shared_ptr<const TetraWalk>> TetraWalks;
+TetraCost tetra_cost(const TetraProds &P, int per, bool f64, TetraWalks &walks);
+void tetra_pack(const TetraProds &P, const TetraWalks &walks, std::vector<TetraPacked> &out);
 template <typename T>
 int launch_tetra(const TetraSched &S, const PropDev<T> *props, const RowDev *rows, int nrows, cx<T> *out,
                  int64_t V3, int T_lat, int nch_total, int ch0, hipStream_t st);

@@ -337,20 +337,8 @@ template int launch_tetra<double>(const TetraSched &, const PropDev<double> *, c
 template int launch_tetra<float>(const TetraSched &, const PropDev<float> *, const RowDev *, int, cx<float> *,
                                  int64_t, int, int, int, hipStream_t);
 
-// a product: its coefficient per operator
-struct TetraProd {
-  std::vector<std::pair<int, std::array<double, 2>>> v;
-};
-
-// the walk of operators k0 .. k0 + nops - 1; index: the product of each
-// set << 17 | structure << 16 | p << 8 | q (structure 0 crossed, 1 direct)
-static void tetra_walk(const std::vector<TetraProd> &prods, const std::vector<int> &index, int k0, int nops,
-                       TetraPacked &out) {
-  out = TetraPacked{};
-  auto used = [&](int id) {
-    return id >= 0 && std::any_of(prods[id].v.begin(), prods[id].v.end(),
-                                  [&](const auto &kv) { return kv.first >= k0 && kv.first < k0 + nops; });
-  };
+// the walk of operators k0 .. k0 + nops - 1: its steps by wave
+struct TetraWalk {
   // per (set, p): its groups of one structure and s2, most products first
   struct Group {
     int s2;
@@ -367,29 +355,68 @@ static void tetra_walk(const std::vector<TetraProd> &prods, const std::vector<in
     std::array<const Item *, 4> it;
     int cost;
   };
+  int k0, nops;
+  std::vector<uint8_t> mask;  // of a product: operator blocks with a real (bits 0-3) and an imaginary (4-7) coefficient
   std::array<std::vector<Item>, 2> items;
   std::vector<Step> steps;
+  std::array<std::vector<const Step *>, TT_WAVES> mine;
+  TetraWalk(const TetraProds &P, int k0, int nops);
+  TetraWalk(const TetraWalk &) = delete;  // steps point at items
+  // the groups of a structure of a step, four quarters each (NULL: none), and the products of a group
+  static size_t groups(const Step &st, int ty) {
+    size_t n = 0;
+    for (const Item *I : st.it) n = I ? std::max(n, I->g[ty].size()) : n;
+    return n;
+  }
+  static std::array<const Group *, 4> group(const Step &st, int ty, size_t g) {
+    std::array<const Group *, 4> G;
+    for (int j = 0; j < 4; j++) G[j] = st.it[j] && g < st.it[j]->g[ty].size() ? &st.it[j]->g[ty][g] : nullptr;
+    return G;
+  }
+  static size_t products(const std::array<const Group *, 4> &G) {
+    size_t n = 0;
+    for (const Group *q : G) n = q ? std::max(n, q->e.size()) : n;
+    return n;
+  }
+  uint32_t blocks(const std::array<const Group *, 4> &G, size_t e) const {
+    uint32_t m = 0;
+    for (const Group *q : G) m |= q && e < q->e.size() ? mask[q->e[e].second] : 0;
+    return m;
+  }
+};
+
+TetraWalk::TetraWalk(const TetraProds &P, int k0, int nops) : k0(k0), nops(nops), mask(P.prods.size(), 0) {
+  std::vector<uint8_t> used(P.prods.size(), 0);
+  for (size_t i = 0; i < P.prods.size(); i++)
+    for (const auto &kv : P.prods[i].v) {
+      const int k = kv.first - k0;
+      if (k < 0 || k >= nops) continue;
+      used[i] = 1;
+      for (int h = 0; h < 2; h++)
+        if (kv.second[h] != 0) mask[i] |= 1u << (4 * h + k / 16);
+    }
   for (int set = 0; set < 2; set++) {
     for (int p = 0; p < 256; p++) {
       Item I;
       I.p = p;
       for (int ty = 0; ty < 2; ty++) {
+        const int *ix = &P.index[set << 17 | ty << 16 | p << 8];
         for (int s2 = 0; s2 < 16; s2++) {
           Group G;
           G.s2 = s2;
           for (int s4 = 0; s4 < 16; s4++) {
-            const int id = index[set << 17 | ty << 16 | p << 8 | s2 * 16 + s4];
-            if (used(id)) G.e.push_back({s4, id});
+            const int id = ix[s2 * 16 + s4];
+            if (id >= 0 && used[id]) G.e.push_back({s4, id});
           }
           I.n += (int)G.e.size();
-          if (!G.e.empty()) I.g[ty].push_back(G);
+          if (!G.e.empty()) I.g[ty].push_back(std::move(G));
         }
         std::stable_sort(I.g[ty].begin(), I.g[ty].end(),
                          [](const Group &a, const Group &b) { return a.e.size() > b.e.size(); });
         for (const Group &G : I.g[ty]) I.sig.push_back((int)G.e.size());
         I.sig.push_back(0);
       }
-      if (I.n) items[set].push_back(I);
+      if (I.n) items[set].push_back(std::move(I));
     }
     // steps of four spin pairs p with like groups
     std::stable_sort(items[set].begin(), items[set].end(),
@@ -407,80 +434,132 @@ static void tetra_walk(const std::vector<TetraProd> &prods, const std::vector<in
     }
   }
   std::stable_sort(steps.begin(), steps.end(), [](const Step &a, const Step &b) { return a.cost > b.cost; });
-  std::array<std::vector<const Step *>, TT_WAVES> mine;
   std::array<int, TT_WAVES> load{};
   for (const Step &st : steps) {
     const int w = (int)(std::min_element(load.begin(), load.end()) - load.begin());
     load[w] += st.cost;
     mine[w].push_back(&st);
   }
-  const int NB = (nops + 15) / 16;
-  for (int w = 0; w < TT_WAVES; w++) {
-    out.s.word0[w] = (int)out.words.size();
-    out.s.coef0[w] = (int)(out.coef.size() / 64);
-    out.s.nsteps[w] = (int)mine[w].size();
-    for (const Step *st : mine[w]) {
-      uint32_t pw = 0;
-      size_t ng[2] = {0, 0};
-      for (int j = 0; j < 4; j++)
-        if (st->it[j]) {
-          pw |= (uint32_t)st->it[j]->p << (8 * j);
-          for (int ty = 0; ty < 2; ty++) ng[ty] = std::max(ng[ty], st->it[j]->g[ty].size());
-        }
-      out.words.push_back(pw);
-      out.cost += 108 + 108 * (int64_t)ng[0] + 36 * (int64_t)ng[1];
-      out.words.push_back((uint32_t)ng[0] | (uint32_t)ng[1] << 8 | (uint32_t)st->set << 16);
-      for (int ty = 0; ty < 2; ty++)
-        for (size_t g = 0; g < ng[ty]; g++) {
-          uint32_t gw = 0;
-          size_t nt = 0;
-          const Group *G[4];
-          for (int j = 0; j < 4; j++) {
-            G[j] = st->it[j] && g < st->it[j]->g[ty].size() ? &st->it[j]->g[ty][g] : nullptr;
-            if (!G[j]) continue;
-            gw |= (uint32_t)G[j]->s2 << (4 * j);
-            nt = std::max(nt, G[j]->e.size());
-          }
-          out.words.push_back(gw | (uint32_t)nt << 16);
-          for (size_t e = 0; e < nt; e++) {
-            uint32_t uw = 0;
-            double V[2][4][64] = {};  // [real, imaginary][operator block][quarter * 16 + operator]
-            for (int j = 0; j < 4; j++) {
-              if (!G[j] || e >= G[j]->e.size()) continue;
-              uw |= (uint32_t)G[j]->e[e].first << (4 * j);
-              for (const auto &kv : prods[G[j]->e[e].second].v) {
-                const int k = kv.first - k0;
-                if (k < 0 || k >= nops) continue;
-                for (int h = 0; h < 2; h++) V[h][k / 16][16 * j + k % 16] = kv.second[h];
-              }
-            }
-            for (int h = 0; h < 2; h++)
-              for (int b = 0; b < NB; b++)
-                if (std::any_of(V[h][b], V[h][b] + 64, [](double v) { return v != 0; })) {
-                  uw |= 1u << (16 + 4 * h + b);
-                  out.coef.insert(out.coef.end(), V[h][b], V[h][b] + 64);
-                }
-            out.words.push_back(uw);
-            out.cost += 36 + 26 * __builtin_popcount(uw >> 16);
-          }
-        }
-    }
-    out.words.resize((out.words.size() + 63) / 64 * 64 + 128, 0u);  // the reads ahead
-  }
-  out.coef.resize(out.coef.size() + 3 * 64, 0.0);
-  out.s.nops = nops;
 }
 
-// host: classify the terms of a table (reference format) and lay out the
-// walks, one per `per` operators
-int tetra_pack(const int16_t *idxs, const int16_t *cols, const float *vals, const int16_t *counts, int nops, int per,
-               std::vector<TetraPacked> &out, bool &by_terms) {
+void tetra_pack(const TetraProds &P, const TetraWalks &walks, std::vector<TetraPacked> &outs) {
+  outs.clear();
+  for (const auto &walk : walks) {
+    const TetraWalk &W = *walk;
+    outs.emplace_back();
+    TetraPacked &out = outs.back();
+    for (int w = 0; w < TT_WAVES; w++) {
+      out.s.word0[w] = (int)out.words.size();
+      out.s.coef0[w] = (int)(out.coef.size() / 64);
+      out.s.nsteps[w] = (int)W.mine[w].size();
+      for (const TetraWalk::Step *st : W.mine[w]) {
+        uint32_t pw = 0;
+        for (int j = 0; j < 4; j++)
+          if (st->it[j]) pw |= (uint32_t)st->it[j]->p << (8 * j);
+        const size_t ng[2] = {TetraWalk::groups(*st, 0), TetraWalk::groups(*st, 1)};
+        out.words.push_back(pw);
+        out.words.push_back((uint32_t)ng[0] | (uint32_t)ng[1] << 8 | (uint32_t)st->set << 16);
+        for (int ty = 0; ty < 2; ty++)
+          for (size_t g = 0; g < ng[ty]; g++) {
+            const auto G = TetraWalk::group(*st, ty, g);
+            const size_t nt = TetraWalk::products(G);
+            uint32_t gw = (uint32_t)nt << 16;
+            for (int j = 0; j < 4; j++)
+              if (G[j]) gw |= (uint32_t)G[j]->s2 << (4 * j);
+            out.words.push_back(gw);
+            for (size_t e = 0; e < nt; e++) {
+              const uint32_t m = W.blocks(G, e);
+              uint32_t uw = m << 16;
+              for (int j = 0; j < 4; j++)
+                if (G[j] && e < G[j]->e.size()) uw |= (uint32_t)G[j]->e[e].first << (4 * j);
+              // a coefficient vector of 64, [quarter][operator of the block], per block of the word
+              double *V[8];
+              size_t at = out.coef.size();
+              out.coef.resize(at + 64 * (size_t)__builtin_popcount(m), 0.0);
+              for (int b = 0; b < 8; b++) {
+                V[b] = m >> b & 1 ? &out.coef[at] : nullptr;
+                at += m >> b & 1 ? 64 : 0;
+              }
+              for (int j = 0; j < 4; j++) {
+                if (!G[j] || e >= G[j]->e.size()) continue;
+                for (const auto &kv : P.prods[G[j]->e[e].second].v) {
+                  const int k = kv.first - W.k0;
+                  if (k < 0 || k >= W.nops) continue;
+                  for (int h = 0; h < 2; h++)
+                    if (double *v = V[4 * h + k / 16]) v[16 * j + k % 16] = kv.second[h];
+                }
+              }
+              out.words.push_back(uw);
+            }
+          }
+      }
+      out.words.resize((out.words.size() + 63) / 64 * 64 + 128, 0u);  // the reads ahead
+    }
+    out.coef.resize(out.coef.size() + 3 * 64, 0.0);
+    out.s.nops = W.nops;
+  }
+}
+
+// The walk against the terms one by one (plg_tetra_terms.hip), fitted to
+// calls with 60 tables -- 1 to 64 operators of 40 to 4 000 terms, real and
+// complex coefficients, few and many shared products -- on 4 096 to 221 184
+// sites.  Microseconds of as many workgroups as the chip holds:
+//   walk   12 and 0.87 per thousand FMAs of a lane, a matrix instruction counted as 26
+//   terms  195, and per operator of the wave with most of them 73, 11.6 per 64
+//          direct and 18.4 (FP64 23.6) per 64 crossed terms
+// (measured walk / terms in ms: the udbb table 1.2 / 3.7 on 98 304 sites; 16
+// operators of 768 random complex terms in FP32 7.8 / 6.6 on 221 184 sites, 0.72
+// / 0.98 on 13 824; in FP64 15.0 / 13.0 and 1.22 / 1.03; 64 operators of 40
+// terms 1.5 / 6.4 on 110 592).  The walk has to be the faster by 1.25, about
+// the error of the fit: so none of those calls is slower than term by term,
+// and the choice is within 1.25 of the better form.
+TetraCost tetra_cost(const TetraProds &P, int per, bool f64, TetraWalks &walks) {
+  TetraCost c;
+  c.slots = f64 ? 256 : 512;
+  for (int k0 = 0; k0 < P.nops; k0 += per) {
+    walks.push_back(std::make_shared<const TetraWalk>(P, k0, std::min(per, P.nops - k0)));
+    const TetraWalk &W = *walks.back();
+    int64_t fma = 0;
+    for (const TetraWalk::Step &st : W.steps) {
+      fma += 108;
+      for (int ty = 0; ty < 2; ty++)
+        for (size_t g = 0; g < TetraWalk::groups(st, ty); g++) {
+          const auto G = TetraWalk::group(st, ty, g);
+          const size_t nt = TetraWalk::products(G);
+          fma += ty ? 36 : 108;
+          for (size_t e = 0; e < nt; e++) fma += 36 + 26 * __builtin_popcount(W.blocks(G, e));
+        }
+    }
+    c.walk += 12 + 0.87e-3 * (double)fma;
+  }
+  for (int set = 0; set < 2; set++) {
+    double wave[4] = {0, 0, 0, 0};
+    bool any = set == 0;
+    for (int k = 0; k < P.nops; k++) {
+      const auto &n = P.terms[set][k];
+      any = any || n[0] + n[1] > 0;
+      wave[k % 4] += 73 + 11.6 * ((n[1] + 63) / 64) + (f64 ? 23.6 : 18.4) * ((n[0] + 63) / 64);
+    }
+    if (any) c.terms += 195 + *std::max_element(wave, wave + 4);
+  }
+  return c;
+}
+
+bool tetra_by_terms(const TetraCost &c, int64_t V3, int64_t nrows) {
+  auto rounds = [&](int64_t sites) { return (double)(((V3 + sites - 1) / sites * nrows + c.slots - 1) / c.slots); };
+  return rounds(64) * c.terms < 1.25 * rounds(16) * c.walk;
+}
+
+// host: the terms of a table (reference format) by product
+int tetra_products(const int16_t *idxs, const int16_t *cols, const float *vals, const int16_t *counts, int nops,
+                   TetraProds &out) {
   if (nops <= 0 || nops > TETRA_MAXOPS) return PLG_ERR_UNSUPPORTED;
   std::map<std::pair<uint32_t, uint32_t>, int> cidx;  // distinct coefficients, zero among them
   cidx.emplace(std::make_pair(0u, 0u), 0);
-  std::vector<TetraProd> prods;
-  std::vector<int> index(1 << 18, -1);
-  int64_t ndirect = 0;
+  out = TetraProds{};
+  out.nops = nops;
+  out.index.assign(1 << 18, -1);
+  for (auto &v : out.terms) v.assign(nops, {0, 0});
   size_t t = 0;
   for (int k = 0; k < nops; k++) {
     if (counts[k] < 0) return PLG_ERR_INVALID;
@@ -508,31 +587,17 @@ int tetra_pack(const int16_t *idxs, const int16_t *cols, const float *vals, cons
       else if (c[0] == c[7] && c[1] == c[6] && c[2] == c[5] && c[3] == c[4]) key = 3 << 16 | u1;
       else if (c[0] == c[7] && c[1] == c[4] && c[2] == c[5] && c[3] == c[6]) key = 2 << 16 | u1;
       else return PLG_ERR_UNSUPPORTED;
-      ndirect += key >> 16 & 1;
-      if (index[key] < 0) {
-        index[key] = (int)prods.size();
-        prods.emplace_back();
+      out.terms[key >> 17][k][key >> 16 & 1]++;
+      if (out.index[key] < 0) {
+        out.index[key] = (int)out.prods.size();
+        out.prods.emplace_back();
       }
-      auto &v = prods[index[key]].v;
+      auto &v = out.prods[out.index[key]].v;
       if (v.empty() || v.back().first != k) v.push_back({k, {0.0, 0.0}});
       v.back().second[0] += (double)vals[2 * t];
       v.back().second[1] += (double)vals[2 * t + 1];
     }
   }
-  out.clear();
-  for (int k0 = 0; k0 < nops; k0 += per) {
-    out.emplace_back();
-    tetra_walk(prods, index, k0, std::min(per, nops - k0), out.back());
-  }
-  // The walk against the terms one by one (plg_tetra_terms.hip), in ns per
-  // site of a full chip: the walk 0.116 per unit of its cost (the udbb table
-  // 12.8, 110 k units), the terms 4 per thousand crossed and 1 per thousand
-  // direct ones and 5 for their spin-pair tables (udbb 37; 12.3 k random terms
-  // with complex coefficients 37, by the walk 42).  Ties go to the walk.
-  int64_t cost = 0;
-  for (const TetraPacked &P : out) cost += P.cost;
-  const double walk = 0.116e-3 * (double)cost, terms = 5 + 4e-3 * (double)((int64_t)t - ndirect) + 1e-3 * (double)ndirect;
-  by_terms = walk > terms;
   return PLG_OK;
 }
 

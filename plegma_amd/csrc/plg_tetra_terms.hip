@@ -272,16 +272,20 @@ template int launch_tetra_terms<float>(const TetraTermsSched &, const PropDev<fl
 // tables the passes per read drop from 1.6 (a Latin-square walk over the
 // buckets) to 1.3.  The sum is the same up to rounding.
 static int run_passes(const TetraTerm *r, int n) {
-  uint16_t mp[16] = {0}, mq[16] = {0};  // distinct spin pairs per residue (bit s1 / s2)
+  // distinct spin pairs per residue (bit s1 / s2) and how many, without branches
+  uint16_t mp[16] = {0}, mq[16] = {0};
+  uint8_t np[16] = {0}, nq[16] = {0}, dp = 0, dq = 0;
+  auto add = [](uint16_t *m, uint8_t *c, int v) {
+    c[v & 15] += ~(m[v & 15] >> (v >> 4)) & 1;
+    m[v & 15] |= (uint16_t)(1u << (v >> 4));
+  };
   for (int i = 0; i < n; i++) {
-    const int p = r[i] & 255, q = (r[i] >> 8) & 255;
-    mp[p & 15] |= (uint16_t)(1u << (p >> 4));
-    mq[q & 15] |= (uint16_t)(1u << (q >> 4));
+    add(mp, np, r[i] & 255);
+    add(mq, nq, (r[i] >> 8) & 255);
   }
-  int dp = 0, dq = 0;
   for (int k = 0; k < 16; k++) {
-    dp = std::max(dp, __builtin_popcount(mp[k]));
-    dq = std::max(dq, __builtin_popcount(mq[k]));
+    dp = std::max(dp, np[k]);
+    dq = std::max(dq, nq[k]);
   }
   return dp + dq;
 }
