@@ -460,66 +460,7 @@ void sep_build(const int L[3], int M, const std::vector<int> &ms, int64_t ncols,
   for (auto &e : pairs) maxcnt = std::max(maxcnt, (int)e.second.size());
   if (maxcnt > 16) return;
   g.small = g.NA <= 5 && g.NB <= 5 && maxcnt <= 9;
-  // tables padded to the kernel's class and momentum counts
-  const int NAP = g.small ? 5 : 8, NBP = g.small ? 5 : 8, NZP = g.small ? 9 : 16;
-  std::vector<int> ryres(g.NYR);
-  for (auto &e : rymap) ryres[e.second] = e.first;
-  std::vector<int> slot(g.NXR * NBP * 2, -1), slm(g.NS * NZP, -1), slrz(g.NS * NZP, 0);
-  {
-    int sidx = 0;
-    for (auto &e : pairs) {
-      // the pair's n_y residue as class b, sign + (r = b) or - (r = Ly - b != b)
-      const int r = ryres[e.first.second], b = std::min(r, Ly - r);
-      slot[(e.first.first * NBP + bmap[b]) * 2 + (r == b ? 0 : 1)] = sidx;
-      for (size_t j = 0; j < e.second.size(); j++) {
-        slm[sidx * NZP + j] = e.second[j];
-        slrz[sidx * NZP + j] = rz[e.second[j]];
-      }
-      sidx++;
-    }
-  }
-  // residue slots of +a and -a
-  std::vector<int> xs(2 * NAP, -1);
-  for (auto &e : amap) {
-    const int a = e.first;
-    auto ip = rxmap.find(a);
-    if (ip != rxmap.end()) xs[2 * e.second] = ip->second;
-    auto im = rxmap.find((Lx - a) % Lx);
-    if (a != 0 && 2 * a != Lx && im != rxmap.end()) xs[2 * e.second + 1] = im->second;
-  }
-  // phases from exact integer residues
-  auto phase = [](int64_t num, int den) {
-    const double t = 2.0 * M_PI * (double)(num % den) / (double)den;
-    return std::make_pair(std::cos(t), std::sin(t));
-  };
-  std::vector<double> ph1(2 * g.W * NAP, 0.0), ph1p(2 * g.NPART * NAP, 0.0), ph2(2 * Ly * NBP, 0.0), ph3;
-  for (auto &e : amap)
-    for (int i = 0; i < g.W; i++) {
-      auto cs = phase((int64_t)e.first * i, Lx);
-      ph1[2 * (i * NAP + e.second)] = cs.first;
-      ph1[2 * (i * NAP + e.second) + 1] = cs.second;
-    }
-  for (auto &e : amap)
-    for (int p = 0; p < g.NPART; p++) {
-      auto cs = phase((int64_t)e.first * p * g.W, Lx);
-      ph1p[2 * (p * NAP + e.second)] = cs.first;
-      ph1p[2 * (p * NAP + e.second) + 1] = cs.second;
-    }
-  for (auto &e : bmap)
-    for (int y = 0; y < Ly; y++) {
-      auto cs = phase((int64_t)e.first * y, Ly);
-      ph2[2 * (y * NBP + e.second)] = cs.first;
-      ph2[2 * (y * NBP + e.second) + 1] = cs.second;
-    }
-  for (int r = 0; r < Lz; r++)
-    for (int z = 0; z < Lz; z++) {
-      auto cs = phase((int64_t)r * z, Lz);
-      ph3.push_back(cs.first);
-      ph3.push_back(cs.second);
-    }
   // the matrix form: functions cos a, sin a (unless the sine vanishes at every site)
-  std::vector<double> pha, ph2f;
-  std::vector<int> slq;
   std::map<int, std::pair<int, int>> fx, fy;
   auto functions = [](const std::map<int, int> &cls, int L, std::map<int, std::pair<int, int>> &f) {
     int n = 0;
@@ -533,6 +474,72 @@ void sep_build(const int L[3], int M, const std::vector<int> &ms, int64_t ncols,
   g.NF = functions(amap, Lx, fx);
   g.NG = functions(bmap, Ly, fy);
   g.mm = g.small && Lx % 4 == 0 && g.NF <= 12 && g.NG <= 9;
+  // tables padded to the kernel's class and momentum counts
+  const int NAP = g.small ? 5 : 8, NBP = g.small ? 5 : 8, NZP = g.small ? 9 : 16;
+  std::vector<int> ryres(g.NYR);
+  for (auto &e : rymap) ryres[e.second] = e.first;
+  std::vector<int> slot, xs, slq, slm(g.NS * NZP, -1), slrz(g.NS * NZP, 0);
+  {
+    int sidx = 0;
+    for (auto &e : pairs) {
+      for (size_t j = 0; j < e.second.size(); j++) {
+        slm[sidx * NZP + j] = e.second[j];
+        slrz[sidx * NZP + j] = rz[e.second[j]];
+      }
+      sidx++;
+    }
+  }
+  // phases from exact integer residues
+  auto phase = [](int64_t num, int den) {
+    const double t = 2.0 * M_PI * (double)(num % den) / (double)den;
+    return std::make_pair(std::cos(t), std::sin(t));
+  };
+  std::vector<double> ph1, ph1p, ph2, pha, ph2f, ph3;
+  if (!g.mm) {  // the staged form's tables
+    slot.assign(g.NXR * NBP * 2, -1);
+    int sidx = 0;
+    for (auto &e : pairs) {
+      // the pair's n_y residue as class b, sign + (r = b) or - (r = Ly - b != b)
+      const int r = ryres[e.first.second], b = std::min(r, Ly - r);
+      slot[(e.first.first * NBP + bmap[b]) * 2 + (r == b ? 0 : 1)] = sidx++;
+    }
+    // residue slots of +a and -a
+    xs.assign(2 * NAP, -1);
+    for (auto &e : amap) {
+      const int a = e.first;
+      auto ip = rxmap.find(a);
+      if (ip != rxmap.end()) xs[2 * e.second] = ip->second;
+      auto im = rxmap.find((Lx - a) % Lx);
+      if (a != 0 && 2 * a != Lx && im != rxmap.end()) xs[2 * e.second + 1] = im->second;
+    }
+    ph1.assign(2 * g.W * NAP, 0.0);
+    ph1p.assign(2 * g.NPART * NAP, 0.0);
+    ph2.assign(2 * Ly * NBP, 0.0);
+    for (auto &e : amap)
+      for (int i = 0; i < g.W; i++) {
+        auto cs = phase((int64_t)e.first * i, Lx);
+        ph1[2 * (i * NAP + e.second)] = cs.first;
+        ph1[2 * (i * NAP + e.second) + 1] = cs.second;
+      }
+    for (auto &e : amap)
+      for (int p = 0; p < g.NPART; p++) {
+        auto cs = phase((int64_t)e.first * p * g.W, Lx);
+        ph1p[2 * (p * NAP + e.second)] = cs.first;
+        ph1p[2 * (p * NAP + e.second) + 1] = cs.second;
+      }
+    for (auto &e : bmap)
+      for (int y = 0; y < Ly; y++) {
+        auto cs = phase((int64_t)e.first * y, Ly);
+        ph2[2 * (y * NBP + e.second)] = cs.first;
+        ph2[2 * (y * NBP + e.second) + 1] = cs.second;
+      }
+  }
+  for (int r = 0; r < Lz; r++)
+    for (int z = 0; z < Lz; z++) {
+      auto cs = phase((int64_t)r * z, Lz);
+      ph3.push_back(cs.first);
+      ph3.push_back(cs.second);
+    }
   if (g.mm) {
     const int NGP = sep_ng(g.NF, g.NG);
     const int EP = sep_epu(Lx, f64);
@@ -560,11 +567,6 @@ void sep_build(const int L[3], int M, const std::vector<int> &ms, int64_t ncols,
       const int a = std::min(rx_, Lx - rx_), b = std::min(ry_, Ly - ry_);
       slq.insert(slq.end(), {fx[a].first, fx[a].second, rx_ == a ? 1 : -1, fy[b].first, fy[b].second, ry_ == b ? 1 : -1});
     }
-    ph1.clear();
-    ph1p.clear();
-    ph2.clear();
-    xs.clear();
-    slot.clear();
   }
   // one blob, 256-byte aligned pieces
   auto put = [&](const void *src, size_t bytes) {
