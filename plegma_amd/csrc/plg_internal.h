@@ -109,12 +109,18 @@ struct UdscTerm {
 // propagators (pa, pb) and so the colour diquarks D of their spin pairs.
 // Product j of a group traces D with propagator third[j] into its nops[j]
 // operators, channels ch0[j]...  A wave's share of a group is nsteps steps
-// from step0.  Step, two words: the spin pairs of its four quads (m01 | m23
-// << 4, a byte each) and the term counts of the products (a byte each, the
-// largest of the four quads).  Per product the step's terms come in units of
-// four, numbered on from unit0: two words with the spin pair of the third
-// propagator (4 bits) of term e of quad i at bit 16 i + 4 e, and the
-// coefficients [quad i][operator k][term e] (0: no such term).
+// from step0, the first npair of them paired: two quads for each quarter of
+// the wave, with terms for the spin pairs of the third propagator that either
+// has (one read of it serves both); the others have one quad.
+// Step, three words: the spin pairs of the four quarters' first quads (m01 |
+// m23 << 4, a byte each), those of the second quads (paired steps), and the
+// term counts of the products (a byte each, the largest of the four quarters).
+// Per product the step's terms come in units of four, numbered on from unit0:
+// two words with the spin pair of the third propagator (4 bits) of term e of
+// quarter i at bit 16 i + 4 e, and for each of the quarters' quads (two blocks
+// in a paired step, else one) 256 coefficients [quarter i][operator k][term e]
+// (0: no such term), numbered in blocks on from coef0.  The kernel reads a
+// wave's next coefficients ahead: four blocks of zeros end coef.
 constexpr int UD_WAVES = 8;       // waves of a workgroup
 constexpr int UD_NJ = 4;          // products of a group
 constexpr int UD_MAXGROUPS = 6;   // uu, dd, ss, cc, ud, sc

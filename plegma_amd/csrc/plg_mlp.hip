@@ -287,7 +287,7 @@ __device__ __forceinline__ void lds_barrier() {
 // its first tile of the next layer before this layer's stores.
 // 17-256-256-11 at 2 048 rows: 17 us (a 256 x 256 layer streams its 131 KB of
 // weights through the CU in about 2 us; the transposed outputs' stores are
-// 4 us), k_mlp_update 6 us; a step takes 28 us against 153 us in 23 launches.
+// 4 us), k_mlp_update 6 us; a step takes 26 us against 153 us in 23 launches.
 template <bool BACK, int Q, int NW>
 __global__ __launch_bounds__(64 * NW) void k_mlp_rows(MlpDev d, const float *__restrict__ x, const float *__restrict__ t,
                                                          float scale, float *__restrict__ y, int *__restrict__ step,

@@ -42,10 +42,13 @@ namespace plg {
 // at the end.
 // Bound by the vector unit: M 108 FMAs, X 108 (crossed) or 36, a product 36
 // and its matrix instructions.
-// Of 2.64 M cycles on 16^3 x 24 sites with the udbb table, FP32, the FMAs take
+// Of 2.7 M cycles on 16^3 x 24 sites with the udbb table, FP32, the FMAs take
 // 1.5 M, the matrix instructions 0.35 M, LDS is busy 1.4 M.  Term by term from
 // tables of B3^dag B1 and B4^dag B2 in LDS, a site at a time, the same took
-// 3.65 ms, bound by the 160 bytes of LDS a term reads; this 1.26 ms.
+// 3.65 ms, bound by the 160 bytes of LDS a term reads; this 1.15 ms.
+// Entries that are not finite, and products that overflow, reach the operators
+// that have a term with them at that site and no others, as term by term (SAFE
+// below).
 template <typename T> struct TtAcc;
 template <> struct TtAcc<float> {
   typedef float v4 __attribute__((ext_vector_type(4)));

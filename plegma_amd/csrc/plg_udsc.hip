@@ -640,11 +640,14 @@ template int launch_udsc<float>(const UdscSched &, const PropDev<float> *, const
 // spin pairs of the third propagator: one read of it serves both.
 // Bound by the vector unit and LDS (a term is 36 FMAs, two matrix instructions
 // and 9 reads; one quad at a time the FMAs took 4.5 M of 9.2 M cycles, the
-// matrix instructions 1.9 M, LDS was busy 5.5 M).  20 products on 24^3 x 16
+// matrix instructions 1.9 M, LDS was busy 5.5 M; two at a time LDS is busy
+// 3.5 M of 8.6 M, 1.4 % of it bank conflicts).  20 products on 24^3 x 16
 // sites, FP32, whole calls: 20 launches of k_udsc 14.6 ms, here one quad at a
 // time 4.16 ms, two 3.89 ms.  k_udsc reads the terms, coefficients and entry
 // indexes of its operator sums and every diquark's blocks from LDS 20 times
 // per site, and is bound there.
+// Entries that are not finite, and products that overflow, reach the operators
+// that have a term with them at that site and no others (SAFE below).
 template <typename T> struct UdAcc;
 template <> struct UdAcc<float> {
   typedef float v4 __attribute__((ext_vector_type(4)));
