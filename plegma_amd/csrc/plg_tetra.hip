@@ -259,6 +259,7 @@ __global__ __launch_bounds__(64 * TT_WAVES, sizeof(T) == 4 ? 4 : 2) void k_tetra
   };
   // the waves' sums: thread tid < 256 holds operator row(lane, wave) of every block at its site
   T o[NB][2];
+  int *flag = (int *)spec;  // [256 / 64]: a sum of the wave is not finite, in the wave's own place of red
   auto reduce = [&]() {
 #pragma unroll
     for (int b = 0; b < NB; b++)
@@ -276,6 +277,13 @@ __global__ __launch_bounds__(64 * TT_WAVES, sizeof(T) == 4 ? 4 : 2) void k_tetra
 #pragma unroll
             for (int w = 0; w < n; w++) v[w] += v[w + n];
           o[b][h] = v[0];
+          if (h == 1 && b + 1 == NB) {
+            bool bad = false;
+#pragma unroll
+            for (int i = 0; i < NB; i++) bad = bad || !__builtin_isfinite(o[i][0]) || !__builtin_isfinite(o[i][1]);
+            const int mine = __any(bad);
+            if (lane == 0) flag[(int)(sizeof(T) / 4) * tid] = mine;
+          }
         }
         __syncthreads();
       }
@@ -284,17 +292,9 @@ __global__ __launch_bounds__(64 * TT_WAVES, sizeof(T) == 4 ? 4 : 2) void k_tetra
   reduce();
   {
     // a sum that is not finite: its tile again, with the care of SAFE
-    bool bad = false;
-    if (tid < 256)
-#pragma unroll
-      for (int b = 0; b < NB; b++) bad = bad || !__builtin_isfinite(o[b][0]) || !__builtin_isfinite(o[b][1]);
-    int *flag = (int *)spec;
-    const int mine = __any(bad);
-    if (lane == 0) flag[wave] = mine;
-    __syncthreads();
     int any = 0;
 #pragma unroll
-    for (int w = 0; w < 4; w++) any |= flag[w];
+    for (int w = 0; w < 4; w++) any |= flag[(int)(sizeof(T) / 4) * 64 * w];
     if (__builtin_amdgcn_readfirstlane(any)) {
       __syncthreads();
       for (int i = tid; i < 512 * NB; i += NT) spec[i] = 0;

@@ -815,6 +815,7 @@ __global__ __launch_bounds__(64 * UD_WAVES, sizeof(T) == 4 ? 4 : 2) void k_udsc_
     T o[UD_NJ][2];
 #pragma unroll
     for (int j = 0; j < UD_NJ; j++) o[j][0] = o[j][1] = 0;
+    int *flag = (int *)spec;  // [256 / 64]: a sum of the wave is not finite, in the wave's own place of red
     auto reduce = [&]() {
 #pragma unroll
       for (int j = 0; j < UD_NJ; j++) {
@@ -833,6 +834,13 @@ __global__ __launch_bounds__(64 * UD_WAVES, sizeof(T) == 4 ? 4 : 2) void k_udsc_
 #pragma unroll
               for (int w = 0; w < n; w++) v[w] += v[w + n];
             o[j][h] = v[0];
+            if (h == 1 && j + 1 == G.nprod) {
+              bool bad = false;
+#pragma unroll
+              for (int i = 0; i <= j; i++) bad = bad || !__builtin_isfinite(o[i][0]) || !__builtin_isfinite(o[i][1]);
+              const int mine = __any(bad);
+              if (ln == 0) flag[(int)(sizeof(T) / 4) * tq] = mine;
+            }
           }
           __syncthreads();
         }
@@ -840,16 +848,9 @@ __global__ __launch_bounds__(64 * UD_WAVES, sizeof(T) == 4 ? 4 : 2) void k_udsc_
     };
     reduce();
     // a sum that is not finite: the group again, with the care of SAFE
-    bool bad = false;
-#pragma unroll
-    for (int j = 0; j < UD_NJ; j++) bad = bad || !__builtin_isfinite(o[j][0]) || !__builtin_isfinite(o[j][1]);
-    int *flag = (int *)spec;
-    const int mine = __any(bad);
-    if (ln == 0) flag[wave] = mine;
-    __syncthreads();
     int any = 0;
 #pragma unroll
-    for (int w = 0; w < 4; w++) any |= flag[w];
+    for (int w = 0; w < 4; w++) any |= flag[(int)(sizeof(T) / 4) * 64 * w];
     __syncthreads();  // red is the next group's (or SAFE's) after this
     if (__builtin_amdgcn_readfirstlane(any)) {
       for (int i = tq; i < 512 * UD_NJ; i += NT) spec[i] = 0;
