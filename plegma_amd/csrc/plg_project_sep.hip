@@ -280,13 +280,7 @@ __global__ __launch_bounds__(256, 3) void k_sep_xy_mm(SepGeom s, const cx<T> *__
     vec cur[SEP_PF];
 #pragma unroll
     for (int u = 0; u < SEP_PF; u++) cur[u] = fetch();
-    // a line's sums, those of every other unit apart where the registers allow:
-    // a chain half as long rounds less (FP64 field of 24^3, rms error against 64
-    // bits 5.0 -> 4.8 e-16 of the sums'; the staged lines 4.9), at the same speed
-    constexpr int ND = RF == 2 ? 2 : 1;
-    sep_v4 Dr[ND], Di[ND];
-#pragma unroll
-    for (int q = 0; q < ND; q++) Dr[q] = Di[q] = (sep_v4)0.0;
+    sep_v4 Dr = (sep_v4)0.0, Di = (sep_v4)0.0;
     int y = wave, g = 0;
     double ph[NG];  // the line's phases, loaded a line ahead
 #pragma unroll
@@ -301,14 +295,10 @@ __global__ __launch_bounds__(256, 3) void k_sep_xy_mm(SepGeom s, const cx<T> *__
 #pragma unroll
           for (int e = 0; e < EPU; e++) {
             const double a = pha[(g * EPU + e) * 64 + lane];
-            Dr[u % ND] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, (double)cur[u][2 * e], Dr[u % ND], 0, 0, 0);
-            Di[u % ND] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, (double)cur[u][2 * e + 1], Di[u % ND], 0, 0, 0);
+            Dr = __builtin_amdgcn_mfma_f64_16x16x4f64(a, (double)cur[u][2 * e], Dr, 0, 0, 0);
+            Di = __builtin_amdgcn_mfma_f64_16x16x4f64(a, (double)cur[u][2 * e + 1], Di, 0, 0, 0);
           }
           if (++g == U) {  // the line is whole
-            if (ND == 2) {
-              Dr[0] += Dr[ND - 1];
-              Di[0] += Di[ND - 1];
-            }
             y += 4;
             const int yn = min(y, s.Ly - 1);
 #pragma unroll
@@ -317,12 +307,11 @@ __global__ __launch_bounds__(256, 3) void k_sep_xy_mm(SepGeom s, const cx<T> *__
               ph[j] = s.ph2f[yn * NG + j];
 #pragma unroll
               for (int r = 0; r < RF; r++) {
-                acc[r][j].re = fma(p, Dr[0][r], acc[r][j].re);
-                acc[r][j].im = fma(p, Di[0][r], acc[r][j].im);
+                acc[r][j].re = fma(p, Dr[r], acc[r][j].re);
+                acc[r][j].im = fma(p, Di[r], acc[r][j].im);
               }
             }
-#pragma unroll
-            for (int q = 0; q < ND; q++) Dr[q] = Di[q] = (sep_v4)0.0;
+            Dr = Di = (sep_v4)0.0;
             g = 0;
           }
         }
