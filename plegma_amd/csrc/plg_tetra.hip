@@ -217,12 +217,13 @@ __global__ __launch_bounds__(64 * TT_WAVES, sizeof(T) == 4 ? 4 : 2) void k_tetra
           }
           // operators of block b that have a coefficient v: real sum += v re, imaginary sum += v im
           auto apart = [&](int b, T v, T re, T im) {
-#pragma unroll 1
-            for (int k = 0; k < 16; k++) {
+            const bool r = !__builtin_isfinite(re), i = !__builtin_isfinite(im);
+            for (unsigned ops = (unsigned)(__ballot(v != 0) >> (16 * kq)) & 0xffff; __any(ops); ops &= ops - 1) {
+              const int k = ops ? __ffs(ops) - 1 : 0;
               const T w = __shfl(v, 16 * kq + k);
               T *d = spec + 512 * b + TtAcc<T>::slot(k, s);
-              if (w != 0 && !__builtin_isfinite(re)) atomicAdd(d, w * re);
-              if (w != 0 && !__builtin_isfinite(im)) atomicAdd(d + 256, w * im);
+              if (ops && r) atomicAdd(d, w * re);
+              if (ops && i) atomicAdd(d + 256, w * im);
             }
           };
           // O[k] += V[k] t in the operator blocks the products have coefficients in

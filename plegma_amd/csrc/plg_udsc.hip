@@ -781,12 +781,13 @@ __global__ __launch_bounds__(64 * UD_WAVES, sizeof(T) == 4 ? 4 : 2) void k_udsc_
                 if constexpr (safe) {
                   const bool fr = __builtin_isfinite(t[b].re), fi = __builtin_isfinite(t[b].im);
                   if (__any(!fr || !fi)) {
-#pragma unroll 1
-                    for (int k = 0; k < 16; k++) {
+                    // (each quarter's operators with a coefficient in turn)
+                    for (unsigned ops = (unsigned)(__ballot(cf[b][e] != 0) >> (16 * kq)) & 0xffff; __any(ops); ops &= ops - 1) {
+                      const int k = ops ? __ffs(ops) - 1 : 0;
                       const T w = __shfl(cf[b][e], 16 * kq + k);
                       T *o = spec + 512 * j + UdAcc<T>::slot(k, s);
-                      if (w != 0 && !fr) atomicAdd(o, w * t[b].re);
-                      if (w != 0 && !fi) atomicAdd(o + 256, w * t[b].im);
+                      if (ops && !fr) atomicAdd(o, w * t[b].re);
+                      if (ops && !fi) atomicAdd(o + 256, w * t[b].im);
                     }
                     t[b] = cmake<T>(fr ? t[b].re : (T)0, fi ? t[b].im : (T)0);
                   }
